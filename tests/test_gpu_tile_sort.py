@@ -1,0 +1,116 @@
+"""Depth order inside every tile (gfx950), at the sizes where the tile sort changes its way:
+list lengths around a wave, one bin per thread, the LDS capacities (512, 2048 and 8192 entries)
+and the lists spread over depth bins in global memory; depths spread, all equal, half equal, and
+in a few float steps beside one far outlier.
+
+Every list must hold each of its records once, in strictly ascending (depth bits, Gaussian ID)
+order, with the keys of those records.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from vgr_amd import CustomHipBackend, RendererService, synthetic
+from vgr_amd.batched import BatchedRenderer, CameraSpec
+
+pytestmark = pytest.mark.gpu
+
+DEPTHS = ("spread", "equal", "half", "steps")
+
+
+def column_scene(count: int, depths: str, seed: int = 5) -> synthetic.SyntheticScene:
+    """``count`` small Gaussians in front of an identity camera, near its axis."""
+    rng = np.random.default_rng(seed)
+    z = rng.uniform(4.0, 8.0, count)
+    if depths == "equal":
+        z[:] = 5.0
+    elif depths == "half":
+        z[rng.permutation(count)[: count // 2]] = 5.0
+    elif depths == "steps":
+        # 64 consecutive floats, and one far Gaussian that stretches the range of the depths.
+        z = (np.float32(2.0).view(np.int32) + rng.integers(0, 64, count)).astype(np.int32).view(np.float32)
+        z = z.astype(np.float64)
+        z[0] = 50.0
+    xy = rng.uniform(-0.2, 0.2, (count, 2)) * z[:, None]
+    means = torch.tensor(np.concatenate([xy, z[:, None]], axis=1), dtype=torch.float32)
+    return synthetic.SyntheticScene(
+        means, torch.full((count, 3), 0.05), torch.tensor([1.0, 0.0, 0.0, 0.0]).repeat(count, 1),
+        torch.full((count,), 0.3), torch.rand((count, 3), generator=torch.Generator().manual_seed(seed)),
+        torch.arange(count, dtype=torch.int64))
+
+
+def identity_rig(size: int):
+    intrinsics = synthetic.pinhole(1, size, size, float(size))
+    return torch.eye(4).unsqueeze(0).contiguous(), intrinsics
+
+
+def check_lists(backend) -> int:
+    counters = backend.read_counters()
+    assert not counters["sort_lookback_failures"] and not counters["intersection_overflow"]
+    ws = backend.workspace
+    total = counters["tile_intersections"]
+    starts, ends = ws["tile_starts"].cpu().numpy(), ws["tile_ends"].cpu().numpy()
+    keys = ws["keys_out"][:total].cpu().numpy()
+    values = ws["values_out"][:total].cpu().numpy()
+    depth_bits = ws["visible_depths"].cpu().numpy().view(np.uint32)
+    ids = ws["visible_gaussian_ids"].cpu().numpy()
+    covered, longest = 0, 0
+    for tile in np.flatnonzero(ends > starts):
+        part = values[starts[tile]:ends[tile]]
+        bits, part_ids = depth_bits[part].astype(np.uint64), ids[part].astype(np.int64)
+        np.testing.assert_array_equal(keys[starts[tile]:ends[tile]], (np.uint64(tile) << np.uint64(32)) | bits)
+        step = np.diff(bits.astype(np.int64))
+        assert np.all((step > 0) | ((step == 0) & (np.diff(part_ids) > 0)))
+        assert np.unique(part).size == part.size
+        covered += part.size
+        longest = max(longest, part.size)
+    assert covered == total
+    return longest
+
+
+def render(scene, size: int, **knobs):
+    dev = torch.device("cuda", 0)
+    backend = CustomHipBackend(output_srgb=False, **knobs)
+    service = RendererService(backend, height=size, width=size, max_views=1)
+    service.initialize(stage=None, device=dev)
+    service.load_scene(0, **scene.to(dev).as_kwargs())
+    viewmats, intrinsics = identity_rig(size)
+    out = service.render(viewmats.to(dev), intrinsics.to(dev), torch.zeros(1, dtype=torch.int64, device=dev))
+    service.synchronize()
+    return backend, out
+
+
+@pytest.mark.parametrize("depths", DEPTHS)
+@pytest.mark.parametrize("count", [1, 2, 64, 255, 257, 2047, 2048, 2049, 8191, 8192, 8193, 30_000])
+def test_one_tile_lists(count, depths):
+    backend, _ = render(column_scene(count, depths), 16)
+    assert check_lists(backend) == count  # every Gaussian is in the image's one tile
+
+
+@pytest.mark.parametrize("depths", DEPTHS)
+@pytest.mark.parametrize("count", [63, 512, 513, 3000])
+def test_one_pixel_lists(count, depths):
+    scene = column_scene(count, depths)
+    scene.scales = torch.full_like(scene.scales, 4.0)  # wide enough to reach every pixel
+    backend, _ = render(scene, 4, tile_size=1, deterministic=True)
+    assert check_lists(backend) == count
+
+
+@pytest.mark.parametrize("depths", ["equal", "half", "steps"])
+@pytest.mark.parametrize("count", [300, 2500, 9000])
+def test_ties_of_a_spatially_ordered_scene(count, depths):
+    """Records of a Morton-ordered scene are not in Gaussian order: ties go by the record's ID."""
+    dev = torch.device("cuda", 0)
+    renderer = BatchedRenderer(device=dev, ordering="global")
+    renderer.register_scene(0, **column_scene(count, depths).to(dev).as_kwargs())
+    renderer.plan([CameraSpec(0, 16, 16)])
+    viewmats, intrinsics = identity_rig(16)
+    renderer.calibrate(viewmats.to(dev), intrinsics.to(dev))
+    out = {name: tensor.clone() for name, tensor in renderer.render().items()}
+    plain = renderer.render_plain()[0]["outputs"]
+    torch.cuda.synchronize()
+    for name, tensor in out.items():
+        assert torch.equal(tensor.view(plain[name].shape), plain[name]), name

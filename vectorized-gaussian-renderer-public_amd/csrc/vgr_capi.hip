@@ -37,11 +37,11 @@ int64_t global_tile_count(const vgr_cameras& cameras, const vgr_options& options
   return static_cast<int64_t>(cameras.batch) * tiles_x * tiles_y;
 }
 
-// Default digit width: 8 bits, or 9 where that saves a radix pass (a 44-bit key:
-// 5 passes instead of 6; an 8192-key tile still averages 16 keys per digit).
+// Default digit width of the partition: 9 bits (an 8192-key tile still averages 16
+// keys per digit), or what a single pass over the whole key needs.
 int resolve_digit_bits(const vgr_options& options, int key_bits) {
   if (options.sort_digit_bits != 0) return options.sort_digit_bits;
-  return (key_bits + 8) / 9 < (key_bits + 7) / 8 ? 9 : 8;
+  return key_bits >= 9 ? 9 : (key_bits < 4 ? 4 : key_bits);
 }
 
 // Default camera group: 32 cameras per projection workgroup.  Each group re-reads
@@ -105,22 +105,30 @@ ScratchLayout compute_layout(int32_t active_count, int64_t gaussian_count, const
   layout.depth_bits = bit_length_u64(static_cast<uint64_t>(far_bits - near_bits) + 1u);
   layout.tile_bits = global_tiles > 1 ? bit_length_u64(static_cast<uint64_t>(global_tiles - 1)) : 0;
   layout.sort_key_bits = layout.tile_bits + layout.depth_bits;
-  layout.sort_digit_bits = resolve_digit_bits(options, layout.sort_key_bits);
-  layout.sort_passes = (layout.sort_key_bits + layout.sort_digit_bits - 1) / layout.sort_digit_bits;
+  // The partition's digits cover the tile index, with an image above every tile for
+  // the sentinel, and leading depth bits as far as the last digit has room.
+  const int partition_bits = bit_length_u64(static_cast<uint64_t>(global_tiles > 0 ? global_tiles : 1));
+  layout.sort_digit_bits = resolve_digit_bits(options, partition_bits + layout.depth_bits);
+  layout.sort_passes = (partition_bits + layout.sort_digit_bits - 1) / layout.sort_digit_bits;
+  int lead = layout.sort_passes * layout.sort_digit_bits - partition_bits;
+  lead = lead < layout.depth_bits ? lead : layout.depth_bits;
+  lead = lead < 32 - partition_bits ? lead : 32 - partition_bits;
+  layout.partition = PartitionKey{near_bits, lead, layout.depth_bits - lead};
   layout.sort_tile = kSortThreads * (options.sort_tile_items == 0 ? kDefaultSortItems : options.sort_tile_items);
   layout.sort_tiles = (intersection_capacity + layout.sort_tile - 1) / layout.sort_tile;
-  const int64_t radix = 1 << layout.sort_digit_bits;
-  // Per-pass sort arrays hold passes x radix slots.  With the default digit width
-  // they are sized for the larger of the 8- and 9-bit choices, which grows with the
-  // key width, so scratch sized for the largest tile count fits every smaller render.
-  int64_t pass_slots = static_cast<int64_t>(layout.sort_passes) * radix;
-  int64_t pass_count = layout.sort_passes;
-  if (options.sort_digit_bits == 0) {
-    const int64_t passes8 = (layout.sort_key_bits + 7) / 8, passes9 = (layout.sort_key_bits + 8) / 9;
-    pass_slots = passes8 * 256 > passes9 * 512 ? passes8 * 256 : passes9 * 512;
-    pass_count = passes8;
-  }
-
+  // Per-pass sort arrays hold passes x radix slots.  They are sized for passes over
+  // the whole key, at least twice what the partition uses: a size that grows with
+  // the key width alone (scratch sized for the largest tile count fits every smaller
+  // render) and does not depend on how the passes split the tile bits.
+  const int key_bits = layout.sort_key_bits;
+  const int64_t fixed_digit = options.sort_digit_bits;
+  const int64_t passes8 = (key_bits + 7) / 8, passes9 = (key_bits + 8) / 9;
+  const int64_t pass_count = fixed_digit != 0 ? (key_bits + fixed_digit - 1) / fixed_digit : passes8;
+  int64_t pass_slots = fixed_digit != 0 ? pass_count << fixed_digit
+                                        : (passes8 * 256 > passes9 * 512 ? passes8 * 256 : passes9 * 512);
+  // The flags' space later holds the tile sort's runs.
+  constexpr int64_t kRunSlots = kRunsPerSortTile * 4;
+  if (pass_slots < kRunSlots) pass_slots = kRunSlots;
   size_t offset = 0;
   layout.camera_table = offset;
   offset = align_up(offset + sizeof(CameraParams) * static_cast<size_t>(active_count > 0 ? active_count : 1));
@@ -140,7 +148,7 @@ ScratchLayout compute_layout(int32_t active_count, int64_t gaussian_count, const
   const size_t flag_tiles = layout.front ? 0u : static_cast<size_t>(layout.sort_tiles);  // no radix pass
   offset = align_up(offset + sizeof(uint32_t) * static_cast<size_t>(pass_slots) * flag_tiles);
   layout.work_counter = offset;
-  offset = align_up(offset + sizeof(uint32_t) * 4);
+  offset = align_up(offset + sizeof(uint32_t) * 8);
   layout.tile_order = offset;
   offset = align_up(offset + sizeof(int32_t) * static_cast<size_t>(global_tiles > 0 ? global_tiles : 1));
   layout.culling = options.chunk_culling != 0;
@@ -531,11 +539,15 @@ int render_submission(const vgr_scene& sc, const vgr_cameras& cams, const vgr_ou
   } else if (!opt.reuse_projection) {
     if ((status = launch_projection(sc, cams, resolved, ws, layout, scratch_base, stream)) != 0) return status;
     if ((status = mark(1)) != 0) return status;
-    if ((status = launch_sort(ws, layout, scratch_base, static_cast<uint32_t>(opt.lookback_spin_limit), stream,
-                              &sorted_in_out, sc.gaussian_ids != nullptr)) != 0)
+    if ((status = launch_sort(ws, layout, scratch_base, tiles, static_cast<uint32_t>(opt.lookback_spin_limit), stream,
+                              &sorted_in_out)) != 0)
       return status;
     if ((status = mark(2)) != 0) return status;
     if ((status = launch_ranges(ws, tiles, sorted_in_out != 0, stream)) != 0) return status;
+    if ((status = launch_tile_sort(sc, ws, layout, scratch_base, tiles, opt.tile_size, sorted_in_out != 0,
+                                   stream)) != 0)
+      return status;
+    sorted_in_out = 1 - sorted_in_out;
     if ((status = mark(3)) != 0) return status;
   } else {
     if ((status = mark(1)) != 0 || (status = mark(2)) != 0 || (status = mark(3)) != 0) return status;

@@ -39,6 +39,14 @@ struct alignas(16) CameraParams {
 };
 static_assert(sizeof(CameraParams) == 256, "camera table row must be 256 bytes");
 
+// What the radix passes partition by: the tile index followed by the leading
+// `lead_bits` bits of the depth relative to the near plane.
+struct PartitionKey {
+  uint32_t depth_base;  // float bits of the near plane
+  int32_t lead_bits;
+  int32_t lead_shift;   // relative depth bits below the leading ones
+};
+
 // Scratch layout inside workspace.scratch (all offsets 256-byte aligned).
 struct ScratchLayout {
   size_t camera_table;     // CameraParams[active_count]
@@ -48,15 +56,16 @@ struct ScratchLayout {
   size_t sort_histogram;   // uint32[passes * 256]
   size_t sort_digit_base;  // uint32[passes * 256]
   size_t sort_tickets;     // uint32[passes]
-  size_t sort_flags;       // uint32[passes * sort_tiles * 256]
+  size_t sort_flags;       // uint32[passes * sort_tiles * radix]: look-back flags, then the tile sort's runs
   size_t cull_counts;      // int64[2 * (projection_blocks + 1)]   (chunk culling only)
   size_t cull_bases;       // int64[2 * (projection_blocks + scan_blocks + 1)]
   size_t cull_masks;       // uint64[projection_blocks]: camera mask per candidate block
   size_t item_blocks;      // int32[projection_blocks]: kept block ids in order
   size_t item_masks;       // uint64[projection_blocks]
   size_t item_totals;      // int64[2]: kept item count
-  size_t work_counter;     // uint32[4]: persistent compositor queue
-  size_t tile_order;       // int32[global_tiles]: backward tile launch order (longest lists first)
+  size_t work_counter;     // uint32[8]: [0] persistent compositor queue, [4..7] queues of the tile sort
+  size_t tile_order;       // int32[global_tiles]: long-list queue of the tile sort, then the compositing order
+                           // (longest lists first), which the backward reuses
   // Tile-front ordering only (zero-sized otherwise).
   size_t front_counts;       // int64[2 * global_tiles]: (entries, 0) per tile
   size_t front_bases;        // int64[2 * (global_tiles + scan partials)]: exclusive bases per tile
@@ -90,9 +99,10 @@ struct ScratchLayout {
   int32_t cameras_per_block;
   int64_t sort_tiles;
   int32_t sort_tile;        // keys per sort tile
-  int32_t sort_passes;
+  int32_t sort_passes;      // partition passes
+  PartitionKey partition;
   int32_t sort_digit_bits;
-  int32_t sort_key_bits;
+  int32_t sort_key_bits;    // significant bits of the whole (tile, depth) order
   int32_t tile_bits;
   int32_t depth_bits;
   uint32_t depth_base;     // float bits of the near plane
@@ -104,6 +114,7 @@ constexpr int kProjectionWaves = kBlockThreads / kWave;  // waves of a projectio
 constexpr int64_t kOrderedCompositeBlocks = 32768;
 constexpr int kSortThreads = 512;      // threads per onesweep workgroup (8 waves)
 constexpr int kDefaultSortItems = 16;  // keys per thread per sort tile (tile = kSortThreads * items keys)
+constexpr int kRunsPerSortTile = 96;   // queued runs of 16 bytes per sort tile (at most 8192 keys)
 
 // Host helpers implemented in vgr_capi.hip.
 void set_error(const char* fmt, ...);
@@ -116,10 +127,15 @@ int launch_projection(const vgr_scene& scene, const vgr_cameras& cameras,
                       const vgr_options& options, const vgr_workspace& ws,
                       const ScratchLayout& layout, char* scratch,
                       hipStream_t stream);
-int launch_sort(const vgr_workspace& ws, const ScratchLayout& layout, char* scratch, uint32_t spin_limit,
-                hipStream_t stream, int* result_in_out_buffer, bool restore_id_order);
+// Partition by tile (also clears the tile ranges and the long-list queue), ranges of
+// the partitioned tiles, then the depth order inside every tile; the depth order
+// leaves the result in the other buffer pair than the partition.
+int launch_sort(const vgr_workspace& ws, const ScratchLayout& layout, char* scratch, int64_t global_tiles,
+                uint32_t spin_limit, hipStream_t stream, int* result_in_out_buffer);
 int launch_ranges(const vgr_workspace& ws, int64_t global_tiles, bool sorted_in_out,
                   hipStream_t stream);
+int launch_tile_sort(const vgr_scene& scene, const vgr_workspace& ws, const ScratchLayout& layout, char* scratch,
+                     int64_t global_tiles, int tile_size, bool partitioned_in_out, hipStream_t stream);
 int launch_composite(const vgr_scene& scene, const vgr_cameras& cameras,
                      const vgr_outputs& outputs, const vgr_options& options,
                      const vgr_workspace& ws, const ScratchLayout& layout,

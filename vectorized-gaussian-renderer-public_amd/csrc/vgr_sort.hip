@@ -1,16 +1,16 @@
-// Stable LSD radix ordering of tile intersections and tile-range marking.
+// Stable LSD radix partition of the tile intersections by tile, and tile ranges.
 //
-// Replaces the reference's cub::DeviceRadixSort::SortPairs (DoubleBuffer) call
-// and mark_sorted_tile_ranges_kernel (renderer_cuda.cu:3215-3286, 1908-1942).
+// Replaces, together with the per-tile depth sort (vgr_tile_sort.hip), the
+// reference's cub::DeviceRadixSort::SortPairs (DoubleBuffer) call and
+// mark_sorted_tile_ranges_kernel (renderer_cuda.cu:3215-3286, 1908-1942).
 //
 // Keys keep the reference layout (uint64 global_tile << 32 | float_bits(depth)).
-// The sort digits are taken from a compressed, order-preserving image of the
-// key: (tile << depth_bits) | (depth_bits_value - bits(near_plane)).  Every
-// emitted depth lies in [near, far], and positive floats order like their bit
-// patterns, so the image orders exactly like the key while needing
-// bit_length(GT-1) + bit_length(bits(far) - bits(near) + 1) bits instead of
-// 32 + bit_length(GT-1).  Sentinel keys (all ones) map to the all-ones image,
-// which is strictly larger than any valid image.
+// The digits are taken from the tile index and from as many leading bits of the
+// depth as the same number of 9-bit passes has room for: two passes cover up to
+// 2^18 tiles, where the whole key (tile and 27 depth bits) took five.  What is
+// left of the depth order costs one more read and write of the lists, and the
+// leading bits cut long lists into parts that fit the LDS.  Sentinel keys (all
+// ones) map to the all-ones image, which no tile has.
 //
 // Structure (onesweep):
 //   1. one histogram pass over the keys fills the digit histograms of every
@@ -44,17 +44,12 @@ constexpr uint32_t kFlagValueMask = kFlagPrefix - 1u;
 constexpr uint32_t kDefaultSpinLimit = 1u << 22;
 constexpr uint32_t kForceGiveUp = 0xffffffffu;  // test hook: every look-back gives up at once
 
-struct SortKeyParams {
-  int depth_bits;
-  uint32_t depth_base;
-  int key_bits;
-};
-
-__device__ __forceinline__ uint64_t compressed_key(uint64_t key, const SortKeyParams& p) {
-  if (key == kSentinelKey) return (1ull << p.key_bits) - 1ull;
-  const uint64_t tile = key >> 32;
+// Order-preserving image of a key that the partition sorts by; the sentinel's has
+// every digit at its maximum.
+__device__ __forceinline__ uint32_t key_image(uint64_t key, PartitionKey p) {
+  if (key == kSentinelKey) return 0xffffffffu;
   const uint32_t depth = static_cast<uint32_t>(key) - p.depth_base;
-  return (tile << p.depth_bits) | static_cast<uint64_t>(depth);
+  return (static_cast<uint32_t>(key >> 32) << p.lead_bits) | (depth >> p.lead_shift);
 }
 
 __device__ __forceinline__ int64_t element_count(const int64_t* counters, int64_t capacity) {
@@ -65,9 +60,8 @@ __device__ __forceinline__ int64_t element_count(const int64_t* counters, int64_
 
 __global__ __launch_bounds__(kBlockThreads) void sort_histogram_kernel(const uint64_t* __restrict__ keys,
                                                                        const int64_t* __restrict__ counters,
-                                                                       int64_t capacity, SortKeyParams kp,
-                                                                       int digit_bits, int passes,
-                                                                       uint32_t* __restrict__ histogram) {
+                                                                       int64_t capacity, PartitionKey pk, int digit_bits,
+                                                                       int passes, uint32_t* __restrict__ histogram) {
   __shared__ uint32_t local[16 * 256];
   const int radix = 1 << digit_bits;
   for (int i = threadIdx.x; i < passes * radix; i += kBlockThreads) local[i] = 0;
@@ -87,11 +81,11 @@ __global__ __launch_bounds__(kBlockThreads) void sort_histogram_kernel(const uin
   const int64_t wave_count = static_cast<int64_t>(gridDim.x) * (kBlockThreads / kWave);
   const uint64_t above = lane == kWave - 1 ? 0ull : (~0ull << (lane + 1));
   for (int64_t base = wave_id * kRuns * kWave; base < n; base += wave_count * kRuns * kWave) {
-    uint64_t ck[kRuns];
+    uint32_t image[kRuns];
 #pragma unroll
     for (int r = 0; r < kRuns; ++r) {
       const int64_t i = base + r * kWave + lane;
-      ck[r] = i < n ? compressed_key(keys[i], kp) : 0ull;
+      image[r] = i < n ? key_image(keys[i], pk) : 0u;
     }
 #pragma unroll
     for (int r = 0; r < kRuns; ++r) {
@@ -99,7 +93,7 @@ __global__ __launch_bounds__(kBlockThreads) void sort_histogram_kernel(const uin
       const uint64_t live = __ballot(valid);
       if (live == 0ull) break;
       for (int p = 0; p < passes; ++p) {
-        const uint32_t digit = static_cast<uint32_t>(ck[r] >> (p * digit_bits)) & mask;
+        const uint32_t digit = (image[r] >> (p * digit_bits)) & mask;
         const uint32_t before = __shfl_up(digit, 1, kWave);
         const bool head = valid && (lane == 0 || digit != before);
         const uint64_t heads = __ballot(head);
@@ -143,14 +137,19 @@ __global__ __launch_bounds__(kSortThreads) void sort_digit_scan_kernel(const uin
   }
 }
 
-// Clears histogram, tickets and the look-back flags of the tiles the device
-// count needs (graph-safe replacement for hipMemsetAsync).
+// Clears histogram, tickets, the look-back flags of the sort tiles the device
+// count needs, the tile ranges and the tile sort's queues (graph-safe replacement
+// for hipMemsetAsync).
 __global__ __launch_bounds__(kBlockThreads) void sort_clear_kernel(const int64_t* __restrict__ counters,
                                                                    int64_t capacity, int digit_bits, int passes,
                                                                    int64_t max_tiles, int tile_keys,
                                                                    uint32_t* __restrict__ histogram,
                                                                    uint32_t* __restrict__ tickets,
-                                                                   uint32_t* __restrict__ flags) {
+                                                                   uint32_t* __restrict__ flags,
+                                                                   int64_t global_tiles,
+                                                                   int32_t* __restrict__ tile_starts,
+                                                                   int32_t* __restrict__ tile_ends,
+                                                                   uint32_t* __restrict__ queue_state) {
   const int radix = 1 << digit_bits;
   const int64_t n = element_count(counters, capacity);
   int64_t tiles = (n + tile_keys - 1) / tile_keys;
@@ -161,6 +160,11 @@ __global__ __launch_bounds__(kBlockThreads) void sort_clear_kernel(const int64_t
     for (int64_t i = first; i < static_cast<int64_t>(passes) * radix; i += stride) histogram[i] = 0;
   }
   if (first < passes) tickets[first] = 0;
+  if (first < 4) queue_state[first] = 0;
+  for (int64_t i = first; i < global_tiles; i += stride) {
+    tile_starts[i] = 0;
+    tile_ends[i] = 0;
+  }
   const int64_t per_pass = tiles * radix;
   for (int p = 0; p < passes; ++p) {
     uint32_t* pass_flags = flags + static_cast<int64_t>(p) * max_tiles * radix;
@@ -176,7 +180,7 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
 template <int kDigitBits, int kSortItems>
 __global__ __launch_bounds__(kSortThreads) void sort_onesweep_pass_kernel(
     const uint64_t* __restrict__ keys_in, const int32_t* __restrict__ values_in, uint64_t* __restrict__ keys_out,
-    int32_t* __restrict__ values_out, const int64_t* __restrict__ counters, int64_t capacity, SortKeyParams kp,
+    int32_t* __restrict__ values_out, const int64_t* __restrict__ counters, int64_t capacity, PartitionKey pk,
     int shift, const uint32_t* __restrict__ digit_base, uint32_t* __restrict__ flags, uint32_t* __restrict__ ticket,
     int64_t* __restrict__ failures, uint32_t spin_limit) {
   constexpr int kRadix = 1 << kDigitBits;
@@ -234,7 +238,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_onesweep_pass_kernel(
   for (int r = 0; r < kSortItems; ++r) {
     const int local = wave * kWaveRun + r * kWave + lane;
     const bool valid = local < valid_count;
-    const uint32_t digit = valid ? static_cast<uint32_t>(compressed_key(keys[r], kp) >> shift) & kMask : 0u;
+    const uint32_t digit = valid ? (key_image(keys[r], pk) >> shift) & kMask : 0u;
     uint64_t peers = __ballot(valid);
 #pragma unroll
     for (int b = 0; b < kDigitBits; ++b) {
@@ -356,7 +360,7 @@ __global__ __launch_bounds__(kSortThreads) void sort_onesweep_pass_kernel(
     destinations[k] = -1;
     if (j < valid_count) {
       const uint64_t key = s_keys[j];
-      const uint32_t digit = static_cast<uint32_t>(compressed_key(key, kp) >> shift) & kMask;
+      const uint32_t digit = (key_image(key, pk) >> shift) & kMask;
       const int64_t out = static_cast<int64_t>(s_global_start[digit]) + j;
       // Always true for a consistent histogram; keeps a corrupted input in bounds.
       if (out >= 0 && out < capacity) {
@@ -434,80 +438,6 @@ __global__ __launch_bounds__(kBlockThreads) void ranges_kernel(const uint64_t* _
   }
 }
 
-// Order key of a run member: its record's Gaussian ID, then the record index
-// (IDs are unique within one camera's records; the index only orders records
-// that a corrupted list could repeat).
-__device__ __forceinline__ uint64_t tie_key(const vgr_record* __restrict__ records, int64_t visible_capacity,
-                                            int32_t value) {
-  const int32_t id = (value >= 0 && value < visible_capacity) ? records[value].gaussian_id : 0;
-  return (static_cast<uint64_t>(static_cast<uint32_t>(id)) << 32) | static_cast<uint32_t>(value);
-}
-
-// Restores Gaussian-ID order inside runs of equal keys (same tile, same depth
-// bits).  Needed only when the packed scene is stored in a spatial order, in
-// which case records of a camera are not in registration-id order.  Every
-// run is owned by the thread that sees its first element: insertion sort for
-// short runs, in-place heap sort (O(n log n)) for runs longer than 32, such as
-// the many equal depths of a fronto-parallel plane.
-__global__ __launch_bounds__(kBlockThreads) void tie_order_kernel(const uint64_t* __restrict__ keys,
-                                                                  int32_t* __restrict__ values,
-                                                                  const vgr_record* __restrict__ records,
-                                                                  const int64_t* __restrict__ counters,
-                                                                  int64_t capacity, int64_t visible_capacity) {
-  constexpr int64_t kInsertionRun = 32;
-  const int64_t n = element_count(counters, capacity);
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlockThreads + threadIdx.x; i + 1 < n;
-       i += static_cast<int64_t>(gridDim.x) * kBlockThreads) {
-    const uint64_t key = keys[i];
-    if (key == kSentinelKey || keys[i + 1] != key || (i > 0 && keys[i - 1] == key)) continue;
-    int64_t end = i + 1;
-    while (end < n && keys[end] == key) ++end;
-    int32_t* run = values + i;
-    const int64_t length = end - i;
-    if (length <= kInsertionRun) {
-      for (int64_t j = 1; j < length; ++j) {
-        const int32_t moving = run[j];
-        const uint64_t moving_key = tie_key(records, visible_capacity, moving);
-        int64_t k = j - 1;
-        while (k >= 0 && tie_key(records, visible_capacity, run[k]) > moving_key) {
-          run[k + 1] = run[k];
-          --k;
-        }
-        run[k + 1] = moving;
-      }
-      continue;
-    }
-    // Max-heap on the keys, then repeated extraction to the back.
-    auto sift_down = [&](int64_t root, int64_t size) {
-      const int32_t item = run[root];
-      const uint64_t item_key = tie_key(records, visible_capacity, item);
-      for (;;) {
-        int64_t child = 2 * root + 1;
-        if (child >= size) break;
-        uint64_t child_key = tie_key(records, visible_capacity, run[child]);
-        if (child + 1 < size) {
-          const uint64_t right_key = tie_key(records, visible_capacity, run[child + 1]);
-          if (right_key > child_key) {
-            ++child;
-            child_key = right_key;
-          }
-        }
-        if (child_key <= item_key) break;
-        run[root] = run[child];
-        root = child;
-      }
-      run[root] = item;
-    };
-    for (int64_t root = length / 2 - 1; root >= 0; --root) sift_down(root, length);
-    for (int64_t last = length - 1; last > 0; --last) {
-      const int32_t top = run[0];
-      run[0] = run[last];
-      run[last] = top;
-      sift_down(0, last);
-    }
-  }
-}
-
 __global__ void fill_u32_kernel(uint32_t* __restrict__ data, int64_t n, uint32_t value) {
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
        i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
@@ -546,21 +476,21 @@ unsigned fill_grid(int64_t n) {
 
 template <int kDigitBits>
 void launch_pass(int items, const uint64_t* keys_in, const int32_t* values_in, uint64_t* keys_out,
-                 int32_t* values_out, const int64_t* counters, int64_t capacity, SortKeyParams kp, int shift,
+                 int32_t* values_out, const int64_t* counters, int64_t capacity, PartitionKey pk, int shift,
                  const uint32_t* digit_base, uint32_t* flags, uint32_t* ticket, int64_t* failures,
                  uint32_t spin_limit, int64_t tiles, hipStream_t stream) {
   if (items == 8) {
     hipLaunchKernelGGL((sort_onesweep_pass_kernel<kDigitBits, 8>), dim3(static_cast<unsigned>(tiles)),
                        dim3(kSortThreads), 0, stream, keys_in, values_in, keys_out, values_out, counters, capacity,
-                       kp, shift, digit_base, flags, ticket, failures, spin_limit);
+                       pk, shift, digit_base, flags, ticket, failures, spin_limit);
   } else if (items == 12) {
     hipLaunchKernelGGL((sort_onesweep_pass_kernel<kDigitBits, 12>), dim3(static_cast<unsigned>(tiles)),
                        dim3(kSortThreads), 0, stream, keys_in, values_in, keys_out, values_out, counters, capacity,
-                       kp, shift, digit_base, flags, ticket, failures, spin_limit);
+                       pk, shift, digit_base, flags, ticket, failures, spin_limit);
   } else {
     hipLaunchKernelGGL((sort_onesweep_pass_kernel<kDigitBits, 16>), dim3(static_cast<unsigned>(tiles)),
                        dim3(kSortThreads), 0, stream, keys_in, values_in, keys_out, values_out, counters, capacity,
-                       kp, shift, digit_base, flags, ticket, failures, spin_limit);
+                       pk, shift, digit_base, flags, ticket, failures, spin_limit);
   }
 }
 
@@ -594,8 +524,8 @@ int launch_fill_f32(float* data, int64_t n, float value, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? 0 : VGR_E_LAUNCH;
 }
 
-int launch_sort(const vgr_workspace& ws, const ScratchLayout& layout, char* scratch, uint32_t spin_limit,
-                hipStream_t stream, int* result_in_out_buffer, bool restore_id_order) {
+int launch_sort(const vgr_workspace& ws, const ScratchLayout& layout, char* scratch, int64_t global_tiles,
+                uint32_t spin_limit, hipStream_t stream, int* result_in_out_buffer) {
   const int digit_bits = layout.sort_digit_bits;
   const int passes = layout.sort_passes;
   const int radix = 1 << digit_bits;
@@ -603,22 +533,22 @@ int launch_sort(const vgr_workspace& ws, const ScratchLayout& layout, char* scra
   uint32_t* digit_base = reinterpret_cast<uint32_t*>(scratch + layout.sort_digit_base);
   uint32_t* tickets = reinterpret_cast<uint32_t*>(scratch + layout.sort_tickets);
   uint32_t* flags = reinterpret_cast<uint32_t*>(scratch + layout.sort_flags);
-  SortKeyParams kp;
-  kp.depth_bits = layout.depth_bits;
-  kp.depth_base = layout.depth_base;
-  kp.key_bits = layout.sort_key_bits;
+  const PartitionKey pk = layout.partition;
   const int64_t capacity = ws.intersection_capacity;
   const int64_t tiles = layout.sort_tiles;
   int64_t* failures = ws.counters + VGR_COUNTER_SORT_FAILURES;
   const uint32_t limit = spin_limit == 0 ? kDefaultSpinLimit : spin_limit;
 
   hipLaunchKernelGGL(sort_clear_kernel, dim3(1024), dim3(kBlockThreads), 0, stream, ws.counters, capacity,
-                     digit_bits, passes, tiles, layout.sort_tile, histogram, tickets, flags);
+                     digit_bits, passes, tiles, layout.sort_tile, histogram, tickets, flags, global_tiles, ws.tile_starts,
+                     ws.tile_ends, reinterpret_cast<uint32_t*>(scratch + layout.work_counter) + 4);
   const int items = layout.sort_tile / kSortThreads;
   int64_t histogram_blocks = (capacity + kBlockThreads * 16 - 1) / (kBlockThreads * 16);
-  histogram_blocks = histogram_blocks > 2048 ? 2048 : (histogram_blocks < 1 ? 1 : histogram_blocks);
+  // Every workgroup ends with an atomic per digit value on the same counters: 512 of
+  // them already read at the rate of the memory.
+  histogram_blocks = histogram_blocks > 512 ? 512 : (histogram_blocks < 1 ? 1 : histogram_blocks);
   hipLaunchKernelGGL(sort_histogram_kernel, dim3(static_cast<unsigned>(histogram_blocks)), dim3(kBlockThreads), 0,
-                     stream, ws.keys_in, ws.counters, capacity, kp, digit_bits, passes, histogram);
+                     stream, ws.keys_in, ws.counters, capacity, pk, digit_bits, passes, histogram);
   hipLaunchKernelGGL(sort_digit_scan_kernel, dim3(1), dim3(kSortThreads), 0, stream, histogram, digit_bits, passes,
                      digit_base);
   const uint64_t* source_keys = ws.keys_in;
@@ -631,27 +561,27 @@ int launch_sort(const vgr_workspace& ws, const ScratchLayout& layout, char* scra
     const uint32_t* pass_base = digit_base + p * radix;
     switch (digit_bits) {
       case 4:
-        launch_pass<4>(items, source_keys, source_values, target_keys, target_values, ws.counters, capacity, kp, shift,
+        launch_pass<4>(items, source_keys, source_values, target_keys, target_values, ws.counters, capacity, pk, shift,
                        pass_base, pass_flags, tickets + p, failures, limit, tiles, stream);
         break;
       case 5:
-        launch_pass<5>(items, source_keys, source_values, target_keys, target_values, ws.counters, capacity, kp, shift,
+        launch_pass<5>(items, source_keys, source_values, target_keys, target_values, ws.counters, capacity, pk, shift,
                        pass_base, pass_flags, tickets + p, failures, limit, tiles, stream);
         break;
       case 6:
-        launch_pass<6>(items, source_keys, source_values, target_keys, target_values, ws.counters, capacity, kp, shift,
+        launch_pass<6>(items, source_keys, source_values, target_keys, target_values, ws.counters, capacity, pk, shift,
                        pass_base, pass_flags, tickets + p, failures, limit, tiles, stream);
         break;
       case 7:
-        launch_pass<7>(items, source_keys, source_values, target_keys, target_values, ws.counters, capacity, kp, shift,
+        launch_pass<7>(items, source_keys, source_values, target_keys, target_values, ws.counters, capacity, pk, shift,
                        pass_base, pass_flags, tickets + p, failures, limit, tiles, stream);
         break;
       case 9:
-        launch_pass<9>(items, source_keys, source_values, target_keys, target_values, ws.counters, capacity, kp, shift,
+        launch_pass<9>(items, source_keys, source_values, target_keys, target_values, ws.counters, capacity, pk, shift,
                        pass_base, pass_flags, tickets + p, failures, limit, tiles, stream);
         break;
       default:
-        launch_pass<8>(items, source_keys, source_values, target_keys, target_values, ws.counters, capacity, kp, shift,
+        launch_pass<8>(items, source_keys, source_values, target_keys, target_values, ws.counters, capacity, pk, shift,
                        pass_base, pass_flags, tickets + p, failures, limit, tiles, stream);
         break;
     }
@@ -663,14 +593,6 @@ int launch_sort(const vgr_workspace& ws, const ScratchLayout& layout, char* scra
     source_values = next_values;
   }
   *result_in_out_buffer = (passes % 2) == 1 ? 1 : 0;
-  if (restore_id_order) {
-    int64_t tie_blocks = (capacity + kBlockThreads * 8 - 1) / (kBlockThreads * 8);
-    tie_blocks = tie_blocks > 4096 ? 4096 : (tie_blocks < 1 ? 1 : tie_blocks);
-    hipLaunchKernelGGL(tie_order_kernel, dim3(static_cast<unsigned>(tie_blocks)), dim3(kBlockThreads), 0, stream,
-                       *result_in_out_buffer ? ws.keys_out : ws.keys_in,
-                       *result_in_out_buffer ? ws.values_out : ws.values_in, ws.records, ws.counters, capacity,
-                       ws.visible_capacity);
-  }
   const hipError_t error = hipGetLastError();
   if (error != hipSuccess) {
     set_error("sort launch failed: %s", hipGetErrorString(error));
@@ -680,10 +602,6 @@ int launch_sort(const vgr_workspace& ws, const ScratchLayout& layout, char* scra
 }
 
 int launch_ranges(const vgr_workspace& ws, int64_t global_tiles, bool sorted_in_out, hipStream_t stream) {
-  if (global_tiles > 0) {
-    launch_fill_u32(reinterpret_cast<uint32_t*>(ws.tile_starts), global_tiles, 0u, stream);
-    launch_fill_u32(reinterpret_cast<uint32_t*>(ws.tile_ends), global_tiles, 0u, stream);
-  }
   const uint64_t* keys = sorted_in_out ? ws.keys_out : ws.keys_in;
   int64_t blocks = (ws.intersection_capacity + kBlockThreads * 16 - 1) / (kBlockThreads * 16);
   blocks = blocks > 4096 ? 4096 : (blocks < 1 ? 1 : blocks);

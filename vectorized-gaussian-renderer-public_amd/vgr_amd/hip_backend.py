@@ -79,8 +79,9 @@ def emitted_sort_key_end_bit(global_tiles: int) -> int:
 
 
 def default_sort_digit_bits(key_bits: int) -> int:
-    """The library's default radix digit width: 8, or 9 where that saves a pass."""
-    return 9 if -(-key_bits // 9) < -(-key_bits // 8) else 8
+    """The library's default digit width of the partition: 9 bits, or what one pass over the whole
+    key needs."""
+    return min(9, max(4, key_bits))
 
 
 def compressed_sort_key_bits(global_tiles: int, near_plane: float, far_plane: float) -> int:
@@ -319,6 +320,9 @@ class CustomHipBackend:
         o = self.options
         tiles = self._global_tiles()
         key_bits = compressed_sort_key_bits(tiles, o.near_plane, o.far_plane)
+        # The radix passes partition by tile (one image above every tile is the sentinel's) and by the
+        # leading depth bits that fit the same number of passes.
+        partition_bits = max(tiles, 1).bit_length()
         digit_bits = o.sort_digit_bits or default_sort_digit_bits(key_bits)
         scratch = self._scratch_bytes(capacity.tile_intersections)
         n, v = capacity.tile_intersections, capacity.visible_records
@@ -356,7 +360,7 @@ class CustomHipBackend:
             "sort_key_end_bit": emitted_sort_key_end_bit(max(tiles, 1)),
             "sort_key_bits": key_bits,
             "sort_radix_digit_bits_assumption": digit_bits,
-            "sort_radix_passes_expected": math.ceil(key_bits / digit_bits),
+            "sort_radix_passes_expected": math.ceil(partition_bits / digit_bits),
         }
         return WorkspacePlan.build(buffers, facts)
 
