@@ -420,8 +420,8 @@ template <int kDegree>
 __device__ __forceinline__ void gaussian_pose_terms(const ProjectionArgs& pa, const CameraParams& cam, int32_t g,
                                                     const float (&r)[kRecordGrads], float (&pose)[kCameraGrads]) {
   bool loaded;
-  float m0, m1, m2, opacity, cov[6];
-  load_gaussian(pa, g, loaded, m0, m1, m2, opacity, cov);
+  float m0, m1, m2, opacity, cov[6], extend;
+  load_gaussian(pa, g, loaded, m0, m1, m2, opacity, cov, extend);
   constexpr int kChannels = 3 * (kDegree + 1) * (kDegree + 1);
   float f[kChannels];
   load_features<kDegree>(pa.features, g, pa.feature_width, f);
@@ -1077,8 +1077,8 @@ __global__ __launch_bounds__(kBlockThreads) void projection_backward_kernel(Proj
   const int64_t chunk = block - static_cast<int64_t>(group) * fw.chunks;
   const int64_t g = chunk * kBlockThreads + threadIdx.x;
   bool loaded;
-  float m0, m1, m2, opacity, cov[6];
-  load_gaussian(fw, g, loaded, m0, m1, m2, opacity, cov);
+  float m0, m1, m2, opacity, cov[6], extend;
+  load_gaussian(fw, g, loaded, m0, m1, m2, opacity, cov, extend);
   constexpr int kChannels = 3 * (kDegree + 1) * (kDegree + 1);
   float f[kChannels];
   float grad_f[kChannels];
@@ -1113,7 +1113,7 @@ __global__ __launch_bounds__(kBlockThreads) void projection_backward_kernel(Proj
     Projected p;
     TileRect rect;
     int tiles;
-    const bool visible = evaluate_pair(fw, cam, g, loaded, m0, m1, m2, opacity, cov, p, rect, tiles);
+    const bool visible = evaluate_pair(fw, cam, g, loaded, m0, m1, m2, opacity, cov, extend, p, rect, tiles);
     int inclusive_visible = visible ? 1 : 0;
     int inclusive_tiles = tiles;
     wave_inclusive_scan2(inclusive_visible, inclusive_tiles);

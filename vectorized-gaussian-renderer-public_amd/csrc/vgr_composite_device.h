@@ -222,10 +222,10 @@ template <int kDegree>
 __device__ __forceinline__ void record_from_gaussian(const ProjectionArgs& pa, const CameraParams& cam, int32_t g,
                                                      f32x4& a, f32x4& b, f32x4& c) {
   bool loaded;
-  float m0, m1, m2, opacity, cov[6];
-  load_gaussian(pa, g, loaded, m0, m1, m2, opacity, cov);
+  float m0, m1, m2, opacity, cov[6], extend;
+  load_gaussian(pa, g, loaded, m0, m1, m2, opacity, cov, extend);
   Projected p;
-  if (!loaded || !project_pair(cam, m0, m1, m2, opacity, cov, pa.near_plane, pa.far_plane, pa.support_sigma,
+  if (!loaded || !project_pair(cam, m0, m1, m2, opacity, cov, extend, pa.near_plane, pa.far_plane, pa.support_sigma,
                                pa.covariance_epsilon, pa.antialiased != 0, p)) {
     a = f32x4{0.0f, 0.0f, 0.0f, 0.0f};  // unreachable for listed pairs: contributes nothing
     b = f32x4{0.0f, 0.0f, 0.0f, 0.0f};

@@ -102,8 +102,8 @@ __global__ __launch_bounds__(kBlockThreads) void front_count_kernel(ProjectionAr
   if (threadIdx.x == 0) s_mask = 0ull;
   __syncthreads();
   bool loaded;
-  float m0, m1, m2, opacity, cov[6];
-  load_gaussian(args, g, loaded, m0, m1, m2, opacity, cov);
+  float m0, m1, m2, opacity, cov[6], extend;
+  load_gaussian(args, g, loaded, m0, m1, m2, opacity, cov, extend);
   int64_t visible = 0;
   uint64_t wave_mask = 0;
   for (int a = first; a < last; ++a) {
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(kBlockThreads) void front_count_kernel(ProjectionAr
     Projected p;
     TileRect rect;
     int tiles;
-    const bool seen = evaluate_pair(args, cam, g, loaded, m0, m1, m2, opacity, cov, p, rect, tiles);
+    const bool seen = evaluate_pair(args, cam, g, loaded, m0, m1, m2, opacity, cov, extend, p, rect, tiles);
     if (seen) {
       ++visible;
       const int local = static_cast<int>(static_cast<int64_t>(cam.tile_base) - group_base);
@@ -242,8 +242,8 @@ __global__ __launch_bounds__(kBlockThreads) void front_write_kernel(ProjectionAr
   }
   __syncthreads();
   bool loaded;
-  float m0, m1, m2, opacity, cov[6];
-  load_gaussian(args, g, loaded, m0, m1, m2, opacity, cov);
+  float m0, m1, m2, opacity, cov[6], extend;
+  load_gaussian(args, g, loaded, m0, m1, m2, opacity, cov, extend);
   while (cameras != 0ull) {  // uniform over the workgroup
     const int a = first + __ffsll(static_cast<unsigned long long>(cameras)) - 1;
     cameras &= cameras - 1ull;
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(kBlockThreads) void front_write_kernel(ProjectionAr
     TileRect rect;
     int tiles = 0;
     const bool seen = ((wave_cameras >> (a - first)) & 1ull) != 0ull &&
-                      evaluate_pair(args, cam, g, loaded, m0, m1, m2, opacity, cov, p, rect, tiles);
+                      evaluate_pair(args, cam, g, loaded, m0, m1, m2, opacity, cov, extend, p, rect, tiles);
     const bool ranked = seen && tiles <= kRanks;
     uint32_t rank[kRanks] = {0u, 0u, 0u, 0u};
     if (ranked) {

@@ -171,8 +171,8 @@ __global__ __launch_bounds__(kBlockThreads) void projection_count_kernel(Project
   const int64_t chunk = block - static_cast<int64_t>(group) * args.chunks;
   const int64_t g = chunk * kBlockThreads + threadIdx.x;
   bool loaded;
-  float m0, m1, m2, opacity, cov[6];
-  load_gaussian(args, g, loaded, m0, m1, m2, opacity, cov);
+  float m0, m1, m2, opacity, cov[6], extend;
+  load_gaussian(args, g, loaded, m0, m1, m2, opacity, cov, extend);
   int64_t visible = 0, intersections = 0;
   uint64_t wave_mask = 0;  // cameras with at least one visible pair among the wave's Gaussians
   const int first = group * args.cameras_per_block;
@@ -186,9 +186,9 @@ __global__ __launch_bounds__(kBlockThreads) void projection_count_kernel(Project
     bool seen;
     if constexpr (kMode == 2) {
       RayData ray;
-      seen = evaluate_ray_pair(args, cam, g, loaded, m0, m1, m2, opacity, cov, p, rect, tiles, ray);
+      seen = evaluate_ray_pair(args, cam, g, loaded, m0, m1, m2, opacity, cov, extend, p, rect, tiles, ray);
     } else {
-      seen = evaluate_pair(args, cam, g, loaded, m0, m1, m2, opacity, cov, p, rect, tiles);
+      seen = evaluate_pair(args, cam, g, loaded, m0, m1, m2, opacity, cov, extend, p, rect, tiles);
     }
     if constexpr (kMode == 1) {
       // Pixel intersections, counted by the wave together (added once, on lane 0).
@@ -237,8 +237,8 @@ __global__ __launch_bounds__(kBlockThreads, 4) void projection_write_kernel(
   const int64_t g = chunk * kBlockThreads + threadIdx.x;
   const int lane = threadIdx.x & (kWave - 1);
   bool loaded;
-  float m0, m1, m2, opacity, cov[6];
-  load_gaussian(args, g, loaded, m0, m1, m2, opacity, cov);
+  float m0, m1, m2, opacity, cov[6], extend;
+  load_gaussian(args, g, loaded, m0, m1, m2, opacity, cov, extend);
   constexpr int kChannels = 3 * (kDegree + 1) * (kDegree + 1);
   float f[kChannels];
 #pragma unroll
@@ -264,12 +264,12 @@ __global__ __launch_bounds__(kBlockThreads, 4) void projection_write_kernel(
     RayData ray;
     bool visible;
     if constexpr (kMode == 1) {
-      visible = evaluate_pair(args, cam, g, loaded, m0, m1, m2, opacity, cov, p, rect, tiles);
+      visible = evaluate_pair(args, cam, g, loaded, m0, m1, m2, opacity, cov, extend, p, rect, tiles);
       tiles = 0;  // pixel intersections are placed by the wave together below
     } else if constexpr (kMode == 2) {
-      visible = evaluate_ray_pair(args, cam, g, loaded, m0, m1, m2, opacity, cov, p, rect, tiles, ray);
+      visible = evaluate_ray_pair(args, cam, g, loaded, m0, m1, m2, opacity, cov, extend, p, rect, tiles, ray);
     } else {
-      visible = evaluate_pair(args, cam, g, loaded, m0, m1, m2, opacity, cov, p, rect, tiles);
+      visible = evaluate_pair(args, cam, g, loaded, m0, m1, m2, opacity, cov, extend, p, rect, tiles);
     }
     int inclusive_visible = visible ? 1 : 0;
     int inclusive_tiles = tiles;

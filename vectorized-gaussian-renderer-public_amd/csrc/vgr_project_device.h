@@ -39,15 +39,25 @@ struct Projected {
   int radius_x, radius_y;
 };
 
+// Standard deviations from the mean that a splat of this opacity (at least the alpha
+// threshold) reaches.  It does not depend on the camera: a logarithm, a division and
+// a square root that the projection kernels evaluate once per Gaussian instead of
+// once per pair.
+__device__ __forceinline__ float splat_extend(float opacity, float support_sigma) {
+  return fminf(support_sigma, sqrtf(2.0f * vgr_logf(opacity / VGR_ALPHA_THRESHOLD)));
+}
+
 // Screen-space projection of one (camera, Gaussian) pair.  Operation order
 // follows renderer_cuda.cu:614-1055 term by term (left-to-right sums, no
 // contraction), with vgr_logf in place of __logf.
+// `extend` is the Gaussian's splat_extend, which the antialiased mode forms anew from
+// the compensated opacity.
 // kRay: exact-ray renders cull on the support quadric's screen ellipse instead
 // (ray_extent), so the screen-space cull of the splat is skipped here.
 template <bool kRay = false>
 __device__ __forceinline__ bool project_pair(
     const CameraParams& cam, float m0, float m1, float m2, float opacity,
-    const float* cov, float near_plane, float far_plane, float support_sigma,
+    const float* cov, float extend, float near_plane, float far_plane, float support_sigma,
     float covariance_epsilon, bool antialiased, Projected& out) {
   if (!(opacity >= VGR_ALPHA_THRESHOLD)) return false;
   const float* e = cam.env;
@@ -103,9 +113,8 @@ __device__ __forceinline__ bool project_pair(
         original / determinant));
     opacity *= compensation;
     if (!(opacity >= VGR_ALPHA_THRESHOLD)) return false;
+    extend = splat_extend(opacity, support_sigma);
   }
-  const float opacity_extend = sqrtf(2.0f * vgr_logf(opacity / VGR_ALPHA_THRESHOLD));
-  const float extend = fminf(support_sigma, opacity_extend);
   const int radius_x = float_to_int_clamped(ceilf(extend * sqrtf(cov00)));
   const int radius_y = float_to_int_clamped(ceilf(extend * sqrtf(cov11)));
   if (radius_x <= 0 && radius_y <= 0) return false;
@@ -270,14 +279,16 @@ struct TileRect {
   int min_x, min_y, max_x, max_y;
 };
 
-// Tile rectangle of a projected splat (renderer_cuda.cu:1729-1748).
+// Tile rectangle of a projected splat (renderer_cuda.cu:1729-1748).  The tile size is
+// a power of two, so its reciprocal is exact and the products round like the
+// reference's quotients.
 __device__ __forceinline__ TileRect tile_rect(const Projected& p, int tile_size, int tiles_x, int tiles_y) {
-  const float ts = static_cast<float>(tile_size);
+  const float per_tile = 1.0f / static_cast<float>(tile_size);
   TileRect rect;
-  rect.min_x = max(0, static_cast<int>(floorf(p.mean_x / ts - static_cast<float>(p.radius_x) / ts)));
-  rect.min_y = max(0, static_cast<int>(floorf(p.mean_y / ts - static_cast<float>(p.radius_y) / ts)));
-  rect.max_x = min(tiles_x, static_cast<int>(ceilf(p.mean_x / ts + static_cast<float>(p.radius_x) / ts)));
-  rect.max_y = min(tiles_y, static_cast<int>(ceilf(p.mean_y / ts + static_cast<float>(p.radius_y) / ts)));
+  rect.min_x = max(0, static_cast<int>(floorf(p.mean_x * per_tile - static_cast<float>(p.radius_x) * per_tile)));
+  rect.min_y = max(0, static_cast<int>(floorf(p.mean_y * per_tile - static_cast<float>(p.radius_y) * per_tile)));
+  rect.max_x = min(tiles_x, static_cast<int>(ceilf(p.mean_x * per_tile + static_cast<float>(p.radius_x) * per_tile)));
+  rect.max_y = min(tiles_y, static_cast<int>(ceilf(p.mean_y * per_tile + static_cast<float>(p.radius_y) * per_tile)));
   return rect;
 }
 
@@ -441,10 +452,11 @@ __device__ __forceinline__ bool resolve_block(const ProjectionArgs& args, int64_
 // Pair results for one camera of the group; identical in both passes.
 __device__ __forceinline__ bool evaluate_pair(const ProjectionArgs& args, const CameraParams& cam, int64_t g,
                                               bool loaded, float m0, float m1, float m2, float opacity,
-                                              const float* cov, Projected& p, TileRect& rect, int& tiles) {
+                                              const float* cov, float extend, Projected& p, TileRect& rect,
+                                              int& tiles) {
   tiles = 0;
   if (!loaded || cam.scene_slot < 0 || g < cam.gaussian_begin || g >= cam.gaussian_end) return false;
-  if (!project_pair(cam, m0, m1, m2, opacity, cov, args.near_plane, args.far_plane, args.support_sigma,
+  if (!project_pair(cam, m0, m1, m2, opacity, cov, extend, args.near_plane, args.far_plane, args.support_sigma,
                     args.covariance_epsilon, args.antialiased != 0, p)) {
     return false;
   }
@@ -546,11 +558,11 @@ __device__ __forceinline__ bool dense_rect_reaches(const TileRect& rect, uint32_
 // and radii (binning and culling); `ray` receives the record's precision data.
 __device__ __forceinline__ bool evaluate_ray_pair(const ProjectionArgs& args, const CameraParams& cam, int64_t g,
                                                   bool loaded, float m0, float m1, float m2, float opacity,
-                                                  const float* cov, Projected& p, TileRect& rect, int& tiles,
-                                                  RayData& ray) {
+                                                  const float* cov, float extend, Projected& p, TileRect& rect,
+                                                  int& tiles, RayData& ray) {
   tiles = 0;
   if (!loaded || cam.scene_slot < 0 || g < cam.gaussian_begin || g >= cam.gaussian_end) return false;
-  if (!project_pair<true>(cam, m0, m1, m2, opacity, cov, args.near_plane, args.far_plane, args.support_sigma,
+  if (!project_pair<true>(cam, m0, m1, m2, opacity, cov, extend, args.near_plane, args.far_plane, args.support_sigma,
                           args.covariance_epsilon, args.antialiased != 0, p)) {
     return false;
   }
@@ -562,9 +574,9 @@ __device__ __forceinline__ bool evaluate_ray_pair(const ProjectionArgs& args, co
 
 
 __device__ __forceinline__ void load_gaussian(const ProjectionArgs& args, int64_t g, bool& loaded, float& m0,
-                                              float& m1, float& m2, float& opacity, float* cov) {
+                                              float& m1, float& m2, float& opacity, float* cov, float& extend) {
   loaded = g < args.gaussian_count;
-  m0 = m1 = m2 = opacity = 0.0f;
+  m0 = m1 = m2 = opacity = extend = 0.0f;
   for (int i = 0; i < 6; ++i) cov[i] = 0.0f;
   if (!loaded) return;
   m0 = args.means[g * 3 + 0];
@@ -572,6 +584,7 @@ __device__ __forceinline__ void load_gaussian(const ProjectionArgs& args, int64_
   m2 = args.means[g * 3 + 2];
   opacity = args.opacities[g];
   for (int i = 0; i < 6; ++i) cov[i] = args.covariances[g * 6 + i];
+  if (opacity >= VGR_ALPHA_THRESHOLD && args.antialiased == 0) extend = splat_extend(opacity, args.support_sigma);
 }
 
 __device__ __forceinline__ int64_t wave_sum_i64(int64_t value) {
