@@ -554,7 +554,6 @@ __global__ __launch_bounds__(kTileSize* kTileSize) void composite_backward_kerne
   const float px = static_cast<float>(pixel_x) + 0.5f;
   const float py = static_cast<float>(pixel_y) + 0.5f;
   const float rect_x0 = static_cast<float>(tile_x * kTileSize) + 0.5f;
-  const float rect_x1 = rect_x0 + static_cast<float>(kTileSize - 1);
   const float rect_y_base = static_cast<float>(tile_y * kTileSize) + 0.5f;
 
   // Per-pixel upstream gradients; depth = D / A is folded into dL/dD and dL/dA.
@@ -617,7 +616,7 @@ __global__ __launch_bounds__(kTileSize* kTileSize) void composite_backward_kerne
         s_blended[slot] = 0u;
       }
     }
-    build_wave_lists<kTileSize, kBatch>(s, next_a, next_b, next_c, count, lane, rect_x0, rect_x1, rect_y_base);
+    build_wave_lists<kTileSize, kBatch>(s, next_a, next_b, next_c, count, lane, rect_x0, rect_y_base);
     if (b > 0) {
       const int64_t start = batch_start - kBatch;
       gather_batch<kThreads, kBatch, kPerThread, true>(args.sorted_values, args.records, args.visible_capacity,
@@ -740,7 +739,7 @@ using BackwardArgsFor = typename std::conditional<(kDegree < 0), CompositeBackwa
 // Wave-per-tile form for 16x16 tiles: one wave64 owns the whole tile and every
 // lane four pixels (column lane % 16, rows lane / 16 + 4k).  Pixel k of every
 // lane lies in the tile's k-th band of four rows, so the per-band reach mask of
-// a splat (the same conservative ellipse box as the forward's per-wave lists)
+// a splat (the same conservative ellipse test as the forward's per-wave lists)
 // is a uniform branch.  Each lane sums its four pixels' gradient terms of a
 // splat; a transposing butterfly (DPP and permlane swaps) sums them over the
 // wave into ten lanes, which park them in LDS, and after the batch every lane
@@ -783,7 +782,6 @@ __global__ __launch_bounds__(kWave, (kDegree < 0 ? 5 : (kDegree >= 2 ? 2 : 3))) 
   const int pixel_x = tile_x * kTileSize + (lane % kTileSize);
   const float px = static_cast<float>(pixel_x) + 0.5f;
   const float rect_x0 = static_cast<float>(tile_x * kTileSize) + 0.5f;
-  const float rect_x1 = rect_x0 + static_cast<float>(kTileSize - 1);
   const float rect_y_base = static_cast<float>(tile_y * kTileSize) + 0.5f;
 
   float py[kBands], transmittance[kBands], grad_r[kBands], grad_g[kBands], grad_b[kBands], grad_d[kBands],
@@ -885,19 +883,11 @@ __global__ __launch_bounds__(kWave, (kDegree < 0 ? 5 : (kDegree >= 2 ? 2 : 3))) 
         s_colour[slot] = staged.colour;
         s_record[slot] = next_ids[k];
         s_blended[slot] = 0u;
-        float half_x, half_y;
-        if (splat_extent(next_a[k], next_b[k], staged.shading.z, half_x, half_y)) {
-          const float mx = next_a[k].x, my = next_a[k].y;
-          if (fabsf(mx - fminf(fmaxf(mx, rect_x0), rect_x1)) <= half_x) {
+        const SplatReach reach(next_a[k], next_b[k], staged.shading.z);
 #pragma unroll
-            for (int band = 0; band < kBands; ++band) {
-              const float y0 = rect_y_base + static_cast<float>(4 * band);
-              const float y1 = y0 + 3.0f;
-              if (fabsf(my - fminf(fmaxf(my, y0), y1)) <= half_y) bands |= 1u << band;
-            }
-          }
-        } else {
-          bands = (1u << kBands) - 1u;
+        for (int band = 0; band < kBands; ++band) {
+          const float y0 = rect_y_base + static_cast<float>(4 * band);
+          if (reach.hits(rect_x0, y0, static_cast<float>(kTileSize - 1), 3.0f)) bands |= 1u << band;
         }
         // Drop bands whose pixels all stopped blending before this list position.
         const int position = static_cast<int>(batch_start - range_start) + slot;

@@ -206,7 +206,6 @@ __device__ __forceinline__ void composite_tile(const CompositeArgsFor<kDegree>& 
   const float py = static_cast<float>(pixel_y) + 0.5f;
   // Pixel-centre rectangle of tile column span and of each wave's rows.
   const float rect_x0 = static_cast<float>(tile_x * kTileSize) + 0.5f;
-  const float rect_x1 = rect_x0 + static_cast<float>(kTileSize - 1);
   const float rect_y_base = static_cast<float>(tile_y * kTileSize) + 0.5f;
 
   float transmittance = 1.0f;
@@ -226,7 +225,7 @@ __device__ __forceinline__ void composite_tile(const CompositeArgsFor<kDegree>& 
     for (int64_t batch_start = range_start; batch_start < range_end; batch_start += kBatch) {
       const int count = static_cast<int>(range_end - batch_start < kBatch ? range_end - batch_start : kBatch);
       __syncthreads();  // previous batch fully consumed
-      build_wave_lists<kTileSize, kBatch>(s, next_a, next_b, next_c, count, lane, rect_x0, rect_x1, rect_y_base);
+      build_wave_lists<kTileSize, kBatch>(s, next_a, next_b, next_c, count, lane, rect_x0, rect_y_base);
       if (batch_start + kBatch < range_end) {
         gather_any<kThreads, kBatch, kPerThread, kDegree, kCheckpoint>(args, cam, batch_start + kBatch, range_end,
                                                                        lane, next_a, next_b, next_c);
@@ -274,7 +273,7 @@ __device__ __forceinline__ void composite_tile(const CompositeArgsFor<kDegree>& 
             const float dx = px - g.x, dy = py - g.y;
             const float power = g.z * dx * dx + g.w * dx * dy + shading[u].x * dy * dy;
             passes[u] = !(power > 0.0f || power < shading[u].z);
-            alphas[u] = passes[u] ? fminf(VGR_MAX_ALPHA, shading[u].y * vgr_expf_nonpositive(power)) : 0.0f;
+            alphas[u] = passes[u] ? fminf(VGR_MAX_ALPHA, shading[u].y * vgr_expf_bounded(power)) : 0.0f;
           }
 #pragma unroll
           for (int u = 0; u < kUnroll; ++u) {
@@ -293,7 +292,7 @@ __device__ __forceinline__ void composite_tile(const CompositeArgsFor<kDegree>& 
           const float delta_y = py - g.y;
           const float power = g.z * delta_x * delta_x + g.w * delta_x * delta_y + sh.x * delta_y * delta_y;
           if (!(power > 0.0f || power < sh.z)) {
-            if (blend(item, sh, fminf(VGR_MAX_ALPHA, sh.y * vgr_expf_nonpositive(power)))) done = true;
+            if (blend(item, sh, fminf(VGR_MAX_ALPHA, sh.y * vgr_expf_bounded(power)))) done = true;
           }
         }
       }

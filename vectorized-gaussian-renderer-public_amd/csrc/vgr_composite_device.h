@@ -1,6 +1,6 @@
 // Device-side compositing helpers shared by the forward compositor and the
 // backward (gradient) compositor: record gathering, the staged splat form with
-// its exact log-threshold, the conservative ellipse box, and the per-wave
+// its exact log-threshold, the conservative ellipse test, and the per-wave
 // ordered sub-lists.  Both passes therefore visit the same (pixel, splat) pairs
 // and evaluate them with bit-identical arithmetic.
 #ifndef VGR_COMPOSITE_DEVICE_H
@@ -62,7 +62,7 @@ __device__ __forceinline__ void gather_batch(const int32_t* __restrict__ sorted_
 }
 
 // Margin subtracted from the per-Gaussian log-threshold: far larger than the
-// error of vgr_logf/vgr_expf and of the alpha product, so "power below the
+// error of the logarithm, of vgr_expf and of the alpha product, so "power below the
 // threshold" implies the exact alpha test fails.
 constexpr float kThresholdMargin = 1.0e-4f;
 
@@ -80,39 +80,66 @@ struct StagedSplat {
 __device__ __forceinline__ StagedSplat stage_record(const f32x4& a, const f32x4& b, const f32x4& c) {
   StagedSplat s;
   const float opacity = b.y;
-  // power < threshold  =>  min(0.99, opacity * exp(power)) < 1/255 exactly.
-  const float threshold = opacity > 0.0f ? vgr_logf(VGR_ALPHA_THRESHOLD / opacity) - kThresholdMargin
-                                         : __int_as_float(0x7f800000);
+  // power < threshold  =>  min(0.99, opacity * exp(power)) < 1/255 exactly.  The
+  // hardware's logarithm and reciprocal are good to one unit in the last place.
+  const float threshold =
+      opacity > 0.0f ? 0.6931472f * __builtin_amdgcn_logf(VGR_ALPHA_THRESHOLD * __builtin_amdgcn_rcpf(opacity)) -
+                           kThresholdMargin
+                     : __int_as_float(0x7f800000);
   s.geometry = f32x4{a.x, a.y, -0.5f * a.z, -a.w};
   s.shading = f32x4{-0.5f * b.x, opacity, threshold, b.z};
   s.colour = f32x4{b.w, c.x, c.y, c.z};
   return s;
 }
 
-// Half extents of a box containing every pixel offset whose float-evaluated
-// power can reach the threshold: the ellipse d^T C d <= R^2 (R^2 = -2 threshold)
-// inflated by a bound on the rounding error of the power expression, which
-// grows with the conic's condition.  Returns false when no finite box is
-// certain (non-positive-definite or extremely anisotropic conic).
-__device__ __forceinline__ bool splat_extent(const f32x4& a, const f32x4& b, float threshold, float& half_x,
-                                             float& half_y) {
-  const double c0 = a.z, c1 = a.w, c2 = b.x;
-  const double det = c0 * c2 - c1 * c1;
-  if (!(det > 0.0) || !(threshold < 0.0f)) return false;
-  const double sxx = c2 / det;
-  const double syy = c0 / det;
-  const double condition = (fabs(c0) + 2.0 * fabs(c1) + fabs(c2)) * (sxx + syy);
-  if (!(condition < 1.0e5)) return false;
-  const double r2 = -2.0 * static_cast<double>(threshold) * (1.0 + 1.0e-6 * condition) * 1.001 + 1.0e-6;
-  half_x = static_cast<float>(sqrt(r2 * sxx)) + 1.0e-3f;
-  half_y = static_cast<float>(sqrt(r2 * syy)) + 1.0e-3f;
-  return true;
-}
+// Where a splat can reach alpha 1/255: the pixel centres at which its quadratic form
+// c0*dx*dx + 2*c1*dx*dy + c2*dy*dy stays within -2 * threshold, inflated by more than
+// the rounding of this test and of the pixels' own evaluation, which grow with the
+// conic's condition.  A rectangle of pixel centres is reached when the smallest value
+// of the form over it is within the bound; leaving a splat out of the lists of blocks
+// it does not reach is therefore exact.  The test against the ellipse itself keeps
+// fewer entries than one against its bounding box, and takes the hardware's
+// reciprocal (one unit in the last place, far inside the margin) where the box took
+// divisions and square roots in double.
+struct SplatReach {
+  float mean_x, mean_y, c0, c1, c2;
+  float slope_x, slope_y;  // -c1 / c0, -c1 / c2: where the form is least along an edge
+  float bound;
+  bool certain;            // the form is clearly positive definite
+
+  __device__ __forceinline__ SplatReach(const f32x4& a, const f32x4& b, float threshold)
+      : mean_x(a.x), mean_y(a.y), c0(a.z), c1(a.w), c2(b.x) {
+    const float product = c1 * c1;
+    const float det = fmaf(c0, c2, -product) - fmaf(c1, c1, -product);  // two roundings, whatever cancels
+    const float condition = (c0 + 2.0f * fabsf(c1) + c2) * (c0 + c2) * __builtin_amdgcn_rcpf(det);
+    slope_x = -c1 * __builtin_amdgcn_rcpf(c0);
+    slope_y = -c1 * __builtin_amdgcn_rcpf(c2);
+    bound = -2.0f * threshold * (1.001f + 4.0e-6f * condition) + 1.0e-5f;
+    certain = det > 0.0f && c0 > 0.0f && c2 > 0.0f && condition < 1.0e5f;
+  }
+
+  // Whether a pixel centre in [x0, x0 + width] x [y0, y0 + height] may be reached.
+  __device__ __forceinline__ bool hits(float x0, float y0, float width, float height) const {
+    const float x_low = x0 - mean_x, y_low = y0 - mean_y;
+    const float x_high = x_low + width, y_high = y_low + height;
+    // Nearest offsets to the mean, zero where the rectangle spans it.  The form is least
+    // on an edge that faces the mean, or at the mean.
+    const float near_x = fminf(fmaxf(0.0f, x_low), x_high);
+    const float near_y = fminf(fmaxf(0.0f, y_low), y_high);
+    const float along_y = fminf(fmaxf(slope_y * near_x, y_low), y_high);
+    const float along_x = fminf(fmaxf(slope_x * near_y, x_low), x_high);
+    const float on_x = c0 * near_x * near_x + 2.0f * c1 * near_x * along_y + c2 * along_y * along_y;
+    const float on_y = c0 * along_x * along_x + 2.0f * c1 * along_x * near_y + c2 * near_y * near_y;
+    float least = near_x != 0.0f ? on_x : 3.4e38f;
+    least = near_y != 0.0f ? fminf(least, on_y) : least;
+    return !certain || least <= bound || (near_x == 0.0f && near_y == 0.0f);
+  }
+};
 
 // Stages one batch of gathered records into LDS and builds, for every wave of
-// the tile, the ordered list of batch slots whose conservative ellipse box
-// reaches that wave's rows of pixel centres.  A slot left out of a wave's list
-// has alpha < 1/255 at every pixel of the wave, so skipping it is exact.
+// the tile, the ordered list of batch slots whose ellipse reaches that wave's
+// block of pixel centres.  A slot left out of a wave's list has alpha < 1/255 at
+// every pixel of the wave, so skipping it is exact.
 // Slots are ordered by (slice k, source wave, lane) = batch-slot order = depth
 // order.  Ends with a __syncthreads(); the caller synchronizes before it (LDS
 // of the previous batch fully consumed).
@@ -152,9 +179,7 @@ __device__ __forceinline__ void build_wave_lists(WaveLists<kTileSize, kBatch>& s
                                                  const f32x4 (&na)[WaveLists<kTileSize, kBatch>::kPerThread],
                                                  const f32x4 (&nb)[WaveLists<kTileSize, kBatch>::kPerThread],
                                                  const f32x4 (&nc)[WaveLists<kTileSize, kBatch>::kPerThread],
-                                                 int count, int lane, float rect_x0, float rect_x1,
-                                                 float rect_y_base) {
-  (void)rect_x1;
+                                                 int count, int lane, float rect_x0, float rect_y_base) {
   using L = WaveLists<kTileSize, kBatch>;
   constexpr int kThreads = L::kThreads;
   constexpr int kWaves = L::kWaves;
@@ -171,19 +196,13 @@ __device__ __forceinline__ void build_wave_lists(WaveLists<kTileSize, kBatch>& s
       s.geometry[slot] = staged.geometry;
       s.shading[slot] = staged.shading;
       s.colour[slot] = staged.colour;
-      float half_x, half_y;
-      if (splat_extent(na[k], nb[k], staged.shading.z, half_x, half_y)) {
-        const float mx = na[k].x, my = na[k].y;
+      const SplatReach reach(na[k], nb[k], staged.shading.z);
+      constexpr float kSpan = static_cast<float>(L::kBlock - 1);
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) {
-          const float x0 = rect_x0 + static_cast<float>((w % L::kBlocksX) * L::kBlock);
-          const float y0 = rect_y_base + static_cast<float>((w / L::kBlocksX) * L::kBlock);
-          const float gap_x = fabsf(mx - fminf(fmaxf(mx, x0), x0 + static_cast<float>(L::kBlock - 1)));
-          const float gap_y = fabsf(my - fminf(fmaxf(my, y0), y0 + static_cast<float>(L::kBlock - 1)));
-          if (gap_x <= half_x && gap_y <= half_y) wave_bits[k] |= 1u << w;
-        }
-      } else {
-        wave_bits[k] = (1u << kWaves) - 1u;  // no certain box: every wave evaluates it
+      for (int w = 0; w < kWaves; ++w) {
+        const float x0 = rect_x0 + static_cast<float>((w % L::kBlocksX) * L::kBlock);
+        const float y0 = rect_y_base + static_cast<float>((w / L::kBlocksX) * L::kBlock);
+        if (reach.hits(x0, y0, kSpan, kSpan)) wave_bits[k] |= 1u << w;
       }
     }
   }

@@ -73,6 +73,18 @@ VGR_HD float vgr_bits_float(uint32_t bits) {
 #endif
 }
 
+// 2^f = 1 + f q(f) on [-0.5, 0.5], q of degree 4 (Lawson-weighted Chebyshev
+// least squares on relative error, coefficients rounded to binary32).  The
+// unit constant term makes 2^0 exactly 1.
+VGR_HD float vgr_exp2_fraction(float f) {
+  float q = 0x1.5bba14p-10f;
+  q = VGR_FMAF(q, f, 0x1.3cea88p-7f);
+  q = VGR_FMAF(q, f, 0x1.c6b752p-5f);
+  q = VGR_FMAF(q, f, 0x1.ebf9bcp-3f);
+  q = VGR_FMAF(q, f, 0x1.62e42ap-1f);
+  return VGR_FMAF(q, f, 1.0f);
+}
+
 // 2^x.  x is clamped to [-126, 127] so the result stays a normal float (or
 // the largest finite power), which keeps denormal handling out of the picture.
 VGR_HD float vgr_exp2f(float x) {
@@ -80,16 +92,7 @@ VGR_HD float vgr_exp2f(float x) {
   x = x > 127.0f ? 127.0f : x;
   const float n = VGR_RINTF(x);
   const float f = x - n;  // exact: |f| <= 0.5 and shares n's ulp scale
-  // 2^f = 1 + f q(f) on [-0.5, 0.5], q of degree 4 (Lawson-weighted Chebyshev
-  // least squares on relative error, coefficients rounded to binary32).  The
-  // unit constant term makes 2^0 exactly 1.
-  float q = 0x1.5bba14p-10f;
-  q = VGR_FMAF(q, f, 0x1.3cea88p-7f);
-  q = VGR_FMAF(q, f, 0x1.c6b752p-5f);
-  q = VGR_FMAF(q, f, 0x1.ebf9bcp-3f);
-  q = VGR_FMAF(q, f, 0x1.62e42ap-1f);
-  const float p = VGR_FMAF(q, f, 1.0f);
-  return VGR_LDEXPF(p, (int)n);
+  return VGR_LDEXPF(vgr_exp2_fraction(f), (int)n);
 }
 
 // e^x evaluated as 2^(x * log2(e)).
@@ -106,13 +109,16 @@ VGR_HD float vgr_expf_nonpositive(float x) {
   y = y < -126.0f ? -126.0f : y;
   const float n = VGR_RINTF(y);
   const float f = y - n;
-  float q = 0x1.5bba14p-10f;
-  q = VGR_FMAF(q, f, 0x1.3cea88p-7f);
-  q = VGR_FMAF(q, f, 0x1.c6b752p-5f);
-  q = VGR_FMAF(q, f, 0x1.ebf9bcp-3f);
-  q = VGR_FMAF(q, f, 0x1.62e42ap-1f);
-  const float p = VGR_FMAF(q, f, 1.0f);
-  return VGR_LDEXPF(p, (int)n);
+  return VGR_LDEXPF(vgr_exp2_fraction(f), (int)n);
+}
+
+// vgr_expf_nonpositive for -87 < x <= 0 (or NaN), where the lower clamp never acts
+// either: the same result bit for bit.  Powers that pass the compositor's threshold
+// are above ln(1/255) - 1e-4.
+VGR_HD float vgr_expf_bounded(float x) {
+  const float y = x * 1.44269504088896340736f;
+  const float n = VGR_RINTF(y);
+  return VGR_LDEXPF(vgr_exp2_fraction(y - n), (int)n);
 }
 
 // Natural logarithm of a positive, normal, finite x.  x = m * 2^e with
