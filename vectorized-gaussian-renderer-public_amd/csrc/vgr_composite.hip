@@ -23,8 +23,8 @@ namespace {
 using namespace dev;
 
 // ---- tile launch order -------------------------------------------------------
-// Blocks sorted by descending list length (counting sort on length / 8, capped):
-// the longest tiles start first and the short ones fill in behind them, instead of
+// Blocks sorted by descending list length (counting sort, 32 buckets an octave): the
+// longest tiles start first and the short ones fill in behind them, instead of
 // a long tile starting late and running alone at the end of the grid.  One
 // workgroup; the order inside a length bucket is unspecified (it changes only the
 // schedule: every tile's outputs are its own).  On 16 cameras of 512x512 (lists
@@ -32,11 +32,21 @@ using namespace dev;
 // forward+backward 9.6 -> 8.0 ms.
 constexpr int kOrderBuckets = 1024;
 constexpr int kOrderThreads = 1024;
+// A tile is long when its list holds more than half of the entries that a CU gets on
+// average: a wave that walks it alone would still run when the other CUs are done.
+// Lists count up to 4,096 entries towards the average, since a tile with more is mostly
+// opaque before its end.  Compositing of 48 room cameras of 160x120 in three submissions
+// of 1,280 tiles, and of one submission of 1,024 tiles of 128x128 views whose lists (23k
+// on average) are opaque early: no tile long 1,829 and 540 us; without the cap 1,699 and
+// 704; cap 4,096 1,186 and 763; cap 2,048 1,127 and 779, but 215 instead of 177 for the
+// 1,200 tiles of a VGA view over 1M Gaussians.
+constexpr int32_t kLongCap = 4096;
+constexpr float kLongShare = 0.5f / 256.0f;
 
-__device__ __forceinline__ int order_bucket(const CameraParams* __restrict__ table,
-                                            const int32_t* __restrict__ tile_starts,
-                                            const int32_t* __restrict__ tile_ends, int active_count,
-                                            int uniform_tiles, int64_t block) {
+__device__ __forceinline__ int32_t list_length(const CameraParams* __restrict__ table,
+                                               const int32_t* __restrict__ tile_starts,
+                                               const int32_t* __restrict__ tile_ends, int active_count,
+                                               int uniform_tiles, int64_t block) {
   int active;
   int64_t image_tile;
   if (uniform_tiles > 0) {
@@ -52,21 +62,35 @@ __device__ __forceinline__ int order_bucket(const CameraParams* __restrict__ tab
   const uint32_t global_tile = table[active].tile_base + static_cast<uint32_t>(image_tile);
   const int64_t start = tile_starts[global_tile];
   const int64_t end = tile_ends[global_tile];
-  const int64_t bucket = (start >= 0 && end > start ? end - start : 0) >> 3;
-  return static_cast<int>(bucket < kOrderBuckets - 1 ? bucket : kOrderBuckets - 1);
+  return static_cast<int32_t>(start >= 0 && end > start ? end - start : 0);
+}
+
+// Empty lists, then 32 buckets an octave (at most 31 octaves).
+__device__ __forceinline__ int order_bucket(int32_t length) {
+  return length <= 0 ? 0 : static_cast<int>(__float_as_uint(static_cast<float>(length)) >> 18) - (127 << 5) + 1;
 }
 
 __global__ __launch_bounds__(kOrderThreads) void tile_order_kernel(const CameraParams* __restrict__ table,
                                                                    const int32_t* __restrict__ tile_starts,
                                                                    const int32_t* __restrict__ tile_ends,
                                                                    int active_count, int uniform_tiles, int64_t blocks,
-                                                                   int32_t* __restrict__ order) {
+                                                                   int32_t* __restrict__ order,
+                                                                   uint32_t* __restrict__ long_tiles) {
   __shared__ uint32_t s_next[kOrderBuckets];
   __shared__ uint32_t s_wave_totals[kOrderThreads / kWave];
+  __shared__ float s_wave_entries[kOrderThreads / kWave];
   for (int i = threadIdx.x; i < kOrderBuckets; i += kOrderThreads) s_next[i] = 0;
   __syncthreads();
+  float entries = 0.0f;
   for (int64_t b = threadIdx.x; b < blocks; b += kOrderThreads) {
-    atomicAdd(&s_next[order_bucket(table, tile_starts, tile_ends, active_count, uniform_tiles, b)], 1u);
+    const int32_t length = list_length(table, tile_starts, tile_ends, active_count, uniform_tiles, b);
+    atomicAdd(&s_next[order_bucket(length)], 1u);
+    entries += static_cast<float>(length < kLongCap ? length : kLongCap);
+  }
+  if (long_tiles != nullptr) {  // uniform
+#pragma unroll
+    for (int offset = kWave / 2; offset > 0; offset >>= 1) entries += __shfl_xor(entries, offset, kWave);
+    if ((threadIdx.x & (kWave - 1)) == 0) s_wave_entries[threadIdx.x / kWave] = entries;
   }
   __syncthreads();
   // Exclusive scan in descending bucket order: thread t owns bucket kOrderBuckets-1-t.
@@ -86,9 +110,15 @@ __global__ __launch_bounds__(kOrderThreads) void tile_order_kernel(const CameraP
   uint32_t prefix = 0;
   for (int w = 0; w < wave; ++w) prefix += s_wave_totals[w];
   s_next[bucket] = prefix + inclusive - count;
+  if (long_tiles != nullptr) {
+    float total = 0.0f;
+    for (int w = 0; w < kOrderThreads / kWave; ++w) total += s_wave_entries[w];
+    const int limit = order_bucket(static_cast<int32_t>(total * kLongShare));
+    if (bucket == limit) *long_tiles = prefix + inclusive - count;  // the tiles of the buckets above
+  }
   __syncthreads();
   for (int64_t b = threadIdx.x; b < blocks; b += kOrderThreads) {
-    const int k = order_bucket(table, tile_starts, tile_ends, active_count, uniform_tiles, b);
+    const int k = order_bucket(list_length(table, tile_starts, tile_ends, active_count, uniform_tiles, b));
     order[atomicAdd(&s_next[k], 1u)] = static_cast<int32_t>(b);
   }
 }
@@ -109,6 +139,7 @@ struct CompositeArgs {
   int64_t gaussian_count;
   uint32_t* work_counter;  // persistent queue counter (zeroed before the launch)
   const int32_t* tile_order;  // launch order of the (camera, tile) items
+  const uint32_t* long_tiles;  // how many of the first in that order are long
   int64_t total_items;     // (camera, tile) items in the launch
   int active_count;
   int uniform_tiles;     // tiles per camera when every camera has the same resolution, else 0
@@ -140,6 +171,29 @@ __device__ __forceinline__ int64_t item_total(const Args& args) {
     if (args.item_count != nullptr) return static_cast<int64_t>(*args.item_count);
   }
   return args.total_items;
+}
+
+// Writes a finished pixel (renderer_cuda.cu:2264-2304).
+template <bool kFull>
+__device__ __forceinline__ void store_pixel(const CompositeArgs& args, int64_t pixel, float transmittance, float red,
+                                            float green, float blue, float depth_sum, float best_weight,
+                                            int best_gaussian) {
+  const float accumulated_alpha = 1.0f - transmittance;
+  if (args.output_srgb) {
+    red = vgr_linear_to_srgb(red);
+    green = vgr_linear_to_srgb(green);
+    blue = vgr_linear_to_srgb(blue);
+  }
+  args.rgb[pixel * 3 + 0] = red;
+  args.rgb[pixel * 3 + 1] = green;
+  args.rgb[pixel * 3 + 2] = blue;
+  if (kFull) {
+    args.alpha[pixel] = accumulated_alpha;
+    args.depth[pixel] = accumulated_alpha > 1.0e-8f ? depth_sum / accumulated_alpha : __int_as_float(0x7f800000);
+    const bool labelled = best_weight >= 0.0f && accumulated_alpha >= args.semantic_min_alpha &&
+                          best_gaussian >= 0 && best_gaussian < args.gaussian_count;
+    args.semantic[pixel] = labelled ? args.semantic_ids[best_gaussian] : -1;
+  }
 }
 
 // Gathers one batch: stored records (kDegree < 0) or records recomputed from
@@ -174,12 +228,12 @@ __device__ __forceinline__ void gather_any(const CompositeArgsFor<kDegree>& args
 // kCheckpoint the final transmittance and the list position one past the last
 // blended splat are stored per pixel for the backward pass.
 template <int kTileSize, int kBatch, bool kFull, bool kCount, bool kCheckpoint, int kDegree = -1>
-__device__ __forceinline__ void composite_tile(const CompositeArgsFor<kDegree>& args, int64_t block) {
+__device__ __forceinline__ void composite_tile(const CompositeArgsFor<kDegree>& args, int64_t block,
+                                               WaveLists<kTileSize, kBatch>& s) {
   using Lists = WaveLists<kTileSize, kBatch>;
   constexpr int kThreads = Lists::kThreads;
   constexpr int kPerThread = Lists::kPerThread;
   static_assert(kThreads % kWave == 0, "tile must be a whole number of waves");
-  __shared__ Lists s;
 
   int active;
   int64_t image_tile;
@@ -320,25 +374,240 @@ __device__ __forceinline__ void composite_tile(const CompositeArgsFor<kDegree>& 
   }
   if (!valid_pixel) return;
   const int64_t pixel = cam.pixel_offset + static_cast<int64_t>(pixel_y) * cam.width + pixel_x;
-  const float accumulated_alpha = 1.0f - transmittance;
-  if (args.output_srgb) {
-    red = vgr_linear_to_srgb(red);
-    green = vgr_linear_to_srgb(green);
-    blue = vgr_linear_to_srgb(blue);
-  }
-  args.rgb[pixel * 3 + 0] = red;
-  args.rgb[pixel * 3 + 1] = green;
-  args.rgb[pixel * 3 + 2] = blue;
-  if (kFull) {
-    args.alpha[pixel] = accumulated_alpha;
-    args.depth[pixel] = accumulated_alpha > 1.0e-8f ? depth_sum / accumulated_alpha : __int_as_float(0x7f800000);
-    const bool labelled = best_weight >= 0.0f && accumulated_alpha >= args.semantic_min_alpha &&
-                          best_gaussian >= 0 && best_gaussian < args.gaussian_count;
-    args.semantic[pixel] = labelled ? args.semantic_ids[best_gaussian] : -1;
-  }
+  store_pixel<kFull>(args, pixel, transmittance, red, green, blue, depth_sum, best_weight, best_gaussian);
   if (kCheckpoint) {
     args.final_transmittance[pixel] = transmittance;
     args.last_blended[pixel] = last_blended;
+  }
+}
+
+// ---- few long lists: a workgroup per 8x8 block ---------------------------------------
+//
+// Where a handful of tiles outlast the rest of the grid (a small image; tiles that
+// look out of a closed scene and never saturate), the time is what one wave takes for
+// its block's list: some 45 vector instructions an entry, four cycles each.  Only a
+// third of them, the blend, has to follow the order of the list.  Here a workgroup
+// renders one 8x8 block: one wave blends while three evaluate the alphas of the
+// entries ahead into LDS, on the other SIMDs of the CU, and all four stage the list,
+// keeping the entries whose ellipse reaches the block.  The alphas, their tests and the
+// blends are those of composite_tile, in the same order.  On a full grid it costs 1.4
+// to 1.7 times the time of composite_tile (every block stages the whole list, the
+// alphas pass through LDS), so only long tiles take it: a 128x96 view of 20k Gaussians
+// composites in 74 us instead of 126, one 320x240 view of 100k in 79 instead of 131,
+// 48 room cameras of 160x120 in 1,186 instead of 1,829.
+constexpr int kBlockBatch = 256;                      // list entries staged at a time, one per thread
+constexpr int kBlockShare = 8;                        // entries of a step per evaluating wave
+constexpr int kBlockStep = 3 * kBlockShare;
+constexpr int kBlockRows = 16 * kBlockStep;           // kept entries: staged while a whole batch fits
+
+struct BlockShared {
+  f32x4 geometry[kBlockRows];
+  f32x4 shading[kBlockRows];
+  f32x4 colour[kBlockRows];
+  int32_t position[kBlockRows];                       // list position
+  float alpha[2][kBlockStep][kWave];                  // one step is blended while the next is evaluated
+  uint32_t live[2][3];                                // its entries with an alpha at some pixel
+  uint32_t totals[2][4];
+  uint32_t open;                                      // a pixel goes on
+};
+
+template <int kTileSize, bool kFull, bool kCheckpoint, int kDegree>
+__device__ __forceinline__ void composite_block(const CompositeArgsFor<kDegree>& args, int64_t block, int quadrant,
+                                                BlockShared& s) {
+  constexpr int kBlocksX = kTileSize / 8;
+  int active;
+  int64_t image_tile;
+  if (args.uniform_tiles > 0) {
+    active = static_cast<int>(block / args.uniform_tiles);
+    if (active >= args.active_count) return;
+    image_tile = block - static_cast<int64_t>(active) * args.uniform_tiles;
+  } else {
+    active = find_active_camera(args.table, args.active_count, block);
+    image_tile = block - args.table[active].active_tile_begin;
+    if (image_tile >= static_cast<int64_t>(args.table[active].tiles_x) * args.table[active].tiles_y) return;
+  }
+  const CameraParams& cam = args.table[active];
+  if (cam.camera < 0) return;
+  const uint32_t global_tile = cam.tile_base + static_cast<uint32_t>(image_tile);
+  const int block_x = static_cast<int>(image_tile % cam.tiles_x) * kTileSize + (quadrant % kBlocksX) * 8;
+  const int block_y = static_cast<int>(image_tile / cam.tiles_x) * kTileSize + (quadrant / kBlocksX) * 8;
+  if (block_x >= cam.width || block_y >= cam.height) return;
+  const int thread = threadIdx.x;
+  const int lane = thread & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(thread / kWave);  // 0 blends, 1 to 3 evaluate
+  const int pixel_x = block_x + (lane & 7), pixel_y = block_y + (lane >> 3);
+  const bool valid_pixel = pixel_x < cam.width && pixel_y < cam.height;
+  const float px = static_cast<float>(pixel_x) + 0.5f, py = static_cast<float>(pixel_y) + 0.5f;
+  const float x0 = static_cast<float>(block_x) + 0.5f, y0 = static_cast<float>(block_y) + 0.5f;
+  const uint64_t below = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
+
+  float transmittance = 1.0f;
+  float red = 0.0f, green = 0.0f, blue = 0.0f, depth_sum = 0.0f;
+  float best_weight = -1.0f;
+  int best_gaussian = -1;
+  int last_blended = 0;
+  bool done = !valid_pixel;
+
+  const int64_t range_start = args.tile_starts[global_tile];
+  const int64_t range_end = args.tile_ends[global_tile];
+  if (range_start >= 0 && range_end > range_start) {
+    // Blends the step evaluated into alpha buffer `buffer`, entries [first, first + kBlockStep).
+    const auto blend_step = [&](int buffer, int first) {
+      uint32_t live = s.live[buffer][0] | (s.live[buffer][1] << kBlockShare) | (s.live[buffer][2] << (2 * kBlockShare));
+      live = __builtin_amdgcn_readfirstlane(live);
+      constexpr int kGroup = 4;  // entries whose LDS reads are issued together
+#pragma unroll
+      for (int u0 = 0; u0 < kBlockStep; u0 += kGroup) {
+        if (((live >> u0) & ((1u << kGroup) - 1u)) == 0u) continue;  // uniform
+        float alphas[kGroup], depths[kGroup];
+        f32x4 colours[kGroup];
+#pragma unroll
+        for (int u = 0; u < kGroup; ++u) {
+          alphas[u] = s.alpha[buffer][u0 + u][lane];
+          colours[u] = s.colour[first + u0 + u];
+          depths[u] = kFull ? s.shading[first + u0 + u].w : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < kGroup; ++u) {
+          if (alphas[u] > 0.0f && !done) {
+            const float next = transmittance * (1.0f - alphas[u]);
+            if (next <= VGR_TRANSMITTANCE_THRESHOLD) {
+              done = true;
+            } else {
+              const float weight = transmittance * alphas[u];
+              red = fmaf(weight, colours[u].x, red);
+              green = fmaf(weight, colours[u].y, green);
+              blue = fmaf(weight, colours[u].z, blue);
+              if (kFull) {
+                depth_sum = fmaf(weight, depths[u], depth_sum);
+                if (weight > best_weight) {
+                  best_weight = weight;
+                  best_gaussian = __float_as_int(colours[u].w);
+                }
+              }
+              if (kCheckpoint) last_blended = s.position[first + u0 + u] + 1;
+              transmittance = next;
+            }
+          }
+        }
+      }
+    };
+    // This wave's share of the step: alphas of entries that pass, else 0.
+    const auto evaluate_step = [&](int buffer, int first, int kept) {
+      const int share = (wave - 1) * kBlockShare;
+      uint32_t live = 0u;
+#pragma unroll
+      for (int u = 0; u < kBlockShare; ++u) {
+        const int row = first + share + u;
+        if (row < kept) {  // uniform
+          const f32x4 g = s.geometry[row];
+          const f32x4 sh = s.shading[row];
+          const float dx = px - g.x, dy = py - g.y;
+          const float power = g.z * dx * dx + g.w * dx * dy + sh.x * dy * dy;
+          const float alpha = fminf(VGR_MAX_ALPHA, sh.y * vgr_expf_bounded(power));
+          const bool passes = !(power > 0.0f || power < sh.z) && alpha >= VGR_ALPHA_THRESHOLD;
+          s.alpha[buffer][share + u][lane] = passes ? alpha : 0.0f;
+          if (__ballot(passes) != 0ull) live |= 1u << u;
+        } else {
+          s.alpha[buffer][share + u][lane] = 0.0f;
+        }
+      }
+      if (lane == 0) s.live[buffer][wave - 1] = live;
+    };
+
+    f32x4 next_a[1] = {}, next_b[1] = {}, next_c[1] = {};
+    gather_any<kBlockBatch, kBlockBatch, 1, kDegree, kCheckpoint>(args, cam, range_start, range_end, thread, next_a,
+                                                                 next_b, next_c);
+    int64_t batch_start = range_start;
+    int parity = 0;
+    while (batch_start < range_end) {  // uniform
+      // Stage batches until the kept entries fill half of the rows.
+      int kept = 0;
+      while (batch_start < range_end && kept <= kBlockRows - kBlockBatch) {
+        const bool listed = batch_start + thread < range_end;
+        StagedSplat staged;
+        bool keep = false;
+        if (listed) {
+          staged = stage_record(next_a[0], next_b[0], next_c[0]);
+          const SplatReach reach(next_a[0], next_b[0], staged.shading.z);
+          keep = reach.hits(x0, y0, 7.0f, 7.0f);
+        }
+        const uint64_t vote = __ballot(keep);
+        if (lane == 0) s.totals[parity][wave] = static_cast<uint32_t>(__popcll(vote));
+        __syncthreads();
+        int row = kept + static_cast<int>(__popcll(vote & below));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int total = static_cast<int>(s.totals[parity][q]);
+          if (q < wave) row += total;
+          kept += total;
+        }
+        parity ^= 1;  // the next batch's totals do not meet late readers of these
+        if (keep) {
+          s.geometry[row] = staged.geometry;
+          s.shading[row] = staged.shading;
+          s.colour[row] = staged.colour;
+          s.position[row] = static_cast<int32_t>(batch_start - range_start) + thread;
+        }
+        batch_start += kBlockBatch;
+        if (batch_start < range_end) {
+          gather_any<kBlockBatch, kBlockBatch, 1, kDegree, kCheckpoint>(args, cam, batch_start, range_end, thread,
+                                                                       next_a, next_b, next_c);
+        }
+      }
+      __syncthreads();
+      // Steps: wave 0 blends one behind the evaluating waves.
+      int buffer = 0;
+      for (int first = 0; first < kept + kBlockStep; first += kBlockStep, buffer ^= 1) {
+        if (wave == 0) {
+          if (first > 0) blend_step(buffer ^ 1, first - kBlockStep);
+        } else if (first < kept) {
+          evaluate_step(buffer, first, kept);
+        }
+        __syncthreads();
+      }
+      if (wave == 0) {
+        const uint64_t going = __ballot(!done);
+        if (lane == 0) s.open = going != 0ull ? 1u : 0u;
+      }
+      __syncthreads();
+      if (s.open == 0u) break;  // uniform
+    }
+  }
+  if (wave != 0 || !valid_pixel) return;
+  const int64_t pixel = cam.pixel_offset + static_cast<int64_t>(pixel_y) * cam.width + pixel_x;
+  store_pixel<kFull>(args, pixel, transmittance, red, green, blue, depth_sum, best_weight, best_gaussian);
+  if (kCheckpoint) {
+    args.final_transmittance[pixel] = transmittance;
+    args.last_blended[pixel] = last_blended;
+  }
+}
+
+template <int kTileSize, bool kFull, bool kCheckpoint>
+__global__ __launch_bounds__(kBlockBatch) void composite_block_kernel(CompositeArgs args) {
+  __shared__ BlockShared s;
+  constexpr int kBlocks = kTileSize * kTileSize / 64;
+  composite_block<kTileSize, kFull, kCheckpoint, -1>(args, args.tile_order[blockIdx.x / kBlocks],
+                                                     static_cast<int>(blockIdx.x % kBlocks), s);
+}
+
+// Over a queue of tiles whose length is known on the device only.
+template <int kTileSize, bool kFull, bool kCheckpoint, int kDegree>
+__global__ __launch_bounds__(kBlockBatch) void composite_block_persistent_kernel(CompositeArgsFor<kDegree> args) {
+  constexpr int kBlocks = kTileSize * kTileSize / 64;
+  __shared__ BlockShared s;
+  __shared__ int64_t s_item;
+  const int64_t total = item_total(args) * kBlocks;
+  for (;;) {
+    if (threadIdx.x == 0) s_item = static_cast<int64_t>(atomicAdd(args.work_counter, 1u));
+    __syncthreads();
+    const int64_t item = s_item;
+    __syncthreads();
+    if (item >= total) break;
+    composite_block<kTileSize, kFull, kCheckpoint, kDegree>(
+        args, args.tile_order != nullptr ? args.tile_order[item / kBlocks] : item / kBlocks,
+        static_cast<int>(item % kBlocks), s);
+    __syncthreads();
   }
 }
 
@@ -397,7 +666,7 @@ __global__ __launch_bounds__(256) void composite_pixels_kernel(CompositeArgs arg
     const float dy = py - a.y;
     const float power = -0.5f * (a.z * dx * dx + 2.0f * a.w * dx * dy + b.x * dy * dy);
     if (power > 0.0f || power < -20.0f) continue;
-    const float alpha = fminf(VGR_MAX_ALPHA, b.y * vgr_expf_nonpositive(power));
+    const float alpha = fminf(VGR_MAX_ALPHA, b.y * vgr_expf_bounded(power));
     if (alpha < VGR_ALPHA_THRESHOLD) continue;
     const float next_transmittance = transmittance * (1.0f - alpha);
     if (next_transmittance <= VGR_TRANSMITTANCE_THRESHOLD) break;
@@ -423,22 +692,7 @@ __global__ __launch_bounds__(256) void composite_pixels_kernel(CompositeArgs arg
     }
   }
   const int64_t pixel = cam.pixel_offset + static_cast<int64_t>(pixel_y) * cam.width + pixel_x;
-  const float accumulated_alpha = 1.0f - transmittance;
-  if (args.output_srgb) {
-    red = vgr_linear_to_srgb(red);
-    green = vgr_linear_to_srgb(green);
-    blue = vgr_linear_to_srgb(blue);
-  }
-  args.rgb[pixel * 3 + 0] = red;
-  args.rgb[pixel * 3 + 1] = green;
-  args.rgb[pixel * 3 + 2] = blue;
-  if (kFull) {
-    args.alpha[pixel] = accumulated_alpha;
-    args.depth[pixel] = accumulated_alpha > 1.0e-8f ? depth_sum / accumulated_alpha : __int_as_float(0x7f800000);
-    const bool labelled = best_weight >= 0.0f && accumulated_alpha >= args.semantic_min_alpha &&
-                          best_gaussian >= 0 && best_gaussian < args.gaussian_count;
-    args.semantic[pixel] = labelled ? args.semantic_ids[best_gaussian] : -1;
-  }
+  store_pixel<kFull>(args, pixel, transmittance, red, green, blue, depth_sum, best_weight, best_gaussian);
 }
 
 // ---- exact-ray compositing ---------------------------------------------------------
@@ -598,22 +852,7 @@ __global__ __launch_bounds__(kRaster* kRaster) void composite_ray_kernel(Composi
   }
   if (!valid_pixel) return;
   const int64_t pixel = cam.pixel_offset + static_cast<int64_t>(pixel_y) * cam.width + pixel_x;
-  const float accumulated_alpha = 1.0f - transmittance;
-  if (args.output_srgb) {
-    red = vgr_linear_to_srgb(red);
-    green = vgr_linear_to_srgb(green);
-    blue = vgr_linear_to_srgb(blue);
-  }
-  args.rgb[pixel * 3 + 0] = red;
-  args.rgb[pixel * 3 + 1] = green;
-  args.rgb[pixel * 3 + 2] = blue;
-  if (kFull) {
-    args.alpha[pixel] = accumulated_alpha;
-    args.depth[pixel] = accumulated_alpha > 1.0e-8f ? depth_sum / accumulated_alpha : __int_as_float(0x7f800000);
-    const bool labelled = best_weight >= 0.0f && accumulated_alpha >= args.semantic_min_alpha &&
-                          best_gaussian >= 0 && best_gaussian < args.gaussian_count;
-    args.semantic[pixel] = labelled ? args.semantic_ids[best_gaussian] : -1;
-  }
+  store_pixel<kFull>(args, pixel, transmittance, red, green, blue, depth_sum, best_weight, best_gaussian);
 }
 
 template <int kRaster>
@@ -648,7 +887,8 @@ template <int kTileSize, int kBatch, bool kFull, bool kCount, bool kCheckpoint, 
 __global__ __launch_bounds__(kTileSize* kTileSize, (kCompositeWavesPerSimd<kTileSize, kBatch, kCount, false, kDegree>)) void
 composite_kernel(CompositeArgsFor<kDegree> args) {
   const int64_t block = args.tile_order != nullptr ? args.tile_order[blockIdx.x] : blockIdx.x;
-  composite_tile<kTileSize, kBatch, kFull, kCount, kCheckpoint, kDegree>(args, block);
+  __shared__ WaveLists<kTileSize, kBatch> s;
+  composite_tile<kTileSize, kBatch, kFull, kCount, kCheckpoint, kDegree>(args, block, s);
 }
 
 // Persistent form: a fixed grid whose workgroups pull (camera, tile) items from
@@ -657,6 +897,7 @@ composite_kernel(CompositeArgsFor<kDegree> args) {
 template <int kTileSize, int kBatch, bool kFull, bool kCount, bool kCheckpoint, int kDegree = -1>
 __global__ __launch_bounds__(kTileSize* kTileSize, (kCompositeWavesPerSimd<kTileSize, kBatch, kCount, true, kDegree>)) void
 composite_persistent_kernel(CompositeArgsFor<kDegree> args) {
+  __shared__ WaveLists<kTileSize, kBatch> s;
   __shared__ int64_t s_item;
   const int64_t total = item_total(args);
   for (;;) {
@@ -666,13 +907,91 @@ composite_persistent_kernel(CompositeArgsFor<kDegree> args) {
     __syncthreads();
     if (item >= total) break;
     composite_tile<kTileSize, kBatch, kFull, kCount, kCheckpoint, kDegree>(
-        args, args.tile_order != nullptr ? args.tile_order[item] : item);
+        args, args.tile_order != nullptr ? args.tile_order[item] : item, s);
   }
 }
+
+// The long tiles of a grid by block, the others whole.  The longest of both start
+// first, four blocks and a whole tile in turn: with all blocks in front, the whole
+// tiles just below the limit started late and ran on at the end (16 views of 128x128
+// over 1M Gaussians: 933 us, in turn 763).
+constexpr int kMixedWavesPerSimd = 5;  // what the LDS allows
+
+template <int kBatch, bool kFull, bool kCheckpoint>
+__global__ __launch_bounds__(kBlockBatch, kMixedWavesPerSimd) void composite_mixed_kernel(CompositeArgs args) {
+  constexpr int kBlocks = 4;
+  using Lists = WaveLists<16, kBatch>;
+  __shared__ alignas(16) char lds[sizeof(Lists) > sizeof(BlockShared) ? sizeof(Lists) : sizeof(BlockShared)];
+  const int64_t long_tiles = *args.long_tiles;
+  const int64_t whole_tiles = args.total_items - long_tiles;
+  const int64_t pairs = long_tiles < whole_tiles ? long_tiles : whole_tiles;
+  const int64_t item = blockIdx.x;
+  int64_t tile;
+  int quadrant = -1;
+  if (item < pairs * (kBlocks + 1)) {
+    tile = item / (kBlocks + 1);
+    quadrant = static_cast<int>(item % (kBlocks + 1));
+    if (quadrant == kBlocks) {
+      tile += long_tiles;
+      quadrant = -1;
+    }
+  } else if (pairs < long_tiles) {
+    const int64_t rest = item - pairs * (kBlocks + 1);
+    tile = pairs + rest / kBlocks;
+    quadrant = static_cast<int>(rest % kBlocks);
+    if (tile >= long_tiles) return;
+  } else {
+    tile = item - long_tiles * (kBlocks - 1);
+    if (tile >= args.total_items) return;
+  }
+  tile = args.tile_order[tile];
+  if (quadrant >= 0) {
+    composite_block<16, kFull, kCheckpoint, -1>(args, tile, quadrant, *reinterpret_cast<BlockShared*>(lds));
+  } else {
+    composite_tile<16, kBatch, kFull, false, kCheckpoint, -1>(args, tile, *reinterpret_cast<Lists*>(lds));
+  }
+}
+
+// Grids up to this many tiles: at five workgroups a CU all of them are resident, so the
+// lower occupancy of the mixed kernel (five waves a SIMD for eight) costs little.  1,200
+// tiles: VGA views of 100k, 300k and 1M Gaussians 51 -> 43, 134 -> 109 and 168 -> 177 us,
+// four 320x240 views of 500k 294 -> 313, of a room 154 -> 83.  At 2,400 and 3,600 tiles of
+// open scenes the occupancy alone costs 36 and 41 %.
+constexpr int64_t kMixedCompositeTiles = 1280;
+// 8x8 tiles are a block each; up to this many all take the block kernel.  2,400 tiles
+// 166 -> 81 us, 4,800 tiles 124 -> 128 (open scene) and 176 -> 115 (room); 14,400 tiles
+// would go 182 -> 253.
+constexpr int64_t kBlockCompositeTiles = 5120;
 
 template <int kTileSize, int kBatch, bool kFull, bool kCount, bool kCheckpoint = false, int kDegree = -1>
 void launch_variant(const CompositeArgsFor<kDegree>& args, int64_t blocks, int persistent, hipStream_t stream) {
   const dim3 block(kTileSize * kTileSize);
+  if constexpr (!kCount) {
+    constexpr int kBlocks = kTileSize * kTileSize / 64;
+    if constexpr (kDegree >= 0) {
+      // The tiles left open: few, with the longest lists, so always by block.  1024 room
+      // cameras of 160x120 over 5M Gaussians (121 such tiles, lists up to 200k): 7.4 ->
+      // 4.4 ms, 256 of 2M with checkpoints (385 tiles) 0.97 -> 0.79.
+      if (args.item_count != nullptr) {
+        hipLaunchKernelGGL((composite_block_persistent_kernel<kTileSize, kFull, kCheckpoint, kDegree>),
+                           dim3(static_cast<unsigned>(persistent * 2)), dim3(kBlockBatch), 0, stream, args);
+        return;
+      }
+    } else if (persistent == 0) {
+      const dim3 grid(static_cast<unsigned>(blocks * kBlocks));
+      if constexpr (kTileSize == 16) {
+        if (blocks <= kMixedCompositeTiles) {
+          hipLaunchKernelGGL((composite_mixed_kernel<kBatch, kFull, kCheckpoint>), grid, dim3(kBlockBatch), 0, stream,
+                             args);
+          return;
+        }
+      } else if (blocks <= kBlockCompositeTiles) {
+        hipLaunchKernelGGL((composite_block_kernel<kTileSize, kFull, kCheckpoint>), grid, dim3(kBlockBatch), 0,
+                           stream, args);
+        return;
+      }
+    }
+  }
   if (persistent > 0) {
     const int64_t grid = blocks < persistent ? blocks : persistent;
     hipLaunchKernelGGL((composite_persistent_kernel<kTileSize, kBatch, kFull, kCount, kCheckpoint, kDegree>),
@@ -760,10 +1079,11 @@ void launch_batch(int batch, bool full, const CompositeArgs& args, int64_t block
 }  // namespace
 
 int launch_tile_order(const CameraParams* table, const int32_t* tile_starts, const int32_t* tile_ends,
-                      int active_count, int uniform_tiles, int64_t blocks, int32_t* order, hipStream_t stream) {
+                      int active_count, int uniform_tiles, int64_t blocks, int32_t* order, hipStream_t stream,
+                      uint32_t* long_tiles) {
   if (blocks <= 0 || active_count <= 0) return 0;
   hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(kOrderThreads), 0, stream, table, tile_starts, tile_ends,
-                     active_count, uniform_tiles, blocks, order);
+                     active_count, uniform_tiles, blocks, order, long_tiles);
   const hipError_t error = hipGetLastError();
   if (error != hipSuccess) {
     set_error("tile order launch failed: %s", hipGetErrorString(error));
@@ -871,9 +1191,10 @@ int launch_composite(const vgr_scene& scene, const vgr_cameras& cameras, const v
   if (blocks <= kOrderedCompositeBlocks) {
     int32_t* order = reinterpret_cast<int32_t*>(const_cast<char*>(scratch) + layout.tile_order);
     const int order_status = launch_tile_order(args.table, args.tile_starts, args.tile_ends, args.active_count,
-                                               args.uniform_tiles, blocks, order, stream);
+                                               args.uniform_tiles, blocks, order, stream, args.work_counter + 1);
     if (order_status != 0) return order_status;
     args.tile_order = order;
+    args.long_tiles = args.work_counter + 1;
   }
   const int persistent = options.persistent_composite;
   if (persistent > 0) launch_fill_u32(args.work_counter, 1, 0u, stream);
