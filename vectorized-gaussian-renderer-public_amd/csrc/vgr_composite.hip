@@ -705,23 +705,51 @@ __global__ __launch_bounds__(256) void composite_pixels_kernel(CompositeArgs arg
 // ray's closest approach m (0 beyond the support, capped at 1), each entry with
 // alpha > 0 is blended, and the pixel stops after the entry that takes its
 // transmittance to 1e-4.
-__device__ __forceinline__ float ray_alpha(float ray_x, float ray_y, const f32x4& a, const f32x4& b,
-                                           const f32x4& c, float support_sigma) {
-  // a = (P00, P01, P02, P11), b = (P12, P22, Pm0, Pm1), c = (Pm2, mPm, opacity, depth).
-  const float along = a.x * ray_x * ray_x + 2.0f * a.y * ray_x * ray_y + 2.0f * a.z * ray_x + a.w * ray_y * ray_y +
-                      2.0f * b.x * ray_y + b.y;
-  if (!(along > 0.0f)) return 0.0f;
+//
+// Bound by vector instructions on large grids and by the latency of the gathers on
+// small ones.  The closest approach is first tested without its division (ray_misses),
+// four entries at a time; the division, the exponential and the blend follow where a
+// ray of the wave may pass within the support.  The next batch is loaded while this
+// one is composited, and the raster tiles of a bin, which stage the same list, run on
+// one XCD.  One VGA view of 300k Gaussians 292 -> 232 us, six 333x251 views of 200k
+// 620 -> 536, four 320x240 views of 200k with 8x8 tiles 366 -> 329; 16 VGA views of 1M
+// stay at 4.18 ms (86M staged entries, most of those kept hit some ray of their wave).
+struct RayApproach {
+  float along, cross2;  // the squared approach is mPm - cross2 / along
+};
+
+// a = (P00, 2 P01, 2 P02, P11), b = (2 P12, P22, Pm0, Pm1), c = (Pm2, mPm, opacity, depth).
+__device__ __forceinline__ RayApproach ray_approach(float ray_x, float ray_y, const f32x4& a, const f32x4& b,
+                                                    const f32x4& c) {
+  RayApproach r;
+  r.along = a.x * ray_x * ray_x + a.y * ray_x * ray_y + a.z * ray_x + a.w * ray_y * ray_y + b.x * ray_y + b.y;
   const float cross = ray_x * b.z + ray_y * b.w + c.x;
-  const float distance2 = fmaxf(0.0f, c.y - cross * cross / along);
-  if (distance2 > support_sigma * support_sigma) return 0.0f;
-  return fminf(1.0f, c.z * vgr_expf(-0.5f * distance2));
+  r.cross2 = cross * cross;
+  return r;
 }
 
+// The ray's alpha is 0: it runs away from the splat, or its approach is beyond the
+// support by more than the rounding of the exact test in ray_alpha (mPm lowered by
+// 2^-20 of itself, against 2^-24 for each of the four roundings; the constant covers
+// products in the denormal range).  `limit` is the squared support raised by 2^-20.
+__device__ __forceinline__ bool ray_misses(const RayApproach& r, float mpm, float limit) {
+  const float beyond = fmaf(mpm, 1.0f - 0x1p-20f, -limit);
+  return !(r.along > 0.0f) || r.cross2 < fmaf(beyond, r.along, -1.0e-36f);
+}
+
+__device__ __forceinline__ float ray_alpha(const RayApproach& r, float mpm, float opacity, float support_sigma) {
+  const float distance2 = fmaxf(0.0f, mpm - r.cross2 / r.along);
+  if (distance2 > support_sigma * support_sigma) return 0.0f;
+  return fminf(1.0f, opacity * vgr_expf_nonpositive(-0.5f * distance2));
+}
+
+constexpr int kXcds = 8;
+constexpr int kXcdBins = 4;  // 1, 4 and 16 measure the same within 2 %
+
 template <int kRaster, bool kFull>
-__global__ __launch_bounds__(kRaster* kRaster) void composite_ray_kernel(CompositeArgs args,
+__global__ __launch_bounds__(kRaster* kRaster, kRaster == 16 ? 4 : 1) void composite_ray_kernel(CompositeArgs args,
                                                                          const float* __restrict__ ray_records,
-                                                                         float support_sigma, int raster_tiles_x,
-                                                                         int raster_tiles, int bin_size) {
+                                                                         float support_sigma, int bins, int bin_size) {
   constexpr int kThreads = kRaster * kRaster;
   __shared__ f32x4 s_a[kThreads];
   __shared__ f32x4 s_b[kThreads];
@@ -738,19 +766,25 @@ __global__ __launch_bounds__(kRaster* kRaster) void composite_ray_kernel(Composi
   const int wave = static_cast<int>(threadIdx.x) / kWave;
   const int wave_lane = static_cast<int>(threadIdx.x) & (kWave - 1);
   const int block_x0 = (wave % kBlocksX) * 8, block_y0 = (wave / kBlocksX) * 8;
-  const int64_t block = blockIdx.x;
-  const int active = static_cast<int>(block / raster_tiles);
+  // Workgroups go round robin over the XCDs: those of one XCD (blockIdx.x mod kXcds)
+  // take kXcdBins neighbouring bins at a time, the raster tiles of a bin in turn.
+  const int split = bin_size / kRaster;
+  const int64_t turn = blockIdx.x / kXcds;
+  const int64_t bin_turn = turn / (split * split);
+  const int part = static_cast<int>(turn - bin_turn * (split * split));
+  const int64_t bin = (bin_turn / kXcdBins * kXcds + blockIdx.x % kXcds) * kXcdBins + bin_turn % kXcdBins;
+  const int active = static_cast<int>(bin / bins);
   if (active >= args.active_count) return;
   const CameraParams& cam = args.table[active];
   if (cam.camera < 0) return;
-  const int raster_tile = static_cast<int>(block - static_cast<int64_t>(active) * raster_tiles);
-  const int tile_x = raster_tile % raster_tiles_x;
-  const int tile_y = raster_tile / raster_tiles_x;
+  const int camera_bin = static_cast<int>(bin - static_cast<int64_t>(active) * bins);
+  const int bin_x = camera_bin % cam.tiles_x, bin_y = camera_bin / cam.tiles_x;
+  const int tile_x = bin_x * split + part % split;
+  const int tile_y = bin_y * split + part / split;
+  if (tile_x * kRaster >= cam.width || tile_y * kRaster >= cam.height) return;  // past a ragged edge
   const int pixel_x = tile_x * kRaster + block_x0 + (wave_lane & 7);
   const int pixel_y = tile_y * kRaster + block_y0 + (wave_lane >> 3);
   const bool valid_pixel = pixel_x < cam.width && pixel_y < cam.height;
-  const int bin_x = tile_x * kRaster / bin_size;
-  const int bin_y = tile_y * kRaster / bin_size;
   const uint32_t global_bin = cam.tile_base + static_cast<uint32_t>(bin_y * cam.tiles_x + bin_x);
   const float ray_x = ((static_cast<float>(pixel_x) + 0.5f) - cam.center_x) / cam.focal_x;
   const float ray_y = ((static_cast<float>(pixel_y) + 0.5f) - cam.center_y) / cam.focal_y;
@@ -762,23 +796,42 @@ __global__ __launch_bounds__(kRaster* kRaster) void composite_ray_kernel(Composi
   bool done = !valid_pixel;
   const int64_t range_start = args.tile_starts[global_bin];
   const int64_t range_end = args.tile_ends[global_bin];
+  const float support_limit = support_sigma * support_sigma * (1.0f + 0x1p-20f);
   if (range_start >= 0 && range_end > range_start) {
+    f32x4 next_a, next_b, next_c, next_colour;
+    float next_x = 0.0f, next_y = 0.0f, next_half_x = 0.0f, next_half_y = 0.0f;
+    bool next_valid = false;
+    const auto gather = [&](int64_t begin) {
+      next_valid = false;
+      if (begin + threadIdx.x >= range_end) return;
+      const int32_t record = args.sorted_values[begin + threadIdx.x];
+      if (record < 0 || record >= args.visible_capacity) return;  // a corrupted list: an entry that never blends
+      next_valid = true;
+      const f32x4* rec = reinterpret_cast<const f32x4*>(args.records + record);
+      const f32x4* ray = reinterpret_cast<const f32x4*>(ray_records + static_cast<int64_t>(record) * 12);
+      const f32x4 r0 = rec[0], r1 = rec[1], r2 = rec[2], q2 = ray[2];
+      next_a = ray[0];
+      next_b = ray[1];
+      next_c = f32x4{q2.x, q2.y, r1.y, r1.z};
+      next_colour = f32x4{r1.w, r2.x, r2.y, r2.z};
+      next_x = r0.x;
+      next_y = r0.y;
+      next_half_x = q2.z;
+      next_half_y = q2.w;
+    };
+    gather(range_start);
     for (int64_t batch_start = range_start; batch_start < range_end; batch_start += kThreads) {
       const int count = static_cast<int>(range_end - batch_start < kThreads ? range_end - batch_start : kThreads);
       __syncthreads();  // previous batch fully consumed
       uint32_t waves = 0u;
       if (static_cast<int>(threadIdx.x) < count) {
-        const int32_t record = args.sorted_values[batch_start + threadIdx.x];
-        if (record >= 0 && record < args.visible_capacity) {
-          const f32x4* rec = reinterpret_cast<const f32x4*>(args.records + record);
-          const f32x4* ray = reinterpret_cast<const f32x4*>(ray_records + static_cast<int64_t>(record) * 12);
-          const f32x4 r0 = rec[0], r1 = rec[1], r2 = rec[2], q2 = ray[2];
-          s_a[threadIdx.x] = ray[0];
-          s_b[threadIdx.x] = ray[1];
-          s_c[threadIdx.x] = f32x4{q2.x, q2.y, r1.y, r1.z};
-          s_colour[threadIdx.x] = f32x4{r1.w, r2.x, r2.y, r2.z};
+        if (next_valid) {
+          s_a[threadIdx.x] = f32x4{next_a.x, 2.0f * next_a.y, 2.0f * next_a.z, next_a.w};
+          s_b[threadIdx.x] = f32x4{2.0f * next_b.x, next_b.y, next_b.z, next_b.w};
+          s_c[threadIdx.x] = next_c;
+          s_colour[threadIdx.x] = next_colour;
           // Each wave's block of pixel centres against the entry's cull box (centre
-          // r0.xy, half extents q2.zw): a wave outside it has alpha 0 at every
+          // next_x, next_y, half extents next_half_*): a wave outside it has alpha 0 at every
           // pixel, so the entry is left out of its list.
           waves = kCull ? 0u : 1u;
           if constexpr (kCull) {
@@ -786,14 +839,13 @@ __global__ __launch_bounds__(kRaster* kRaster) void composite_ray_kernel(Composi
             for (int w = 0; w < kWaves; ++w) {
               const float x0 = static_cast<float>(tile_x * kRaster + (w % kBlocksX) * 8) + 0.5f;
               const float y0 = static_cast<float>(tile_y * kRaster + (w / kBlocksX) * 8) + 0.5f;
-              if (fabsf(r0.x - fminf(fmaxf(r0.x, x0), x0 + 7.0f)) <= q2.z &&
-                  fabsf(r0.y - fminf(fmaxf(r0.y, y0), y0 + 7.0f)) <= q2.w) {
+              if (fabsf(next_x - fminf(fmaxf(next_x, x0), x0 + 7.0f)) <= next_half_x &&
+                  fabsf(next_y - fminf(fmaxf(next_y, y0), y0 + 7.0f)) <= next_half_y) {
                 waves |= 1u << w;
               }
             }
           }
         } else {
-          // Only reachable with a corrupted list: an entry that never blends.
           s_a[threadIdx.x] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
           s_b[threadIdx.x] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
           s_c[threadIdx.x] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -825,27 +877,51 @@ __global__ __launch_bounds__(kRaster* kRaster) void composite_ray_kernel(Composi
 #pragma unroll
         for (int q = 0; q < kWaves; ++q) list_count += static_cast<int>(s_totals[q][wave]);
       }
+      if (batch_start + kThreads < range_end) gather(batch_start + kThreads);
       __syncthreads();
-      for (int i = 0; !done && i < list_count; ++i) {
-        const int item = kCull ? static_cast<int>(s_list[wave][i]) : i;
-        const f32x4 c = s_c[item];
-        const float alpha = ray_alpha(ray_x, ray_y, s_a[item], s_b[item], c, support_sigma);
-        if (!(alpha > 0.0f)) continue;
-        const float next_transmittance = transmittance * (1.0f - alpha);
-        const f32x4 col = s_colour[item];
-        const float weight = transmittance * alpha;
-        red = fmaf(weight, col.x, red);
-        green = fmaf(weight, col.y, green);
-        blue = fmaf(weight, col.z, blue);
-        if (kFull) {
-          depth_sum = fmaf(weight, c.w, depth_sum);
-          if (weight > best_weight) {
-            best_weight = weight;
-            best_gaussian = __float_as_int(col.w);
+      if (!done) {
+        constexpr int kUnroll = 4;
+        for (int i = 0; !done && i < list_count; i += kUnroll) {
+          int items[kUnroll];
+          RayApproach approach[kUnroll];
+          float mpm[kUnroll];
+          bool hits[kUnroll];
+#pragma unroll
+          for (int u = 0; u < kUnroll; ++u) {
+            // Past the end the last entry again, left out below.
+            const int at = i + u < list_count ? i + u : list_count - 1;
+            items[u] = kCull ? static_cast<int>(s_list[wave][at]) : at;
+          }
+#pragma unroll
+          for (int u = 0; u < kUnroll; ++u) {
+            const f32x4 c = s_c[items[u]];
+            approach[u] = ray_approach(ray_x, ray_y, s_a[items[u]], s_b[items[u]], c);
+            mpm[u] = c.y;
+            hits[u] = i + u < list_count && !ray_misses(approach[u], c.y, support_limit);
+          }
+#pragma unroll
+          for (int u = 0; u < kUnroll; ++u) {
+            if (!hits[u] || done) continue;
+            const f32x4 c = s_c[items[u]];
+            const float alpha = ray_alpha(approach[u], mpm[u], c.z, support_sigma);
+            if (!(alpha > 0.0f)) continue;
+            const float next_transmittance = transmittance * (1.0f - alpha);
+            const f32x4 col = s_colour[items[u]];
+            const float weight = transmittance * alpha;
+            red = fmaf(weight, col.x, red);
+            green = fmaf(weight, col.y, green);
+            blue = fmaf(weight, col.z, blue);
+            if (kFull) {
+              depth_sum = fmaf(weight, c.w, depth_sum);
+              if (weight > best_weight) {
+                best_weight = weight;
+                best_gaussian = __float_as_int(col.w);
+              }
+            }
+            transmittance = next_transmittance;
+            if (next_transmittance <= VGR_TRANSMITTANCE_THRESHOLD) done = true;
           }
         }
-        transmittance = next_transmittance;
-        if (next_transmittance <= VGR_TRANSMITTANCE_THRESHOLD) done = true;
       }
       if (!__syncthreads_or(done ? 0 : 1)) break;
     }
@@ -858,17 +934,18 @@ __global__ __launch_bounds__(kRaster* kRaster) void composite_ray_kernel(Composi
 template <int kRaster>
 void launch_ray(const CompositeArgs& args, const vgr_options& options, const float* ray_records, int active_count,
                 bool full, hipStream_t stream) {
-  const int raster_tiles_x = (options.width + kRaster - 1) / kRaster;
-  const int raster_tiles = raster_tiles_x * ((options.height + kRaster - 1) / kRaster);
-  const int64_t blocks = static_cast<int64_t>(active_count) * raster_tiles;
+  const int split = options.tile_size / kRaster;
+  const int bins = args.uniform_tiles;
+  constexpr int64_t kRound = kXcds * kXcdBins;
+  const int64_t blocks = (static_cast<int64_t>(active_count) * bins + kRound - 1) / kRound * kRound * split * split;
   if (blocks <= 0) return;
   const dim3 grid(static_cast<unsigned>(blocks)), block(kRaster * kRaster);
   if (full) {
     hipLaunchKernelGGL((composite_ray_kernel<kRaster, true>), grid, block, 0, stream, args, ray_records,
-                       options.gaussian_support_sigma, raster_tiles_x, raster_tiles, options.tile_size);
+                       options.gaussian_support_sigma, bins, options.tile_size);
   } else {
     hipLaunchKernelGGL((composite_ray_kernel<kRaster, false>), grid, block, 0, stream, args, ray_records,
-                       options.gaussian_support_sigma, raster_tiles_x, raster_tiles, options.tile_size);
+                       options.gaussian_support_sigma, bins, options.tile_size);
   }
 }
 
