@@ -191,8 +191,8 @@ typedef struct vgr_options {
                                        evaluations; [1] sort look-back give-ups (as counters[5]);
                                        [2] projection work items kept by chunk culling; [3] tiles the
                                        tile-front ordering had to sort in full */
-  int32_t persistent_composite;     /* 0: one workgroup per (camera, tile); N > 0: N workgroups pull
-                                       (camera, tile) items from a device queue */
+  int32_t persistent_composite;     /* >= 0, accepted for any value: the compositor launches one
+                                       workgroup per (camera, tile), which is the faster form */
   int32_t chunk_culling;            /* 1: cull (camera group x chunk) items against camera frusta using
                                        scene.chunk_bounds (scratch sized for it) */
   int32_t lookback_spin_limit;      /* radix-sort look-back polls of an unpublished predecessor before the

@@ -137,7 +137,7 @@ struct CompositeArgs {
   int64_t* statistics;   // optional: [0] += evaluated (pixel, Gaussian) pairs
   int64_t visible_capacity;
   int64_t gaussian_count;
-  uint32_t* work_counter;  // persistent queue counter (zeroed before the launch)
+  uint32_t* work_counter;  // queue of the tiles left open (zeroed before the launch)
   const int32_t* tile_order;  // launch order of the (camera, tile) items
   const uint32_t* long_tiles;  // how many of the first in that order are long
   int64_t total_items;     // (camera, tile) items in the launch
@@ -159,19 +159,11 @@ struct FrontCompositeArgs : CompositeArgs {
   const int32_t* front_lengths;  // null: no open-tile detection (the recomposite pass)
   int32_t* open_tiles;
   uint32_t* open_count;
-  const uint32_t* item_count;  // persistent launches: device item count (overrides total_items)
+  const uint32_t* item_count;  // the pass over the tiles left open: their count, on the device
 };
 
 template <int kDegree>
 using CompositeArgsFor = typename std::conditional<(kDegree < 0), CompositeArgs, FrontCompositeArgs>::type;
-
-template <typename Args>
-__device__ __forceinline__ int64_t item_total(const Args& args) {
-  if constexpr (std::is_same<Args, FrontCompositeArgs>::value) {
-    if (args.item_count != nullptr) return static_cast<int64_t>(*args.item_count);
-  }
-  return args.total_items;
-}
 
 // Writes a finished pixel (renderer_cuda.cu:2264-2304).
 template <bool kFull>
@@ -597,7 +589,7 @@ __global__ __launch_bounds__(kBlockBatch) void composite_block_persistent_kernel
   constexpr int kBlocks = kTileSize * kTileSize / 64;
   __shared__ BlockShared s;
   __shared__ int64_t s_item;
-  const int64_t total = item_total(args) * kBlocks;
+  const int64_t total = static_cast<int64_t>(*args.item_count) * kBlocks;
   for (;;) {
     if (threadIdx.x == 0) s_item = static_cast<int64_t>(atomicAdd(args.work_counter, 1u));
     __syncthreads();
@@ -951,32 +943,32 @@ void launch_ray(const CompositeArgs& args, const vgr_options& options, const flo
 
 // Minimum waves per SIMD for 16x16 tiles (launch-bounds occupancy target): eight
 // means at most 64 VGPRs.  The blend loop is latency-bound, so waves in flight
-// pay more than registers.  The evaluation-counting and persistent variants
-// need a few more registers and take seven and six (no spills).
-template <int kTileSize, int kBatch, bool kCount, bool kPersistent = false, int kDegree = -1>
+// pay more than registers.  The evaluation-counting variant needs a few more
+// registers and takes seven (no spills).
+template <int kTileSize, int kBatch, bool kCount, int kDegree = -1>
 constexpr int kCompositeWavesPerSimd =
     kTileSize != 16 ? 1
                     : (kDegree >= 2 ? 4  // recomputed records with SH2/3 coefficients in registers
                                     : (kDegree >= 0 ? 6
-                                                    : (kBatch >= 512 ? 4 : (kPersistent ? 6 : (kCount ? 7 : 8)))));
+                                                    : (kBatch >= 512 ? 4 : (kCount ? 7 : 8))));
 
 template <int kTileSize, int kBatch, bool kFull, bool kCount, bool kCheckpoint, int kDegree = -1>
-__global__ __launch_bounds__(kTileSize* kTileSize, (kCompositeWavesPerSimd<kTileSize, kBatch, kCount, false, kDegree>)) void
+__global__ __launch_bounds__(kTileSize* kTileSize, (kCompositeWavesPerSimd<kTileSize, kBatch, kCount, kDegree>)) void
 composite_kernel(CompositeArgsFor<kDegree> args) {
   const int64_t block = args.tile_order != nullptr ? args.tile_order[blockIdx.x] : blockIdx.x;
   __shared__ WaveLists<kTileSize, kBatch> s;
   composite_tile<kTileSize, kBatch, kFull, kCount, kCheckpoint, kDegree>(args, block, s);
 }
 
-// Persistent form: a fixed grid whose workgroups pull (camera, tile) items from
-// a device counter until the queue is empty; every workgroup exits once the
-// counter passes the item count.
+// The tiles left open, with evaluations counted: a fixed grid whose workgroups pull
+// items from a device counter until the queue is empty; every workgroup exits once
+// the counter passes the item count.
 template <int kTileSize, int kBatch, bool kFull, bool kCount, bool kCheckpoint, int kDegree = -1>
-__global__ __launch_bounds__(kTileSize* kTileSize, (kCompositeWavesPerSimd<kTileSize, kBatch, kCount, true, kDegree>)) void
+__global__ __launch_bounds__(kTileSize* kTileSize, (kCompositeWavesPerSimd<kTileSize, kBatch, kCount, kDegree>)) void
 composite_persistent_kernel(CompositeArgsFor<kDegree> args) {
   __shared__ WaveLists<kTileSize, kBatch> s;
   __shared__ int64_t s_item;
-  const int64_t total = item_total(args);
+  const int64_t total = static_cast<int64_t>(*args.item_count);
   for (;;) {
     if (threadIdx.x == 0) s_item = static_cast<int64_t>(atomicAdd(args.work_counter, 1u));
     __syncthreads();
@@ -1040,115 +1032,116 @@ constexpr int64_t kMixedCompositeTiles = 1280;
 // would go 182 -> 253.
 constexpr int64_t kBlockCompositeTiles = 5120;
 
+constexpr int kOpenWorkgroups = 256;  // of the pass over the tiles left open
+
 template <int kTileSize, int kBatch, bool kFull, bool kCount, bool kCheckpoint = false, int kDegree = -1>
-void launch_variant(const CompositeArgsFor<kDegree>& args, int64_t blocks, int persistent, hipStream_t stream) {
+void launch_variant(const CompositeArgsFor<kDegree>& args, int64_t blocks, hipStream_t stream) {
   const dim3 block(kTileSize * kTileSize);
-  if constexpr (!kCount) {
-    constexpr int kBlocks = kTileSize * kTileSize / 64;
-    if constexpr (kDegree >= 0) {
-      // The tiles left open: few, with the longest lists, so always by block.  1024 room
-      // cameras of 160x120 over 5M Gaussians (121 such tiles, lists up to 200k): 7.4 ->
-      // 4.4 ms, 256 of 2M with checkpoints (385 tiles) 0.97 -> 0.79.
-      if (args.item_count != nullptr) {
-        hipLaunchKernelGGL((composite_block_persistent_kernel<kTileSize, kFull, kCheckpoint, kDegree>),
-                           dim3(static_cast<unsigned>(persistent * 2)), dim3(kBlockBatch), 0, stream, args);
-        return;
-      }
-    } else if (persistent == 0) {
-      const dim3 grid(static_cast<unsigned>(blocks * kBlocks));
-      if constexpr (kTileSize == 16) {
-        if (blocks <= kMixedCompositeTiles) {
-          hipLaunchKernelGGL((composite_mixed_kernel<kBatch, kFull, kCheckpoint>), grid, dim3(kBlockBatch), 0, stream,
-                             args);
-          return;
-        }
-      } else if (blocks <= kBlockCompositeTiles) {
-        hipLaunchKernelGGL((composite_block_kernel<kTileSize, kFull, kCheckpoint>), grid, dim3(kBlockBatch), 0,
+  constexpr int kBlocks = kTileSize * kTileSize / 64;
+  if constexpr (kDegree >= 0) {
+    // The tiles left open: few, with the longest lists, so always by block.  1024 room
+    // cameras of 160x120 over 5M Gaussians (121 such tiles, lists up to 200k): 7.4 ->
+    // 4.4 ms, 256 of 2M with checkpoints (385 tiles) 0.97 -> 0.79.
+    if (args.item_count != nullptr) {
+      if constexpr (kCount) {
+        hipLaunchKernelGGL((composite_persistent_kernel<kTileSize, kBatch, kFull, kCount, kCheckpoint, kDegree>),
+                           dim3(static_cast<unsigned>(blocks < kOpenWorkgroups ? blocks : kOpenWorkgroups)), block, 0,
                            stream, args);
+      } else {
+        hipLaunchKernelGGL((composite_block_persistent_kernel<kTileSize, kFull, kCheckpoint, kDegree>),
+                           dim3(2 * kOpenWorkgroups), dim3(kBlockBatch), 0, stream, args);
+      }
+      return;
+    }
+  } else if constexpr (!kCount) {
+    const dim3 grid(static_cast<unsigned>(blocks * kBlocks));
+    if constexpr (kTileSize == 16) {
+      if (blocks <= kMixedCompositeTiles) {
+        hipLaunchKernelGGL((composite_mixed_kernel<kBatch, kFull, kCheckpoint>), grid, dim3(kBlockBatch), 0, stream,
+                           args);
         return;
       }
+    } else if (blocks <= kBlockCompositeTiles) {
+      hipLaunchKernelGGL((composite_block_kernel<kTileSize, kFull, kCheckpoint>), grid, dim3(kBlockBatch), 0,
+                         stream, args);
+      return;
     }
   }
-  if (persistent > 0) {
-    const int64_t grid = blocks < persistent ? blocks : persistent;
-    hipLaunchKernelGGL((composite_persistent_kernel<kTileSize, kBatch, kFull, kCount, kCheckpoint, kDegree>),
-                       dim3(static_cast<unsigned>(grid)), block, 0, stream, args);
-  } else {
-    hipLaunchKernelGGL((composite_kernel<kTileSize, kBatch, kFull, kCount, kCheckpoint, kDegree>),
-                       dim3(static_cast<unsigned>(blocks)), block, 0, stream, args);
-  }
+  // One workgroup a tile otherwise: the dispatcher hands tiles out in order as well as
+  // a queue does, at eight waves a SIMD instead of six and without the queue's barriers
+  // (256 cameras of four resolutions, 170k tiles: 21.1 -> 17.0 ms; tile-front lists of
+  // 1024 room cameras 6.49 -> 5.87, of 256 with checkpoints 2.66 -> 2.39).
+  hipLaunchKernelGGL((composite_kernel<kTileSize, kBatch, kFull, kCount, kCheckpoint, kDegree>),
+                     dim3(static_cast<unsigned>(blocks)), block, 0, stream, args);
 }
 
 // Tile-front lists (16x16 tiles, 256-entry batches): records recomputed per SH degree.
 template <int kDegree>
-void launch_projected_degree(bool full, const FrontCompositeArgs& args, int64_t blocks, int persistent,
-                             hipStream_t stream) {
+void launch_projected_degree(bool full, const FrontCompositeArgs& args, int64_t blocks, hipStream_t stream) {
   if (args.final_transmittance != nullptr) {
     // Checkpointed (pose-training) forward: final transmittance and last blended position.
-    launch_variant<16, 256, true, false, true, kDegree>(args, blocks, persistent, stream);
+    launch_variant<16, 256, true, false, true, kDegree>(args, blocks, stream);
   } else if (args.statistics != nullptr) {
     if (full) {
-      launch_variant<16, 256, true, true, false, kDegree>(args, blocks, persistent, stream);
+      launch_variant<16, 256, true, true, false, kDegree>(args, blocks, stream);
     } else {
-      launch_variant<16, 256, false, true, false, kDegree>(args, blocks, persistent, stream);
+      launch_variant<16, 256, false, true, false, kDegree>(args, blocks, stream);
     }
   } else if (full) {
-    launch_variant<16, 256, true, false, false, kDegree>(args, blocks, persistent, stream);
+    launch_variant<16, 256, true, false, false, kDegree>(args, blocks, stream);
   } else {
-    launch_variant<16, 256, false, false, false, kDegree>(args, blocks, persistent, stream);
+    launch_variant<16, 256, false, false, false, kDegree>(args, blocks, stream);
   }
 }
 
-void launch_projected(int degree, bool full, const FrontCompositeArgs& args, int64_t blocks, int persistent,
-                      hipStream_t stream) {
+void launch_projected(int degree, bool full, const FrontCompositeArgs& args, int64_t blocks, hipStream_t stream) {
   switch (degree) {
     case 1:
-      launch_projected_degree<1>(full, args, blocks, persistent, stream);
+      launch_projected_degree<1>(full, args, blocks, stream);
       break;
     case 2:
-      launch_projected_degree<2>(full, args, blocks, persistent, stream);
+      launch_projected_degree<2>(full, args, blocks, stream);
       break;
     case 3:
-      launch_projected_degree<3>(full, args, blocks, persistent, stream);
+      launch_projected_degree<3>(full, args, blocks, stream);
       break;
     default:
-      launch_projected_degree<0>(full, args, blocks, persistent, stream);
+      launch_projected_degree<0>(full, args, blocks, stream);
       break;
   }
 }
 
 template <int kTileSize, int kBatch>
-void launch_full_or_rgb(bool full, const CompositeArgs& args, int64_t blocks, int persistent, hipStream_t stream) {
+void launch_full_or_rgb(bool full, const CompositeArgs& args, int64_t blocks, hipStream_t stream) {
   if (args.final_transmittance != nullptr) {
-    launch_variant<kTileSize, kBatch, true, false, true>(args, blocks, persistent, stream);
+    launch_variant<kTileSize, kBatch, true, false, true>(args, blocks, stream);
   } else if (args.statistics != nullptr) {
     if (full) {
-      launch_variant<kTileSize, kBatch, true, true>(args, blocks, persistent, stream);
+      launch_variant<kTileSize, kBatch, true, true>(args, blocks, stream);
     } else {
-      launch_variant<kTileSize, kBatch, false, true>(args, blocks, persistent, stream);
+      launch_variant<kTileSize, kBatch, false, true>(args, blocks, stream);
     }
   } else if (full) {
-    launch_variant<kTileSize, kBatch, true, false>(args, blocks, persistent, stream);
+    launch_variant<kTileSize, kBatch, true, false>(args, blocks, stream);
   } else {
-    launch_variant<kTileSize, kBatch, false, false>(args, blocks, persistent, stream);
+    launch_variant<kTileSize, kBatch, false, false>(args, blocks, stream);
   }
 }
 
 template <int kTileSize>
-void launch_batch(int batch, bool full, const CompositeArgs& args, int64_t blocks, int persistent,
-                  hipStream_t stream) {
+void launch_batch(int batch, bool full, const CompositeArgs& args, int64_t blocks, hipStream_t stream) {
   switch (batch) {
     case 64:
-      launch_full_or_rgb<kTileSize, 64>(full, args, blocks, persistent, stream);
+      launch_full_or_rgb<kTileSize, 64>(full, args, blocks, stream);
       break;
     case 128:
-      launch_full_or_rgb<kTileSize, 128>(full, args, blocks, persistent, stream);
+      launch_full_or_rgb<kTileSize, 128>(full, args, blocks, stream);
       break;
     case 512:
-      launch_full_or_rgb<kTileSize, 512>(full, args, blocks, persistent, stream);
+      launch_full_or_rgb<kTileSize, 512>(full, args, blocks, stream);
       break;
     default:
-      launch_full_or_rgb<kTileSize, 256>(full, args, blocks, persistent, stream);
+      launch_full_or_rgb<kTileSize, 256>(full, args, blocks, stream);
       break;
   }
 }
@@ -1273,8 +1266,6 @@ int launch_composite(const vgr_scene& scene, const vgr_cameras& cameras, const v
     args.tile_order = order;
     args.long_tiles = args.work_counter + 1;
   }
-  const int persistent = options.persistent_composite;
-  if (persistent > 0) launch_fill_u32(args.work_counter, 1, 0u, stream);
   if (front) {
     FrontCompositeArgs front_args;
     static_cast<CompositeArgs&>(front_args) = args;
@@ -1286,12 +1277,11 @@ int launch_composite(const vgr_scene& scene, const vgr_cameras& cameras, const v
     front_args.open_count = open_state + 0;
     front_args.item_count = nullptr;
     launch_fill_u32(open_state, 4, 0u, stream);
-    launch_projected(scene.sh_degree, full, front_args, blocks, persistent, stream);
+    launch_projected(scene.sh_degree, full, front_args, blocks, stream);
     // Tiles left open at the end of a truncated list: full sort, then composite
     // them again from their complete lists (fixed grids that exit at once when
     // no tile is open).
-    constexpr int kFallbackWorkgroups = 256;
-    const int status = launch_front_fallback_sort(scene, ws, layout, const_cast<char*>(scratch), kFallbackWorkgroups,
+    const int status = launch_front_fallback_sort(scene, ws, layout, const_cast<char*>(scratch), kOpenWorkgroups,
                                                   stream);
     if (status != 0) return status;
     FrontCompositeArgs again = front_args;
@@ -1300,12 +1290,12 @@ int launch_composite(const vgr_scene& scene, const vgr_cameras& cameras, const v
     again.tile_order = open_tiles;
     again.item_count = open_state + 0;
     again.work_counter = open_state + 2;
-    launch_projected(scene.sh_degree, full, again, blocks, kFallbackWorkgroups, stream);
+    launch_projected(scene.sh_degree, full, again, blocks, stream);
     if (options.statistics != nullptr) launch_copy_u32_to_i64(open_state + 0, options.statistics + 3, stream);
   } else if (options.tile_size == 8) {
-    launch_batch<8>(options.raster_batch, full, args, blocks, persistent, stream);
+    launch_batch<8>(options.raster_batch, full, args, blocks, stream);
   } else {
-    launch_batch<16>(options.raster_batch, full, args, blocks, persistent, stream);
+    launch_batch<16>(options.raster_batch, full, args, blocks, stream);
   }
   const hipError_t error = hipGetLastError();
   if (error != hipSuccess) {

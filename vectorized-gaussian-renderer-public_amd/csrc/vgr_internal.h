@@ -63,7 +63,7 @@ struct ScratchLayout {
   size_t item_blocks;      // int32[projection_blocks]: kept block ids in order
   size_t item_masks;       // uint64[projection_blocks]
   size_t item_totals;      // int64[2]: kept item count
-  size_t work_counter;     // uint32[8]: [0] persistent compositor queue, [1] long tiles, [4..7] queues of the tile sort
+  size_t work_counter;     // uint32[8]: [1] long tiles, [4..7] queues of the tile sort
   size_t tile_order;       // int32[global_tiles]: long-list queue of the tile sort, then the compositing order
                            // (longest lists first), which the backward reuses
   // Tile-front ordering only (zero-sized otherwise).

@@ -8,8 +8,8 @@ and output offset on the device, and one submission runs:
 
   camera table -> frustum cull of (camera group x 256-Gaussian chunk) items
   against conservative per-chunk bounds -> projection + emission over the kept
-  items -> onesweep radix ordering -> tile-ID tie order -> tile ranges ->
-  persistent compositing over a (camera, tile) work queue.
+  items -> radix partition by tile -> tile ranges -> depth order inside each
+  tile -> compositing, one workgroup per (camera, tile).
 
 Nothing in the submission reads a count on the host, so after one eager
 calibration render (which sizes the capacities) the whole submission is
