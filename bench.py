@@ -193,7 +193,8 @@ def main() -> int:
         "projection+emission": args.gaussians * (16 + 24 + 12 * bands) + visible * RECORD_BYTES
         + intersections * 12,
         "sort": intersections * (8 + 24 * passes),
-        "tile_ranges": intersections * 8 + global_tiles * 8,
+        # The ranges, then the depth order inside each tile (keys and values read and written).
+        "tile_ranges": intersections * (8 + 24) + global_tiles * 8,
     }
     composite_flops = COMPOSITE_FLOPS_PER_EVALUATION * evaluations
     dominant = max(stage_ms, key=stage_ms.get)

@@ -176,7 +176,7 @@ typedef struct vgr_options {
   int32_t deterministic;            /* accepted; ordering is always deterministic */
   int32_t full_sensor_output;       /* 1: rgb+depth+alpha+semantic, 0: rgb only */
   int32_t fixed_capacity_sort;      /* accepted; the sort never reads the count on the host */
-  int32_t sort_digit_bits;          /* 0 = default (8, or 9 where that saves a pass); 4..9 */
+  int32_t sort_digit_bits;          /* 0 = default (9, or what one pass over the partition needs); 4..9 */
   int32_t raster_batch;             /* Gaussians staged per LDS batch: 0 = default (256); 64..512 */
   int32_t cameras_per_block;        /* projection camera group: 0 = default (32); 1..64 */
   int32_t reuse_projection;         /* 1: composite only, reusing the sorted intersections and
