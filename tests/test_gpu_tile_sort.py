@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 import torch
 
-from vgr_amd import CustomHipBackend, RendererService, synthetic
+from vgr_amd import CustomHipBackend, RendererService, native, synthetic
 from vgr_amd.batched import BatchedRenderer, CameraSpec
 
 pytestmark = pytest.mark.gpu
@@ -114,3 +114,63 @@ def test_ties_of_a_spatially_ordered_scene(count, depths):
     torch.cuda.synchronize()
     for name, tensor in out.items():
         assert torch.equal(tensor.view(plain[name].shape), plain[name]), name
+
+
+def sorted_list(scene, size: int, gaussian_ids):
+    """One identity camera through the native entry point; (keys, values, records) of its lists."""
+    dev = torch.device("cuda", 0)
+    module = native.load_native_module()
+    scene = scene.to(dev)
+    count = scene.count
+    covariances = torch.empty((count, 6), device=dev)
+    module.precompute_covariances(scene.scales, scene.rotations, covariances)
+    viewmats, intrinsics = identity_rig(size)
+    tiles = ((size + 15) // 16) ** 2
+    capacity = count * tiles
+    outputs = [torch.empty((1, size, size, 3), device=dev), torch.empty((1, size, size, 1), device=dev),
+               torch.empty((1, size, size, 1), device=dev), torch.empty((1, size, size, 1), dtype=torch.int64, device=dev)]
+    scratch = module.scratch_bytes(max_views=1, height=size, width=size, gaussians=count,
+                                   intersection_capacity=capacity, tile_size=16, near_plane=0.01, far_plane=100.0)
+    keys = [torch.zeros(capacity, dtype=torch.uint64, device=dev) for _ in range(2)]
+    values = [torch.full((capacity,), -1, dtype=torch.int32, device=dev) for _ in range(2)]
+    records = torch.empty((count, native.RECORD_FLOATS), device=dev)
+    counters = torch.zeros(native.COUNTER_SLOTS, dtype=torch.int64, device=dev)
+    workspace = [records, *keys, *values, torch.empty(tiles, dtype=torch.int32, device=dev),
+                 torch.empty(tiles, dtype=torch.int32, device=dev), counters,
+                 torch.empty(scratch, dtype=torch.uint8, device=dev)]
+    selector = module.render(
+        [scene.means, covariances, scene.opacities, scene.features, scene.semantic_ids,
+         torch.zeros(1, dtype=torch.int64, device=dev), torch.tensor([0, count], dtype=torch.int64, device=dev)],
+        [viewmats.to(dev), intrinsics.to(dev), torch.eye(4, device=dev).unsqueeze(0).contiguous(),
+         torch.zeros(1, dtype=torch.int64, device=dev), torch.empty(0, dtype=torch.int64, device=dev)],
+        outputs, workspace, size, size, count, 0.01, 100.0, 3.33, 0.3, False, 0.01, False, 16, 4096, 64, False, False,
+        False, False, True, True, False, gaussian_ids=gaussian_ids.to(dev))
+    torch.cuda.synchronize()
+    total = int(counters[1])
+    assert int(counters[5]) == 0
+    return keys[selector][:total].cpu().numpy(), values[selector][:total].cpu().numpy(), records.cpu().numpy()
+
+
+@pytest.mark.parametrize("distinct_ids", [1, 3])
+@pytest.mark.parametrize("around", [0, 2000])
+def test_more_equal_depths_and_ids_than_the_lds_holds(around, distinct_ids):
+    """Nothing tells these entries apart but the record: 10,000 at each of two neighbouring depths, alone
+    (crowded in the first spread's result) or with others around (crowded in the second's)."""
+    crowd = 10_000
+    scene = column_scene(2 * crowd + around, "spread")
+    rng = np.random.default_rng(9)
+    z = rng.uniform(2.0, 2.1, 2 * crowd + around).astype(np.float32)
+    z[:crowd] = np.float32(2.0)
+    z[crowd:2 * crowd] = np.nextafter(np.float32(2.0), np.float32(3.0))
+    order = rng.permutation(z.size)
+    scene.means = torch.tensor(np.stack([0.01 * rng.uniform(-1, 1, z.size), 0.01 * rng.uniform(-1, 1, z.size),
+                                         z[order]], axis=1), dtype=torch.float32)
+    ids = torch.arange(z.size, dtype=torch.int32) % distinct_ids
+    keys, values, records = sorted_list(scene, 16, ids)
+    assert keys.size == z.size and np.unique(values).size == z.size
+    listed = records[values]
+    np.testing.assert_array_equal(keys.astype(np.uint32), listed[:, 6].view(np.uint32))  # depth bits
+    record_ids = listed[:, 10].view(np.int32).astype(np.int64)
+    tie = record_ids * (1 << 32) + values
+    step = np.diff(keys.astype(np.int64))
+    assert np.all((step > 0) | ((step == 0) & (np.diff(tie) > 0)))

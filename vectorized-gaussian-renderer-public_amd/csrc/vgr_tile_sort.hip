@@ -15,7 +15,8 @@
 //                       spread over 4096 depth bins in global memory and queued as
 //                       runs of whole bins that do; a bin that does not fit is spread
 //                       again over its own range (over the tie order when all its
-//                       depths are equal);
+//                       depths are equal), or sorted in place when its tie words are
+//                       equal too (a scene whose Gaussian IDs repeat);
 //   run_sort_kernel   : a persistent grid over the queue (runs of up to 8192 entries).
 // The split follows the LDS: 2048 entries leave six workgroups on a CU to hide
 // each other's barriers, and two of 8192 entries fit.  Bound by those barriers and
@@ -218,7 +219,8 @@ struct SpreadShared {
 };
 
 // Entries of one crowded bin sorted where they end up, with a bitonic network in
-// global memory: only when more than kSpreadStack bins of one list are crowded.
+// global memory: when more than kSpreadStack bins of one list are crowded, and when
+// nothing but the value itself tells the entries apart.
 __device__ __forceinline__ void sort_in_place(const TileSortArgs& args, const TieOrder& tie, int64_t at,
                                               uint32_t length, const uint64_t* source_keys,
                                               const int32_t* source_values) {
@@ -314,6 +316,12 @@ __global__ __launch_bounds__(kSpreadThreads, 8) void spread_long_kernel(TileSort
           hi = word > hi ? word : hi;
         }
         block_min_max(s, lo, hi);
+        if (lo == hi) {  // uniform
+          // No bin splits entries of one depth and one tie word.  Every other segment comes
+          // out smaller: over an exact range, lo and hi fall into different bins.
+          sort_in_place(args, tie, base, count, source_keys, source_values);
+          continue;
+        }
       }
       const BinMap bin_of(lo, hi, kSpreadBins);
       for (int b = t; b < kSpreadBins; b += kSpreadThreads) s.cursor[b] = 0u;
