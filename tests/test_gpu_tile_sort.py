@@ -116,7 +116,8 @@ def test_ties_of_a_spatially_ordered_scene(count, depths):
         assert torch.equal(tensor.view(plain[name].shape), plain[name]), name
 
 
-def sorted_list(scene, size: int, gaussian_ids):
+def sorted_list(scene, size: int, *, capacity: int, gaussian_ids=None, near: float = 0.01, far: float = 100.0,
+                sort_digit_bits: int = 0):
     """One identity camera through the native entry point; (keys, values, records) of its lists."""
     dev = torch.device("cuda", 0)
     module = native.load_native_module()
@@ -126,11 +127,11 @@ def sorted_list(scene, size: int, gaussian_ids):
     module.precompute_covariances(scene.scales, scene.rotations, covariances)
     viewmats, intrinsics = identity_rig(size)
     tiles = ((size + 15) // 16) ** 2
-    capacity = count * tiles
     outputs = [torch.empty((1, size, size, 3), device=dev), torch.empty((1, size, size, 1), device=dev),
                torch.empty((1, size, size, 1), device=dev), torch.empty((1, size, size, 1), dtype=torch.int64, device=dev)]
     scratch = module.scratch_bytes(max_views=1, height=size, width=size, gaussians=count,
-                                   intersection_capacity=capacity, tile_size=16, near_plane=0.01, far_plane=100.0)
+                                   intersection_capacity=capacity, tile_size=16, near_plane=near, far_plane=far,
+                                   sort_digit_bits=sort_digit_bits)
     keys = [torch.zeros(capacity, dtype=torch.uint64, device=dev) for _ in range(2)]
     values = [torch.full((capacity,), -1, dtype=torch.int32, device=dev) for _ in range(2)]
     records = torch.empty((count, native.RECORD_FLOATS), device=dev)
@@ -143,11 +144,12 @@ def sorted_list(scene, size: int, gaussian_ids):
          torch.zeros(1, dtype=torch.int64, device=dev), torch.tensor([0, count], dtype=torch.int64, device=dev)],
         [viewmats.to(dev), intrinsics.to(dev), torch.eye(4, device=dev).unsqueeze(0).contiguous(),
          torch.zeros(1, dtype=torch.int64, device=dev), torch.empty(0, dtype=torch.int64, device=dev)],
-        outputs, workspace, size, size, count, 0.01, 100.0, 3.33, 0.3, False, 0.01, False, 16, 4096, 64, False, False,
-        False, False, True, True, False, gaussian_ids=gaussian_ids.to(dev))
+        outputs, workspace, size, size, count, near, far, 3.33, 0.3, False, 0.01, False, 16, 4096, 64, False, False, False,
+        False, True, True, False, gaussian_ids=None if gaussian_ids is None else gaussian_ids.to(dev),
+        sort_digit_bits=sort_digit_bits)
     torch.cuda.synchronize()
     total = int(counters[1])
-    assert int(counters[5]) == 0
+    assert int(counters[3]) == 0 and int(counters[5]) == 0
     return keys[selector][:total].cpu().numpy(), values[selector][:total].cpu().numpy(), records.cpu().numpy()
 
 
@@ -166,7 +168,7 @@ def test_more_equal_depths_and_ids_than_the_lds_holds(around, distinct_ids):
     scene.means = torch.tensor(np.stack([0.01 * rng.uniform(-1, 1, z.size), 0.01 * rng.uniform(-1, 1, z.size),
                                          z[order]], axis=1), dtype=torch.float32)
     ids = torch.arange(z.size, dtype=torch.int32) % distinct_ids
-    keys, values, records = sorted_list(scene, 16, ids)
+    keys, values, records = sorted_list(scene, 16, capacity=z.size, gaussian_ids=ids)
     assert keys.size == z.size and np.unique(values).size == z.size
     listed = records[values]
     np.testing.assert_array_equal(keys.astype(np.uint32), listed[:, 6].view(np.uint32))  # depth bits
@@ -174,3 +176,32 @@ def test_more_equal_depths_and_ids_than_the_lds_holds(around, distinct_ids):
     tie = record_ids * (1 << 32) + values
     step = np.diff(keys.astype(np.int64))
     assert np.all((step > 0) | ((step == 0) & (np.diff(tie) > 0)))
+
+
+@pytest.mark.parametrize("depths", ["equal", "mixed"])
+def test_more_crowded_lists_than_queue_places(depths):
+    """Four-bit digits over a 20-bit key leave 19 places per sort tile of 8192 entries; 256 tiles with 300
+    entries at one or two depths each, and one with 20,000 over the whole depth range, want more."""
+    size, per_tile, extra = 256, 300, 20_000
+    rng = np.random.default_rng(3)
+    near, far = np.float32(4.0), np.float32(4.001)
+    tile = np.concatenate([np.repeat(np.arange(256), per_tile), np.full(extra, 77)])
+    z = np.full(tile.size, np.float32(4.0005), dtype=np.float32)
+    if depths == "mixed":
+        z[rng.permutation(256 * per_tile)[:5000]] = np.float32(4.0002)
+    z[256 * per_tile:] = rng.uniform(4.0001, 4.0009, extra).astype(np.float32)
+    order = rng.permutation(tile.size)
+    tile, z = tile[order], z[order]
+    centre = np.stack([tile % 16, tile // 16], axis=1) * 16.0 + 8.0
+    xy = (centre - size / 2) * z[:, None].astype(np.float64) / size
+    scene = column_scene(tile.size, "spread")
+    scene.means = torch.tensor(np.concatenate([xy, z[:, None]], axis=1), dtype=torch.float32)
+    scene.scales = torch.full_like(scene.scales, 0.001)
+    keys, values, records = sorted_list(scene, size, capacity=tile.size, near=float(near), far=float(far),
+                                        sort_digit_bits=4)
+    assert keys.size == tile.size and np.unique(values).size == tile.size
+    listed = records[values]
+    np.testing.assert_array_equal((keys >> np.uint64(32)).astype(np.int64), tile[listed[:, 10].view(np.int32)])
+    np.testing.assert_array_equal(keys.astype(np.uint32), listed[:, 6].view(np.uint32))  # depth bits
+    step = np.diff(keys.astype(np.int64))
+    assert np.all((step > 0) | ((step == 0) & (np.diff(values) > 0)))

@@ -61,6 +61,19 @@ def test_scratch_query_is_monotonic_in_tile_count_with_default_digits():
     assert all(a <= b for a, b in zip(sizes, sizes[1:])), sizes
 
 
+@pytest.mark.parametrize("digit_bits", [4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize(("near", "far", "depth_bits"), [(0.01, 100.0, 27), (4.0, 4.001, 12)])
+def test_scratch_per_sort_tile_is_the_look_back_flags(digit_bits, near, far, depth_bits):
+    """With explicit digits a sort tile of 8192 keys takes one 4-byte flag per digit value and pass over
+    the whole (tile, depth) key, whatever else uses that space later."""
+    module = native.NativeRenderer()
+    sizes = [module.scratch_bytes(max_views=1, height=480, width=640, gaussians=1000,
+                                  intersection_capacity=8192 * sort_tiles, tile_size=16, near_plane=near,
+                                  far_plane=far, sort_digit_bits=digit_bits) for sort_tiles in (64, 128)]
+    key_bits = 11 + depth_bits  # 1,200 tiles
+    assert sizes[1] - sizes[0] == 64 * 4 * (-(-key_bits // digit_bits) << digit_bits)
+
+
 def test_invalid_options_are_reported_with_a_message():
     module = native.NativeRenderer()
     with pytest.raises(RuntimeError, match="tile_size"):

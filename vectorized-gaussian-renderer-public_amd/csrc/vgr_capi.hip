@@ -124,11 +124,8 @@ ScratchLayout compute_layout(int32_t active_count, int64_t gaussian_count, const
   const int64_t fixed_digit = options.sort_digit_bits;
   const int64_t passes8 = (key_bits + 7) / 8, passes9 = (key_bits + 8) / 9;
   const int64_t pass_count = fixed_digit != 0 ? (key_bits + fixed_digit - 1) / fixed_digit : passes8;
-  int64_t pass_slots = fixed_digit != 0 ? pass_count << fixed_digit
-                                        : (passes8 * 256 > passes9 * 512 ? passes8 * 256 : passes9 * 512);
-  // The flags' space later holds the tile sort's runs.
-  constexpr int64_t kRunSlots = kRunsPerSortTile * 4;
-  if (pass_slots < kRunSlots) pass_slots = kRunSlots;
+  const int64_t pass_slots = fixed_digit != 0 ? pass_count << fixed_digit
+                                              : (passes8 * 256 > passes9 * 512 ? passes8 * 256 : passes9 * 512);
   size_t offset = 0;
   layout.camera_table = offset;
   offset = align_up(offset + sizeof(CameraParams) * static_cast<size_t>(active_count > 0 ? active_count : 1));
@@ -145,8 +142,8 @@ ScratchLayout compute_layout(int32_t active_count, int64_t gaussian_count, const
   layout.sort_tickets = offset;
   offset = align_up(offset + sizeof(uint32_t) * static_cast<size_t>(pass_count));
   layout.sort_flags = offset;
-  const size_t flag_tiles = layout.front ? 0u : static_cast<size_t>(layout.sort_tiles);  // no radix pass
-  offset = align_up(offset + sizeof(uint32_t) * static_cast<size_t>(pass_slots) * flag_tiles);
+  layout.sort_flag_words = layout.front ? 0 : pass_slots * layout.sort_tiles;  // tile front: no radix pass
+  offset = align_up(offset + sizeof(uint32_t) * static_cast<size_t>(layout.sort_flag_words));
   layout.work_counter = offset;
   offset = align_up(offset + sizeof(uint32_t) * 8);
   layout.tile_order = offset;

@@ -56,7 +56,8 @@ struct ScratchLayout {
   size_t sort_histogram;   // uint32[passes * 256]
   size_t sort_digit_base;  // uint32[passes * 256]
   size_t sort_tickets;     // uint32[passes]
-  size_t sort_flags;       // uint32[passes * sort_tiles * radix]: look-back flags, then the tile sort's runs
+  size_t sort_flags;       // uint32[sort_flag_words]: look-back flags, then the tile sort's queues
+  int64_t sort_flag_words; // at least passes * sort_tiles * radix, of a radix of at least 16
   size_t cull_counts;      // int64[2 * (projection_blocks + 1)]   (chunk culling only)
   size_t cull_bases;       // int64[2 * (projection_blocks + scan_blocks + 1)]
   size_t cull_masks;       // uint64[projection_blocks]: camera mask per candidate block
@@ -114,7 +115,6 @@ constexpr int kProjectionWaves = kBlockThreads / kWave;  // waves of a projectio
 constexpr int64_t kOrderedCompositeBlocks = 32768;
 constexpr int kSortThreads = 512;      // threads per onesweep workgroup (8 waves)
 constexpr int kDefaultSortItems = 16;  // keys per thread per sort tile (tile = kSortThreads * items keys)
-constexpr int kRunsPerSortTile = 96;   // queued runs of 16 bytes per sort tile (at most 8192 keys)
 
 // Host helpers implemented in vgr_capi.hip.
 void set_error(const char* fmt, ...);

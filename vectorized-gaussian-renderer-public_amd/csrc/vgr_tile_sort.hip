@@ -54,10 +54,10 @@ struct TileSortArgs {
   const int64_t* failures;    // look-back waits the partition gave up: its order is wrong
   const vgr_record* records;  // spatially ordered scenes: ties by the record's Gaussian ID; else null
   int64_t visible_capacity;
-  // Queue of the parts for run_sort_kernel from the front, of those for spread_long_kernel
-  // from the back.
-  Run* runs;
+  Run* runs;                  // queue of the parts for run_sort_kernel
   uint32_t run_capacity;
+  Run* long_runs;             // queue of the parts for spread_long_kernel
+  uint32_t long_capacity;
   uint32_t* state;            // [0] queued runs, [1] taken runs, [2] queued long parts, [3] taken ones
 };
 
@@ -81,11 +81,53 @@ __device__ __forceinline__ uint32_t depth_word(const uint64_t* keys, int64_t i) 
   return reinterpret_cast<const uint32_t*>(keys)[2 * i];  // low half: depth bits
 }
 
-// The queue holds every part that can come up (launch_tile_sort says why).
-__device__ __forceinline__ void push_run(const TileSortArgs& args, const Run& run) {
+// Queues a part; false if the queue is full.  Called by one thread.
+__device__ __forceinline__ bool push_run(const TileSortArgs& args, const Run& run) {
   const bool fits = run.count <= static_cast<uint32_t>(kRunCapacity);
   const uint32_t slot = atomicAdd(&args.state[fits ? 0 : 2], 1u);
-  if (slot < args.run_capacity) args.runs[fits ? slot : args.run_capacity - 1u - slot] = run;
+  if (slot >= (fits ? args.run_capacity : args.long_capacity)) return false;
+  (fits ? args.runs : args.long_runs)[slot] = run;
+  return true;
+}
+
+// Sorts entries [at, at + length) of a buffer pair into the result's buffers with a
+// bitonic network in global memory, by the whole workgroup: for parts that the queue
+// has no room for, crowded bins beyond kSpreadStack in one list, and entries that
+// nothing but the value itself tells apart.  Barriers inside and at the end.
+template <int kThreads>
+__device__ __forceinline__ void sort_in_place(const TileSortArgs& args, int64_t at, uint32_t length,
+                                              const uint64_t* source_keys, const int32_t* source_values) {
+  const TieOrder tie{args.records, args.visible_capacity};
+  if (source_keys != args.keys_out) {
+    for (uint32_t i = threadIdx.x; i < length; i += kThreads) {
+      args.keys_out[at + i] = source_keys[at + i];
+      args.values_out[at + i] = source_values[at + i];
+    }
+  }
+  uint32_t padded = 2u;
+  while (padded < length) padded <<= 1;
+  for (uint32_t size = 2u; size != 0u && size <= padded; size <<= 1) {
+    for (uint32_t stride = size >> 1; stride > 0u; stride >>= 1) {
+      __threadfence_block();
+      __syncthreads();
+      for (uint32_t i = threadIdx.x; i < padded / 2u; i += kThreads) {
+        const uint32_t low_bits = i & (stride - 1u);
+        const uint32_t a = ((i - low_bits) << 1) + low_bits;
+        const uint32_t b = stride == (size >> 1) ? ((i - low_bits) << 1) + size - 1u - low_bits : a + stride;
+        if (b >= length) continue;
+        const uint64_t ka = args.keys_out[at + a], kb = args.keys_out[at + b];
+        const int32_t va = args.values_out[at + a], vb = args.values_out[at + b];
+        if (kb < ka || (kb == ka && tie(vb) < tie(va))) {
+          args.keys_out[at + a] = kb;
+          args.keys_out[at + b] = ka;
+          args.values_out[at + a] = vb;
+          args.values_out[at + b] = va;
+        }
+      }
+    }
+  }
+  __threadfence_block();
+  __syncthreads();
 }
 
 // Entries of the sorted-by-lead list [begin, count) that are counted by `below`, which
@@ -117,6 +159,7 @@ __device__ __forceinline__ uint32_t prefix_length(S& s, uint32_t begin, uint32_t
 template <int kThreads, int kCapacity, int kBins>
 __global__ __launch_bounds__(kThreads, 6) void tile_sort_kernel(TileSortArgs args) {
   __shared__ TileSort<kThreads, kCapacity, kBins> s;
+  __shared__ bool s_queued;
   // A failed partition leaves lists that overlap and slots nobody wrote: the render is
   // invalid and reported as such, and its lists are emptied rather than sorted.
   const bool failed = *args.failures != 0;
@@ -161,8 +204,12 @@ __global__ __launch_bounds__(kThreads, 6) void tile_sort_kernel(TileSortArgs arg
               values_out[rank] = value;
             });
       }
-      if (!sorted && threadIdx.x == 0) {
-        push_run(args, Run{static_cast<uint32_t>(start) + begin, n, static_cast<uint32_t>(tile), 0u});
+      if (!sorted) {  // uniform
+        if (threadIdx.x == 0) {
+          s_queued = push_run(args, Run{static_cast<uint32_t>(start) + begin, n, static_cast<uint32_t>(tile), 0u});
+        }
+        __syncthreads();
+        if (!s_queued) sort_in_place<kThreads>(args, start + begin, n, args.keys_in, args.values_in);
       }
       begin += n;
       __syncthreads();  // LDS free for the next part
@@ -216,45 +263,8 @@ struct SpreadShared {
   uint32_t stack_pair[kSpreadStack];
   uint32_t depth;
   uint32_t item;
+  bool queued;
 };
-
-// Entries of one crowded bin sorted where they end up, with a bitonic network in
-// global memory: when more than kSpreadStack bins of one list are crowded, and when
-// nothing but the value itself tells the entries apart.
-__device__ __forceinline__ void sort_in_place(const TileSortArgs& args, const TieOrder& tie, int64_t at,
-                                              uint32_t length, const uint64_t* source_keys,
-                                              const int32_t* source_values) {
-  if (source_keys != args.keys_out) {
-    for (uint32_t i = threadIdx.x; i < length; i += kSpreadThreads) {
-      args.keys_out[at + i] = source_keys[at + i];
-      args.values_out[at + i] = source_values[at + i];
-    }
-  }
-  uint32_t padded = 2u;
-  while (padded < length) padded <<= 1;
-  for (uint32_t size = 2u; size != 0u && size <= padded; size <<= 1) {
-    for (uint32_t stride = size >> 1; stride > 0u; stride >>= 1) {
-      __threadfence_block();
-      __syncthreads();
-      for (uint32_t i = threadIdx.x; i < padded / 2u; i += kSpreadThreads) {
-        const uint32_t low_bits = i & (stride - 1u);
-        const uint32_t a = ((i - low_bits) << 1) + low_bits;
-        const uint32_t b = stride == (size >> 1) ? ((i - low_bits) << 1) + size - 1u - low_bits : a + stride;
-        if (b >= length) continue;
-        const uint64_t ka = args.keys_out[at + a], kb = args.keys_out[at + b];
-        const int32_t va = args.values_out[at + a], vb = args.values_out[at + b];
-        if (kb < ka || (kb == ka && tie(vb) < tie(va))) {
-          args.keys_out[at + a] = kb;
-          args.keys_out[at + b] = ka;
-          args.values_out[at + a] = vb;
-          args.values_out[at + b] = va;
-        }
-      }
-    }
-  }
-  __threadfence_block();
-  __syncthreads();
-}
 
 __global__ __launch_bounds__(kSpreadThreads, 8) void spread_long_kernel(TileSortArgs args) {
   __shared__ SpreadShared s;
@@ -263,14 +273,14 @@ __global__ __launch_bounds__(kSpreadThreads, 8) void spread_long_kernel(TileSort
   // The spread ping-pongs between the two buffer pairs.
   uint64_t* const keys_of[2] = {const_cast<uint64_t*>(args.keys_in), args.keys_out};
   int32_t* const values_of[2] = {const_cast<int32_t*>(args.values_in), args.values_out};
-  const uint32_t queued = args.state[2] < args.run_capacity ? args.state[2] : args.run_capacity;
+  const uint32_t queued = args.state[2] < args.long_capacity ? args.state[2] : args.long_capacity;
   if (queued == 0u) return;
   for (;;) {
     __syncthreads();
     if (t == 0) s.item = atomicAdd(&args.state[3], 1u);
     __syncthreads();
     if (s.item >= queued) return;
-    const Run part = args.runs[args.run_capacity - 1u - s.item];
+    const Run part = args.long_runs[s.item];
     const int64_t list = part.begin;
     const uint32_t tile = part.tile;
     if (t == 0) {
@@ -319,7 +329,7 @@ __global__ __launch_bounds__(kSpreadThreads, 8) void spread_long_kernel(TileSort
         if (lo == hi) {  // uniform
           // No bin splits entries of one depth and one tie word.  Every other segment comes
           // out smaller: over an exact range, lo and hi fall into different bins.
-          sort_in_place(args, tie, base, count, source_keys, source_values);
+          sort_in_place<kSpreadThreads>(args, base, count, source_keys, source_values);
           continue;
         }
       }
@@ -395,10 +405,15 @@ __global__ __launch_bounds__(kSpreadThreads, 8) void spread_long_kernel(TileSort
         }
         if (low > bin) {
           const uint32_t length = s.first[low] - run_begin;
-          if (t == 0 && length != 0u) {
-            push_run(args, Run{static_cast<uint32_t>(base) + run_begin, length, tile, static_cast<uint32_t>(to)});
-          }
           bin = low;
+          if (length == 0u) continue;  // uniform
+          if (t == 0) {
+            s.queued = push_run(args, Run{static_cast<uint32_t>(base) + run_begin, length, tile,
+                                          static_cast<uint32_t>(to)});
+          }
+          __syncthreads();
+          if (!s.queued) sort_in_place<kSpreadThreads>(args, base + run_begin, length, keys_of[to], values_of[to]);
+          __syncthreads();  // s.queued read before the next run
           continue;
         }
         const uint32_t length = s.first[bin + 1] - run_begin;
@@ -413,7 +428,7 @@ __global__ __launch_bounds__(kSpreadThreads, 8) void spread_long_kernel(TileSort
           }
           __syncthreads();
         } else {
-          sort_in_place(args, tie, base + run_begin, length, keys_of[to], values_of[to]);
+          sort_in_place<kSpreadThreads>(args, base + run_begin, length, keys_of[to], values_of[to]);
         }
         ++bin;
       }
@@ -439,14 +454,20 @@ int launch_tile_sort(const vgr_scene& scene, const vgr_workspace& ws, const Scra
   args.records = scene.gaussian_ids != nullptr ? ws.records : nullptr;
   args.visible_capacity = ws.visible_capacity;
   args.partition = layout.partition;
-  // The look-back flags are read no more: their scratch holds the queue.  Every 8192
-  // entries make at most 32 crowded parts of over kSplitLeast entries, eight parts of
-  // longer lists (two neighbours hold over 2048; 32 of 512 entries under small tiles)
-  // and four runs per spread of the part or bin that holds them, of which a 32-bit
-  // depth and a 32-bit tie word allow six: 88 of 16 bytes, against at least 384 flags
-  // of 4 bytes.
-  args.runs = reinterpret_cast<Run*>(scratch + layout.sort_flags);
-  args.run_capacity = static_cast<uint32_t>(layout.sort_tiles * kRunsPerSortTile);
+  // The look-back flags are read no more: their scratch holds the queues, with a place
+  // per sort tile (at most 8192 entries) for a part of over 8192 entries, so those always
+  // fit.  The other parts number at most 88 per 8192 entries: 32 crowded ones of over
+  // kSplitLeast, 32 of longer lists (two neighbours hold over 512 entries under small
+  // tiles) and four runs per spread of the part or bin that holds them, of which a 32-bit
+  // depth and a 32-bit tie word allow six.  The default digits leave at least 127 places;
+  // explicit digits of four or five bits may leave fewer, and parts beyond them are
+  // sorted where they are found, by the workgroup that found them.
+  static_assert(sizeof(Run) == 16 && kSortThreads * kDefaultSortItems <= kRunCapacity,
+                "a part that is spread takes more entries than a sort tile");
+  args.long_runs = reinterpret_cast<Run*>(scratch + layout.sort_flags);
+  args.long_capacity = static_cast<uint32_t>(layout.sort_tiles);
+  args.runs = args.long_runs + args.long_capacity;
+  args.run_capacity = static_cast<uint32_t>(layout.sort_flag_words / 4 - layout.sort_tiles);
   args.state = reinterpret_cast<uint32_t*>(scratch + layout.work_counter) + 4;
   constexpr int64_t kMaxGrid = 1 << 22;
   const dim3 grid(static_cast<unsigned>(global_tiles < kMaxGrid ? global_tiles : kMaxGrid));
