@@ -205,3 +205,29 @@ def test_more_crowded_lists_than_queue_places(depths):
     np.testing.assert_array_equal(keys.astype(np.uint32), listed[:, 6].view(np.uint32))  # depth bits
     step = np.diff(keys.astype(np.int64))
     assert np.all((step > 0) | ((step == 0) & (np.diff(values) > 0)))
+
+
+@pytest.mark.parametrize("copies", [2, 40])
+@pytest.mark.parametrize("count,depths", [(1, "equal"), (200, "equal"), (200, "steps"), (5000, "equal"), (5000, "spread")])
+def test_a_camera_active_more_than_once(count, depths, copies):
+    """Its lists hold every Gaussian once per copy: longer than the scene, sorted all the same."""
+    dev = torch.device("cuda", 0)
+    backend = CustomHipBackend(output_srgb=False, max_visible_records=count * copies,
+                               max_intersections=count * copies)
+    service = RendererService(backend, height=16, width=16, max_views=copies)
+    service.initialize(stage=None, device=dev)
+    service.load_scene(0, **column_scene(count, depths).to(dev).as_kwargs())
+    viewmats, intrinsics = identity_rig(16)
+    service.render(viewmats.to(dev).repeat(copies, 1, 1), intrinsics.to(dev).repeat(copies, 1, 1),
+                   torch.zeros(copies, dtype=torch.int64, device=dev),
+                   active_camera_ids=torch.ones(copies, dtype=torch.int64, device=dev))
+    service.synchronize()
+    counters = backend.read_counters()
+    assert counters["tile_intersections"] == count * copies and not counters["intersection_overflow"]
+    keys = backend.workspace["keys_out"][: count * copies].cpu().numpy()
+    values = backend.workspace["values_out"][: count * copies].cpu().numpy()
+    depth_bits = backend.workspace["visible_depths"].cpu().numpy().view(np.uint32)
+    assert np.unique(values).size == values.size
+    np.testing.assert_array_equal(keys, (np.uint64(1) << np.uint64(32)) | depth_bits[values].astype(np.uint64))
+    step = np.diff(keys.astype(np.int64))
+    assert np.all((step > 0) | ((step == 0) & (np.diff(values) > 0)))

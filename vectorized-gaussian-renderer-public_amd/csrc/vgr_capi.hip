@@ -541,7 +541,7 @@ int render_submission(const vgr_scene& sc, const vgr_cameras& cams, const vgr_ou
       return status;
     if ((status = mark(2)) != 0) return status;
     if ((status = launch_ranges(ws, tiles, sorted_in_out != 0, stream)) != 0) return status;
-    if ((status = launch_tile_sort(sc, ws, layout, scratch_base, tiles, opt.tile_size, sorted_in_out != 0,
+    if ((status = launch_tile_sort(sc, cams, ws, layout, scratch_base, tiles, opt.tile_size, sorted_in_out != 0,
                                    stream)) != 0)
       return status;
     sorted_in_out = 1 - sorted_in_out;

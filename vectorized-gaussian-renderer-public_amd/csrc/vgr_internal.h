@@ -134,8 +134,9 @@ int launch_sort(const vgr_workspace& ws, const ScratchLayout& layout, char* scra
                 uint32_t spin_limit, hipStream_t stream, int* result_in_out_buffer);
 int launch_ranges(const vgr_workspace& ws, int64_t global_tiles, bool sorted_in_out,
                   hipStream_t stream);
-int launch_tile_sort(const vgr_scene& scene, const vgr_workspace& ws, const ScratchLayout& layout, char* scratch,
-                     int64_t global_tiles, int tile_size, bool partitioned_in_out, hipStream_t stream);
+int launch_tile_sort(const vgr_scene& scene, const vgr_cameras& cameras, const vgr_workspace& ws,
+                     const ScratchLayout& layout, char* scratch, int64_t global_tiles, int tile_size,
+                     bool partitioned_in_out, hipStream_t stream);
 int launch_composite(const vgr_scene& scene, const vgr_cameras& cameras,
                      const vgr_outputs& outputs, const vgr_options& options,
                      const vgr_workspace& ws, const ScratchLayout& layout,

@@ -439,8 +439,9 @@ __global__ __launch_bounds__(kSpreadThreads, 8) void spread_long_kernel(TileSort
 
 }  // namespace
 
-int launch_tile_sort(const vgr_scene& scene, const vgr_workspace& ws, const ScratchLayout& layout, char* scratch,
-                     int64_t global_tiles, int tile_size, bool partitioned_in_out, hipStream_t stream) {
+int launch_tile_sort(const vgr_scene& scene, const vgr_cameras& cameras, const vgr_workspace& ws,
+                     const ScratchLayout& layout, char* scratch, int64_t global_tiles, int tile_size, bool partitioned_in_out,
+                     hipStream_t stream) {
   if (global_tiles <= 0) return 0;
   TileSortArgs args;
   args.keys_in = partitioned_in_out ? ws.keys_out : ws.keys_in;
@@ -475,22 +476,23 @@ int launch_tile_sort(const vgr_scene& scene, const vgr_workspace& ws, const Scra
   // views of 5M Gaussians at tile size 1): one wave each.  8x8 and 16x16 tiles
   // hold hundreds to a few thousand entries: four waves and 2048 entries of LDS.
   const int64_t capacity = ws.intersection_capacity;
-  const int64_t gaussian_count = scene.gaussian_count;
   if (tile_size <= 4) {
     hipLaunchKernelGGL((tile_sort_kernel<64, 512, 512>), grid, dim3(64), 0, stream, args);
   } else {
     hipLaunchKernelGGL((tile_sort_kernel<256, 2048, 2048>), grid, dim3(256), 0, stream, args);
   }
-  // A Gaussian is at most once in a list, so a small scene has no long ones (nor
-  // crowded ones up to kSplitLeast).
+  // A list holds a Gaussian once for every time its camera is active (active_ids may
+  // repeat a camera), so a small scene has no long ones (nor crowded ones up to
+  // kSplitLeast).
+  const int64_t longest = scene.gaussian_count * (cameras.active_ids != nullptr ? cameras.active_count : 1);
   // Persistent grids of two workgroups per CU; an empty queue ends every one at once.
   constexpr int64_t kPersistent = 512;
-  if (gaussian_count > kRunCapacity) {
+  if (longest > kRunCapacity) {
     const int64_t most = capacity / kRunCapacity + 1;
     hipLaunchKernelGGL(spread_long_kernel, dim3(static_cast<unsigned>(most < kPersistent ? most : kPersistent)),
                        dim3(kSpreadThreads), 0, stream, args);
   }
-  if (gaussian_count > kSplitLeast) {
+  if (longest > kSplitLeast) {
     const int64_t most = capacity / kSplitLeast + 1;
     hipLaunchKernelGGL(run_sort_kernel, dim3(static_cast<unsigned>(most < kPersistent ? most : kPersistent)),
                        dim3(kRunThreads), 0, stream, args);
