@@ -141,6 +141,7 @@ struct CompositeArgs {
   const int32_t* tile_order;  // launch order of the (camera, tile) items
   const uint32_t* long_tiles;  // how many of the first in that order are long
   int64_t total_items;     // (camera, tile) items in the launch
+  int64_t first_item;      // of this launch: a grid holds less than 2^32 threads
   int active_count;
   int uniform_tiles;     // tiles per camera when every camera has the same resolution, else 0
   int output_srgb;
@@ -761,7 +762,7 @@ __global__ __launch_bounds__(kRaster* kRaster, kRaster == 16 ? 4 : 1) void compo
   // Workgroups go round robin over the XCDs: those of one XCD (blockIdx.x mod kXcds)
   // take kXcdBins neighbouring bins at a time, the raster tiles of a bin in turn.
   const int split = bin_size / kRaster;
-  const int64_t turn = blockIdx.x / kXcds;
+  const int64_t turn = (args.first_item + blockIdx.x) / kXcds;
   const int64_t bin_turn = turn / (split * split);
   const int part = static_cast<int>(turn - bin_turn * (split * split));
   const int64_t bin = (bin_turn / kXcdBins * kXcds + blockIdx.x % kXcds) * kXcdBins + bin_turn % kXcdBins;
@@ -923,6 +924,18 @@ __global__ __launch_bounds__(kRaster* kRaster, kRaster == 16 ? 4 : 1) void compo
   store_pixel<kFull>(args, pixel, transmittance, red, green, blue, depth_sum, best_weight, best_gaussian);
 }
 
+// Launches items [0, blocks), one workgroup each, in grids of less than 2^32 threads,
+// which is what a dispatch holds.  Slices are whole multiples of the XCD count.
+template <int kThreads, typename Args, typename Launch>
+void launch_slices(const Args& args, int64_t blocks, Launch&& launch) {
+  constexpr int64_t kMost = ((1LL << 32) - 1) / kThreads / kXcds * kXcds;
+  for (int64_t first = 0; first < blocks; first += kMost) {
+    Args slice = args;
+    slice.first_item = first;
+    launch(slice, dim3(static_cast<unsigned>(blocks - first < kMost ? blocks - first : kMost)));
+  }
+}
+
 template <int kRaster>
 void launch_ray(const CompositeArgs& args, const vgr_options& options, const float* ray_records, int active_count,
                 bool full, hipStream_t stream) {
@@ -930,15 +943,16 @@ void launch_ray(const CompositeArgs& args, const vgr_options& options, const flo
   const int bins = args.uniform_tiles;
   constexpr int64_t kRound = kXcds * kXcdBins;
   const int64_t blocks = (static_cast<int64_t>(active_count) * bins + kRound - 1) / kRound * kRound * split * split;
-  if (blocks <= 0) return;
-  const dim3 grid(static_cast<unsigned>(blocks)), block(kRaster * kRaster);
-  if (full) {
-    hipLaunchKernelGGL((composite_ray_kernel<kRaster, true>), grid, block, 0, stream, args, ray_records,
-                       options.gaussian_support_sigma, bins, options.tile_size);
-  } else {
-    hipLaunchKernelGGL((composite_ray_kernel<kRaster, false>), grid, block, 0, stream, args, ray_records,
-                       options.gaussian_support_sigma, bins, options.tile_size);
-  }
+  launch_slices<kRaster * kRaster>(args, blocks, [&](const CompositeArgs& slice, const dim3& grid) {
+    const dim3 block(kRaster * kRaster);
+    if (full) {
+      hipLaunchKernelGGL((composite_ray_kernel<kRaster, true>), grid, block, 0, stream, slice, ray_records,
+                         options.gaussian_support_sigma, bins, options.tile_size);
+    } else {
+      hipLaunchKernelGGL((composite_ray_kernel<kRaster, false>), grid, block, 0, stream, slice, ray_records,
+                         options.gaussian_support_sigma, bins, options.tile_size);
+    }
+  });
 }
 
 // Minimum waves per SIMD for 16x16 tiles (launch-bounds occupancy target): eight
@@ -955,7 +969,7 @@ constexpr int kCompositeWavesPerSimd =
 template <int kTileSize, int kBatch, bool kFull, bool kCount, bool kCheckpoint, int kDegree = -1>
 __global__ __launch_bounds__(kTileSize* kTileSize, (kCompositeWavesPerSimd<kTileSize, kBatch, kCount, kDegree>)) void
 composite_kernel(CompositeArgsFor<kDegree> args) {
-  const int64_t block = args.tile_order != nullptr ? args.tile_order[blockIdx.x] : blockIdx.x;
+  const int64_t block = args.tile_order != nullptr ? args.tile_order[blockIdx.x] : args.first_item + blockIdx.x;
   __shared__ WaveLists<kTileSize, kBatch> s;
   composite_tile<kTileSize, kBatch, kFull, kCount, kCheckpoint, kDegree>(args, block, s);
 }
@@ -1071,8 +1085,10 @@ void launch_variant(const CompositeArgsFor<kDegree>& args, int64_t blocks, hipSt
   // a queue does, at eight waves a SIMD instead of six and without the queue's barriers
   // (256 cameras of four resolutions, 170k tiles: 21.1 -> 17.0 ms; tile-front lists of
   // 1024 room cameras 6.49 -> 5.87, of 256 with checkpoints 2.66 -> 2.39).
-  hipLaunchKernelGGL((composite_kernel<kTileSize, kBatch, kFull, kCount, kCheckpoint, kDegree>),
-                     dim3(static_cast<unsigned>(blocks)), block, 0, stream, args);
+  launch_slices<kTileSize * kTileSize>(args, blocks, [&](const CompositeArgsFor<kDegree>& slice, const dim3& grid) {
+    hipLaunchKernelGGL((composite_kernel<kTileSize, kBatch, kFull, kCount, kCheckpoint, kDegree>), grid, block, 0,
+                       stream, slice);
+  });
 }
 
 // Tile-front lists (16x16 tiles, 256-entry batches): records recomputed per SH degree.
@@ -1254,6 +1270,7 @@ int launch_composite(const vgr_scene& scene, const vgr_cameras& cameras, const v
     return 0;
   }
   args.total_items = blocks;
+  args.first_item = 0;
   args.work_counter = reinterpret_cast<uint32_t*>(const_cast<char*>(scratch) + layout.work_counter);
   // Longest tiles first pays when the grid is a few waves deep per SIMD; on deep
   // grids the tail is short already.

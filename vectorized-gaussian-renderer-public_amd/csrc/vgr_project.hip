@@ -32,13 +32,13 @@ constexpr int kScanTile = kBlockThreads * kScanItems;
 __global__ __launch_bounds__(kWave) void build_camera_table_kernel(
     const float* __restrict__ viewmats, const float* __restrict__ intrinsics,
     const float* __restrict__ env_xforms, const int64_t* __restrict__ camera_scene_ids,
-    const int64_t* __restrict__ active_ids, int batch,
+    const int64_t* __restrict__ active_ids, int first_active, int batch,
     const int32_t* __restrict__ widths, const int32_t* __restrict__ heights,
     const int64_t* __restrict__ pixel_offsets, int default_width, int default_height,
     int tile_size, const int64_t* __restrict__ registered_scene_ids,
     const int64_t* __restrict__ scene_offsets, int scene_count,
     CameraParams* __restrict__ table) {
-  const int a = blockIdx.x;
+  const int a = first_active + static_cast<int>(blockIdx.x);
   const int lane = threadIdx.x;
   CameraParams p;
   const int64_t camera64 = active_ids == nullptr ? a : active_ids[a];
@@ -705,11 +705,18 @@ __global__ void precompute_covariances_kernel(const float* __restrict__ scales, 
 int launch_camera_table(const vgr_scene& scene, const vgr_cameras& cameras, const vgr_options& options,
                         CameraParams* table, hipStream_t stream) {
   if (cameras.active_count <= 0) return 0;
-  hipLaunchKernelGGL(build_camera_table_kernel, dim3(cameras.active_count), dim3(kWave), 0, stream, cameras.viewmats,
-                     cameras.intrinsics, cameras.env_xforms, cameras.scene_ids, cameras.active_ids,
-                     cameras.batch, cameras.widths, cameras.heights, cameras.pixel_offsets,
-                     options.width, options.height, options.tile_size, scene.registered_scene_ids,
-                     scene.scene_offsets, scene.scene_count, table);
+  // A grid holds less than 2^32 threads.
+  constexpr int kMost = 1 << 25;
+  for (int first = 0; first < cameras.active_count;) {
+    const int count = cameras.active_count - first < kMost ? cameras.active_count - first : kMost;
+    hipLaunchKernelGGL(build_camera_table_kernel, dim3(count), dim3(kWave), 0, stream, cameras.viewmats,
+                       cameras.intrinsics, cameras.env_xforms, cameras.scene_ids, cameras.active_ids, first,
+                       cameras.batch, cameras.widths, cameras.heights, cameras.pixel_offsets, options.width,
+                       options.height, options.tile_size, scene.registered_scene_ids, scene.scene_offsets,
+                       scene.scene_count, table);
+    if (count == cameras.active_count - first) break;
+    first += count;
+  }
   const hipError_t status = hipGetLastError();
   if (status != hipSuccess) {
     set_error("camera table launch failed: %s", hipGetErrorString(status));
