@@ -1,5 +1,5 @@
 """Depth order inside every tile (gfx950), at the sizes where the tile sort changes its way:
-list lengths around a wave, one bin per thread, the LDS capacities (512, 2048 and 8192 entries)
+list lengths around a wave and its share of the LDS, one bin per thread, the LDS capacities (512, 2048 and 8192 entries)
 and the lists spread over depth bins in global memory; depths spread, all equal, half equal, and
 in a few float steps beside one far outlier.
 
@@ -97,6 +97,26 @@ def test_one_pixel_lists(count, depths):
     scene.scales = torch.full_like(scene.scales, 4.0)  # wide enough to reach every pixel
     backend, _ = render(scene, 4, tile_size=1, deterministic=True)
     assert check_lists(backend) == count
+
+
+@pytest.mark.parametrize("depths", DEPTHS)
+@pytest.mark.parametrize("counts", [(0, 1, 512, 513), (2048, 300, 2049, 64), (400, 0, 0, 8193), (257, 256, 9000, 1)])
+def test_neighbouring_small_tiles_of_different_lengths(counts, depths):
+    """Four neighbouring 4x4 tiles share a workgroup: each wave's own list, then the longer and the
+    crowded ones together.  Sixteen tiles, every list in its own order of lengths."""
+    size, tiles = 16, 16
+    counts = np.array(counts * 4)
+    scene = column_scene(int(counts.sum()), depths)
+    tile = np.random.default_rng(1).permutation(np.repeat(np.arange(tiles), counts))
+    z = scene.means[:, 2].numpy().astype(np.float64)
+    centre = np.stack([tile % 4, tile // 4], axis=1) * 4.0 + 2.0
+    scene.means[:, :2] = torch.tensor((centre - size / 2) * z[:, None] / size, dtype=torch.float32)
+    scene.scales = torch.full_like(scene.scales, 1.0e-4)
+    scene.opacities = torch.full_like(scene.opacities, 0.006)  # reaches one pixel
+    backend, _ = render(scene, size, tile_size=4)
+    check_lists(backend)
+    lengths = (backend.workspace["tile_ends"] - backend.workspace["tile_starts"]).cpu().numpy()
+    np.testing.assert_array_equal(lengths[:tiles], counts)
 
 
 @pytest.mark.parametrize("depths", ["equal", "half", "steps"])

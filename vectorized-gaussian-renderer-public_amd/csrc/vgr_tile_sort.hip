@@ -7,10 +7,12 @@
 // radix passes over the depth bits move 72 and pay a look-back chain each.
 //
 //   tile_sort_kernel  : one workgroup per tile sorts lists of up to 2048 entries
-//                       (512 under small tiles) in LDS.  A longer list is cut where
-//                       the leading depth bits change into parts that fit: they are
-//                       sorted one after the other, or queued when there are many
-//                       or one does not fit;
+//                       in LDS.  A longer list is cut where the leading depth bits
+//                       change into parts that fit: they are sorted one after the
+//                       other, or queued when there are many or one does not fit;
+//   small_tile_sort_kernel : the same for tiles of up to 4x4 pixels, of which a
+//                       workgroup takes four: a list of up to 512 entries is one
+//                       wave's, the rest the workgroup's;
 //   spread_long_kernel: parts that do not fit the LDS of run_sort_kernel either are
 //                       spread over 4096 depth bins in global memory and queued as
 //                       runs of whole bins that do; a bin that does not fit is spread
@@ -38,6 +40,9 @@ struct alignas(16) Run {
   uint32_t begin, count, tile, pair;
 };
 
+constexpr int kTileThreads = 256;
+constexpr int kTileCapacity = 2048;  // 24 KB of LDS: six workgroups per CU
+constexpr int kWaveCapacity = 512;   // of a wave that sorts a list alone
 constexpr int kRunThreads = 512;
 constexpr int kRunCapacity = 8192;
 constexpr int kRunBins = 3072;  // 78 KB of LDS with the entries: two workgroups per CU
@@ -156,64 +161,127 @@ __device__ __forceinline__ uint32_t prefix_length(S& s, uint32_t begin, uint32_t
   return low - begin;
 }
 
-template <int kThreads, int kCapacity, int kBins>
-__global__ __launch_bounds__(kThreads, 6) void tile_sort_kernel(TileSortArgs args) {
-  __shared__ TileSort<kThreads, kCapacity, kBins> s;
+// Sorts the list [start, start + count) of a tile, or queues it or parts of it, with the
+// workgroup.  Without kSplit crowded parts are queued.  Ends behind a barrier.
+template <bool kSplit, int kThreads, int kCapacity, int kBins>
+__device__ __forceinline__ void sort_list(const TileSortArgs& args, TileSort<kThreads, kCapacity, kBins>& s,
+                                          bool& s_queued, int64_t tile, int64_t start, uint32_t count) {
+  // Uniform bases and 32-bit offsets: the addresses stay out of the vector registers.
+  const uint32_t* const all_depths = reinterpret_cast<const uint32_t*>(args.keys_in + start);
+  const auto lead = [&](uint32_t i) {
+    return (all_depths[2u * static_cast<uint64_t>(i)] - args.partition.depth_base) >> args.partition.lead_shift;
+  };
+  const uint64_t tile_bits = static_cast<uint64_t>(tile) << 32;
+  // Lists of a few parts are sorted here; more parts share the work with run_sort_kernel.
+  const bool here = count <= 4u * kCapacity;
+  for (uint32_t begin = 0u; begin < count;) {  // uniform
+    uint32_t n = count - begin;
+    if (n > static_cast<uint32_t>(kCapacity)) {
+      // Whole leading-bit groups that fit, or the one group that does not.
+      const uint32_t next = lead(begin + kCapacity);
+      n = prefix_length<kThreads>(s, begin, begin + kCapacity, [&](uint32_t i) { return lead(i) < next; });
+      if (n == 0u) {
+        n = kCapacity + prefix_length<kThreads>(s, begin + kCapacity, count,
+                                                [&](uint32_t i) { return lead(i) <= next; });
+      }
+    }
+    bool sorted = false;
+    if (n <= static_cast<uint32_t>(kCapacity) && here) {
+      const uint32_t* const depths = all_depths + 2u * static_cast<uint64_t>(begin);
+      const int32_t* const list = args.values_in + start + begin;
+      uint64_t* const keys_out = args.keys_out + start + begin;
+      int32_t* const values_out = args.values_out + start + begin;
+      sorted = tile_sort<kSplit>(
+          s, n, [&](uint32_t i) { return depths[2u * i]; }, [&](uint32_t i) { return list[i]; },
+          TieOrder{args.records, args.visible_capacity}, [&](uint32_t rank, uint32_t key, int32_t value) {
+            keys_out[rank] = tile_bits | key;
+            values_out[rank] = value;
+          });
+    }
+    if (!sorted) {  // uniform
+      if (threadIdx.x == 0) {
+        s_queued = push_run(args, Run{static_cast<uint32_t>(start) + begin, n, static_cast<uint32_t>(tile), 0u});
+      }
+      __syncthreads();
+      if (!s_queued) sort_in_place<kThreads>(args, start + begin, n, args.keys_in, args.values_in);
+    }
+    begin += n;
+    __syncthreads();  // LDS free for the next part
+  }
+}
+
+// A failed partition leaves lists that overlap and slots nobody wrote: the render is
+// invalid and reported as such, and its lists are emptied rather than sorted.
+
+// 8x8 and 16x16 tiles: a workgroup per tile.
+__global__ __launch_bounds__(kTileThreads, 6) void tile_sort_kernel(TileSortArgs args) {
+  __shared__ TileSort<kTileThreads, kTileCapacity, kTileCapacity> s;
   __shared__ bool s_queued;
-  // A failed partition leaves lists that overlap and slots nobody wrote: the render is
-  // invalid and reported as such, and its lists are emptied rather than sorted.
   const bool failed = *args.failures != 0;
   for (int64_t tile = blockIdx.x; tile < args.tiles; tile += gridDim.x) {
     const int64_t start = args.tile_starts[tile];
-    const int64_t count64 = static_cast<int64_t>(args.tile_ends[tile]) - start;
-    if (count64 <= 0) continue;
+    const int64_t count = static_cast<int64_t>(args.tile_ends[tile]) - start;
+    if (count <= 0) continue;
     if (failed) {
       if (threadIdx.x == 0) args.tile_ends[tile] = static_cast<int32_t>(start);
       continue;
     }
-    const uint32_t count = static_cast<uint32_t>(count64);
-    // Uniform bases and 32-bit offsets: the addresses stay out of the vector registers.
-    const uint32_t* const all_depths = reinterpret_cast<const uint32_t*>(args.keys_in + start);
-    const auto lead = [&](uint32_t i) {
-      return (all_depths[2u * static_cast<uint64_t>(i)] - args.partition.depth_base) >> args.partition.lead_shift;
-    };
-    const uint64_t tile_bits = static_cast<uint64_t>(tile) << 32;
-    // Lists of a few parts are sorted here; more parts share the work with run_sort_kernel.
-    const bool here = count <= 4u * kCapacity;
-    for (uint32_t begin = 0u; begin < count;) {  // uniform
-      uint32_t n = count - begin;
-      if (n > static_cast<uint32_t>(kCapacity)) {
-        // Whole leading-bit groups that fit, or the one group that does not.
-        const uint32_t next = lead(begin + kCapacity);
-        n = prefix_length<kThreads>(s, begin, begin + kCapacity, [&](uint32_t i) { return lead(i) < next; });
-        if (n == 0u) {
-          n = kCapacity + prefix_length<kThreads>(s, begin + kCapacity, count,
-                                                  [&](uint32_t i) { return lead(i) <= next; });
-        }
-      }
-      bool sorted = false;
-      if (n <= static_cast<uint32_t>(kCapacity) && here) {
-        const uint32_t* const depths = all_depths + 2u * static_cast<uint64_t>(begin);
-        const int32_t* const list = args.values_in + start + begin;
-        uint64_t* const keys_out = args.keys_out + start + begin;
-        int32_t* const values_out = args.values_out + start + begin;
-        sorted = tile_sort<false>(
-            s, n, [&](uint32_t i) { return depths[2u * i]; }, [&](uint32_t i) { return list[i]; },
-            TieOrder{args.records, args.visible_capacity}, [&](uint32_t rank, uint32_t key, int32_t value) {
-              keys_out[rank] = tile_bits | key;
-              values_out[rank] = value;
-            });
-      }
-      if (!sorted) {  // uniform
-        if (threadIdx.x == 0) {
-          s_queued = push_run(args, Run{static_cast<uint32_t>(start) + begin, n, static_cast<uint32_t>(tile), 0u});
-        }
-        __syncthreads();
-        if (!s_queued) sort_in_place<kThreads>(args, start + begin, n, args.keys_in, args.values_in);
-      }
-      begin += n;
-      __syncthreads();  // LDS free for the next part
-    }
+    sort_list<false>(args, s, s_queued, tile, start, static_cast<uint32_t>(count));
+  }
+}
+
+// Tiles of up to 4x4 pixels: a workgroup takes four, each wave the list of one if it
+// fits the wave's share of the LDS, then the whole workgroup those that are longer or
+// crowded, which it splits itself: the lists of pixels that look at a wall are.  Their
+// lengths are known on the device only and run from 68 entries on average (128x128
+// views of a 5M-Gaussian room at tile size 1, with the depth cutoff) to 660 (without)
+// and thousands (4x4 tiles).  Lists sorted by one wave each, with longer and crowded
+// ones queued for run_sort_kernel, against this: depth order of that room with the
+// cutoff 120 -> 114 us and without 2,208 -> 1,413, of a room of 1M Gaussians at tile
+// size 1 532 -> 394 and at 2x2 402 -> 290.
+constexpr int kSmallTiles = kTileThreads / kWave;
+
+union SmallTiles {
+  TileSort<kWave, kWaveCapacity, kWaveCapacity> of_wave[kSmallTiles];
+  TileSort<kTileThreads, kTileCapacity, kTileCapacity> of_group;
+};
+
+// Not a loop over groups of tiles: hoisted out of one, the addresses of both forms spill.
+__global__ __launch_bounds__(kTileThreads, 6) void small_tile_sort_kernel(TileSortArgs args, int64_t first_tile) {
+  __shared__ SmallTiles s;
+  __shared__ bool s_queued;
+  __shared__ uint32_t s_left[kSmallTiles];  // entries of the lists that the waves leave to the workgroup
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int64_t first = first_tile + static_cast<int64_t>(blockIdx.x) * kSmallTiles;
+  const int64_t own = first + wave;
+  const int32_t start = __builtin_amdgcn_readfirstlane(own < args.tiles ? args.tile_starts[own] : 0);
+  const int32_t count = __builtin_amdgcn_readfirstlane(own < args.tiles ? args.tile_ends[own] : 0) - start;
+  if (*args.failures != 0) {
+    if (count > 0 && (threadIdx.x & (kWave - 1)) == 0) args.tile_ends[own] = start;
+    return;
+  }
+  bool sorted = count <= 0;
+  if (count > 0 && count <= kWaveCapacity) {
+    const uint32_t* const depths = reinterpret_cast<const uint32_t*>(args.keys_in + start);
+    const int32_t* const list = args.values_in + start;
+    uint64_t* const keys_out = args.keys_out + start;
+    int32_t* const values_out = args.values_out + start;
+    const uint64_t tile_bits = static_cast<uint64_t>(own) << 32;
+    sorted = tile_sort<false>(
+        s.of_wave[wave], static_cast<uint32_t>(count), [&](uint32_t i) { return depths[2u * i]; },
+        [&](uint32_t i) { return list[i]; }, TieOrder{args.records, args.visible_capacity},
+        [&](uint32_t rank, uint32_t key, int32_t value) {
+          keys_out[rank] = tile_bits | key;
+          values_out[rank] = value;
+        });
+  }
+  if ((threadIdx.x & (kWave - 1)) == 0) s_left[wave] = sorted ? 0u : static_cast<uint32_t>(count);
+  if (!__syncthreads_or(sorted ? 0 : 1)) return;
+  for (int q = 0; q < kSmallTiles; ++q) {
+    const uint32_t left = __builtin_amdgcn_readfirstlane(s_left[q]);
+    if (left == 0u) continue;  // uniform
+    const int64_t list_start = __builtin_amdgcn_readfirstlane(args.tile_starts[first + q]);
+    sort_list<true>(args, s.of_group, s_queued, first + q, list_start, left);
   }
 }
 
@@ -471,15 +539,17 @@ int launch_tile_sort(const vgr_scene& scene, const vgr_cameras& cameras, const v
   args.run_capacity = static_cast<uint32_t>(layout.sort_flag_words / 4 - layout.sort_tiles);
   args.state = reinterpret_cast<uint32_t*>(scratch + layout.work_counter) + 4;
   constexpr int64_t kMaxGrid = 1 << 22;
-  const dim3 grid(static_cast<unsigned>(global_tiles < kMaxGrid ? global_tiles : kMaxGrid));
-  // Tiles of up to 4x4 pixels have short lists (68 entries on average for 128x128
-  // views of 5M Gaussians at tile size 1): one wave each.  8x8 and 16x16 tiles
-  // hold hundreds to a few thousand entries: four waves and 2048 entries of LDS.
   const int64_t capacity = ws.intersection_capacity;
   if (tile_size <= 4) {
-    hipLaunchKernelGGL((tile_sort_kernel<64, 512, 512>), grid, dim3(64), 0, stream, args);
+    constexpr int64_t kMost = kMaxGrid * kSmallTiles;  // tiles of a grid
+    for (int64_t first = 0; first < global_tiles; first += kMost) {
+      const int64_t rest = global_tiles - first < kMost ? global_tiles - first : kMost;
+      hipLaunchKernelGGL(small_tile_sort_kernel, dim3(static_cast<unsigned>((rest + kSmallTiles - 1) / kSmallTiles)),
+                         dim3(kTileThreads), 0, stream, args, first);
+    }
   } else {
-    hipLaunchKernelGGL((tile_sort_kernel<256, 2048, 2048>), grid, dim3(256), 0, stream, args);
+    hipLaunchKernelGGL(tile_sort_kernel, dim3(static_cast<unsigned>(global_tiles < kMaxGrid ? global_tiles : kMaxGrid)),
+                       dim3(kTileThreads), 0, stream, args);
   }
   // A list holds a Gaussian once for every time its camera is active (active_ids may
   // repeat a camera), so a small scene has no long ones (nor crowded ones up to

@@ -87,17 +87,36 @@ __device__ __forceinline__ uint32_t wave_inclusive_sum_u32(uint32_t v) {
   return v;
 }
 
-// Smallest and largest of the workgroup's (lo, hi); ends behind a barrier that
-// also orders LDS writes made before the call.
+// Barrier of kThreads threads that sort a list together: a wave, which runs its LDS and
+// memory instructions in order and waits only for the compiler, or the whole workgroup.
+template <int kThreads>
+__device__ __forceinline__ void team_sync() {
+  if constexpr (kThreads == kWave) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
+}
+
+// The calling thread's number among the kThreads that sort a list together.
+template <int kThreads>
+__device__ __forceinline__ uint32_t team_thread() {
+  return kThreads == kWave ? threadIdx.x & (kWave - 1) : threadIdx.x;
+}
+
+// Smallest and largest of the team's (lo, hi); ends behind a barrier that also orders
+// LDS writes made before the call.
 template <typename S>
 __device__ __forceinline__ void block_min_max(S& s, uint32_t& lo, uint32_t& hi) {
+  const uint32_t t = team_thread<S::kWaves * kWave>();
   lo = wave_min_u32(lo);
   hi = wave_max_u32(hi);
-  if ((threadIdx.x & (kWave - 1)) == 0) {
-    s.wave_a[threadIdx.x / kWave] = lo;
-    s.wave_b[threadIdx.x / kWave] = hi;
+  if ((t & (kWave - 1)) == 0) {
+    s.wave_a[t / kWave] = lo;
+    s.wave_b[t / kWave] = hi;
   }
-  __syncthreads();
+  team_sync<S::kWaves * kWave>();
 #pragma unroll
   for (int w = 0; w < S::kWaves; ++w) {
     lo = s.wave_a[w] < lo ? s.wave_a[w] : lo;
@@ -119,7 +138,7 @@ __device__ __forceinline__ bool tile_sort(TileSort<kThreads, kCapacity, kBins>& 
                                           Value&& value_of, Tie&& tie, Emit&& emit) {
   using S = TileSort<kThreads, kCapacity, kBins>;
   constexpr int kItems = S::kItems;
-  const uint32_t t = threadIdx.x;
+  const uint32_t t = team_thread<kThreads>();
   const int lane = t & (kWave - 1);
   const int wave = t / kWave;
   uint32_t keys[kItems];
@@ -154,7 +173,7 @@ __device__ __forceinline__ bool tile_sort(TileSort<kThreads, kCapacity, kBins>& 
     ranks[r] = 0u;
     if (r * kThreads + t < n) ranks[r] = atomicAdd(&s.start[bin_of(keys[r])], 1u);
   }
-  __syncthreads();
+  team_sync<kThreads>();
   // Exclusive scan of the counters (per consecutive bins per thread) and the fullest bin.
   uint32_t own = 0u, fullest = 0u;
   for (uint32_t b = 0; b < per; ++b) {
@@ -168,7 +187,7 @@ __device__ __forceinline__ bool tile_sort(TileSort<kThreads, kCapacity, kBins>& 
     s.wave_a[wave] = inclusive;
     s.wave_b[wave] = fullest;
   }
-  __syncthreads();
+  team_sync<kThreads>();
   uint32_t running = inclusive - own;
 #pragma unroll
   for (int w = 0; w < S::kWaves; ++w) {
@@ -189,16 +208,16 @@ __device__ __forceinline__ bool tile_sort(TileSort<kThreads, kCapacity, kBins>& 
     const uint32_t first = s.start[bin];
     return first + __umulhi(bin_of.fraction(key), s.start[bin + 1] - first);
   };
-  __syncthreads();
+  team_sync<kThreads>();
   if (kSplit && crowded) {
     // The entries are loaded again rather than kept: registers that only this path
     // uses would cost every list some of its waves.
     uint32_t* const parts = reinterpret_cast<uint32_t*>(s.values);
     for (uint32_t i = t; i < n; i += kThreads) parts[i] = 0u;
-    __syncthreads();
+    team_sync<kThreads>();
 #pragma unroll 1
     for (uint32_t i = t; i < n; i += kThreads) atomicAdd(&parts[part_of(key_of(i))], 1u);
-    __syncthreads();
+    team_sync<kThreads>();
     const uint32_t share = (n + kThreads - 1) / kThreads;
     const uint32_t share_begin = t * share, share_end = share_begin + share < n ? share_begin + share : n;
     own = 0u;
@@ -215,7 +234,7 @@ __device__ __forceinline__ bool tile_sort(TileSort<kThreads, kCapacity, kBins>& 
       s.wave_a[wave] = up_to;
       s.wave_b[wave] = fullest;
     }
-    __syncthreads();
+    team_sync<kThreads>();
     running = up_to - own;
     for (int w = 0; w < S::kWaves; ++w) {
       if (w < wave) running += s.wave_a[w];
@@ -227,10 +246,10 @@ __device__ __forceinline__ bool tile_sort(TileSort<kThreads, kCapacity, kBins>& 
       parts[i] = running;
       running += c;
     }
-    __syncthreads();
+    team_sync<kThreads>();
 #pragma unroll 1
     for (uint32_t i = t; i < n; i += kThreads) s.keys[atomicAdd(&parts[part_of(key_of(i))], 1u)] = i;
-    __syncthreads();
+    team_sync<kThreads>();
 #pragma unroll
     for (int r = 0; r < kItems; ++r) {
       const uint32_t i = r * kThreads + t;
@@ -238,7 +257,7 @@ __device__ __forceinline__ bool tile_sort(TileSort<kThreads, kCapacity, kBins>& 
       keys[r] = key_of(entry);
       values[r] = value_of(entry);
     }
-    __syncthreads();
+    team_sync<kThreads>();
 #pragma unroll
     for (int r = 0; r < kItems; ++r) {
       const uint32_t i = r * kThreads + t;
@@ -247,7 +266,7 @@ __device__ __forceinline__ bool tile_sort(TileSort<kThreads, kCapacity, kBins>& 
         s.values[i] = values[r];
       }
     }
-    __syncthreads();
+    team_sync<kThreads>();
     if (fullest <= S::kPartCrowd) {  // uniform over the workgroup
 #pragma unroll 1
       for (uint32_t i = t; i < n; i += kThreads) {
@@ -288,7 +307,7 @@ __device__ __forceinline__ bool tile_sort(TileSort<kThreads, kCapacity, kBins>& 
             }
           }
         }
-        __syncthreads();
+        team_sync<kThreads>();
       }
     }
     for (uint32_t i = t; i < n; i += kThreads) emit(i, s.keys[i], s.values[i]);
@@ -302,7 +321,7 @@ __device__ __forceinline__ bool tile_sort(TileSort<kThreads, kCapacity, kBins>& 
       s.values[position] = values[r];
     }
   }
-  __syncthreads();
+  team_sync<kThreads>();
   // Not unrolled: the workgroups sharing the CU hide the reads, and the registers
   // that eight bins at a time would take cost some of them.
 #pragma unroll 1
