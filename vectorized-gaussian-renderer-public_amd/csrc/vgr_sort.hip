@@ -543,10 +543,14 @@ int launch_sort(const vgr_workspace& ws, const ScratchLayout& layout, char* scra
                      digit_bits, passes, tiles, layout.sort_tile, histogram, tickets, flags, global_tiles, ws.tile_starts,
                      ws.tile_ends, reinterpret_cast<uint32_t*>(scratch + layout.work_counter) + 4);
   const int items = layout.sort_tile / kSortThreads;
+  // Every workgroup ends with an atomic per digit value on the same counters, and 512 of
+  // them (eight waves a CU) are too few to read at the rate of the memory: 87M keys
+  // 500 / 275 / 188 us with 512 / 1,024 / 2,048 workgroups, 9M 59 / 46 / 55.
   int64_t histogram_blocks = (capacity + kBlockThreads * 16 - 1) / (kBlockThreads * 16);
-  // Every workgroup ends with an atomic per digit value on the same counters: 512 of
-  // them already read at the rate of the memory.
-  histogram_blocks = histogram_blocks > 512 ? 512 : (histogram_blocks < 1 ? 1 : histogram_blocks);
+  if (histogram_blocks > 1024) {
+    histogram_blocks = histogram_blocks / 2 < 1024 ? 1024 : (histogram_blocks / 2 > 2048 ? 2048 : histogram_blocks / 2);
+  }
+  histogram_blocks = histogram_blocks < 1 ? 1 : histogram_blocks;
   hipLaunchKernelGGL(sort_histogram_kernel, dim3(static_cast<unsigned>(histogram_blocks)), dim3(kBlockThreads), 0,
                      stream, ws.keys_in, ws.counters, capacity, pk, digit_bits, passes, histogram);
   hipLaunchKernelGGL(sort_digit_scan_kernel, dim3(1), dim3(kSortThreads), 0, stream, histogram, digit_bits, passes,
