@@ -545,7 +545,8 @@ int launch_sort(const vgr_workspace& ws, const ScratchLayout& layout, char* scra
   const int items = layout.sort_tile / kSortThreads;
   // Every workgroup ends with an atomic per digit value on the same counters, and 512 of
   // them (eight waves a CU) are too few to read at the rate of the memory: 87M keys
-  // 500 / 275 / 188 us with 512 / 1,024 / 2,048 workgroups, 9M 59 / 46 / 55.
+  // 500 / 275 / 188 us with 512 / 1,024 / 2,048 workgroups, 9M 59 / 46 / 55; 127M of 64
+  // VGA views 828 with 512 and 296 with this rule.
   int64_t histogram_blocks = (capacity + kBlockThreads * 16 - 1) / (kBlockThreads * 16);
   if (histogram_blocks > 1024) {
     histogram_blocks = histogram_blocks / 2 < 1024 ? 1024 : (histogram_blocks / 2 > 2048 ? 2048 : histogram_blocks / 2);

@@ -56,7 +56,7 @@ struct TileSortArgs {
   int32_t* tile_ends;
   int64_t tiles;
   PartitionKey partition;
-  const int64_t* failures;    // look-back waits the partition gave up: its order is wrong
+  int64_t* failures;          // look-back waits the partition gave up: its order is wrong
   const vgr_record* records;  // spatially ordered scenes: ties by the record's Gaussian ID; else null
   int64_t visible_capacity;
   Run* runs;                  // queue of the parts for run_sort_kernel
@@ -162,8 +162,9 @@ __device__ __forceinline__ uint32_t prefix_length(S& s, uint32_t begin, uint32_t
 }
 
 // Sorts the list [start, start + count) of a tile, or queues it or parts of it, with the
-// workgroup.  Without kSplit crowded parts are queued.  Ends behind a barrier.
-template <bool kSplit, int kThreads, int kCapacity, int kBins>
+// workgroup.  Without kSplit crowded parts are queued; kMayRefuse where the queue may have
+// no place for them (launch_tile_sort).  Ends behind a barrier.
+template <bool kSplit, bool kMayRefuse, int kThreads, int kCapacity, int kBins>
 __device__ __forceinline__ void sort_list(const TileSortArgs& args, TileSort<kThreads, kCapacity, kBins>& s,
                                           bool& s_queued, int64_t tile, int64_t start, uint32_t count) {
   // Uniform bases and 32-bit offsets: the addresses stay out of the vector registers.
@@ -200,10 +201,18 @@ __device__ __forceinline__ void sort_list(const TileSortArgs& args, TileSort<kTh
     }
     if (!sorted) {  // uniform
       if (threadIdx.x == 0) {
-        s_queued = push_run(args, Run{static_cast<uint32_t>(start) + begin, n, static_cast<uint32_t>(tile), 0u});
+        const bool queued =
+            push_run(args, Run{static_cast<uint32_t>(start) + begin, n, static_cast<uint32_t>(tile), 0u});
+        if constexpr (kMayRefuse) {
+          s_queued = queued;
+        } else if (!queued) {
+          atomicAdd(reinterpret_cast<unsigned long long*>(args.failures), 1ull);  // never, by the bound
+        }
       }
-      __syncthreads();
-      if (!s_queued) sort_in_place<kThreads>(args, start + begin, n, args.keys_in, args.values_in);
+      if constexpr (kMayRefuse) {
+        __syncthreads();
+        if (!s_queued) sort_in_place<kThreads>(args, start + begin, n, args.keys_in, args.values_in);
+      }
     }
     begin += n;
     __syncthreads();  // LDS free for the next part
@@ -214,6 +223,7 @@ __device__ __forceinline__ void sort_list(const TileSortArgs& args, TileSort<kTh
 // invalid and reported as such, and its lists are emptied rather than sorted.
 
 // 8x8 and 16x16 tiles: a workgroup per tile.
+template <bool kMayRefuse>
 __global__ __launch_bounds__(kTileThreads, 6) void tile_sort_kernel(TileSortArgs args) {
   __shared__ TileSort<kTileThreads, kTileCapacity, kTileCapacity> s;
   __shared__ bool s_queued;
@@ -226,7 +236,7 @@ __global__ __launch_bounds__(kTileThreads, 6) void tile_sort_kernel(TileSortArgs
       if (threadIdx.x == 0) args.tile_ends[tile] = static_cast<int32_t>(start);
       continue;
     }
-    sort_list<false>(args, s, s_queued, tile, start, static_cast<uint32_t>(count));
+    sort_list<false, kMayRefuse>(args, s, s_queued, tile, start, static_cast<uint32_t>(count));
   }
 }
 
@@ -281,7 +291,7 @@ __global__ __launch_bounds__(kTileThreads, 6) void small_tile_sort_kernel(TileSo
     const uint32_t left = __builtin_amdgcn_readfirstlane(s_left[q]);
     if (left == 0u) continue;  // uniform
     const int64_t list_start = __builtin_amdgcn_readfirstlane(args.tile_starts[first + q]);
-    sort_list<true>(args, s.of_group, s_queued, first + q, list_start, left);
+    sort_list<true, true>(args, s.of_group, s_queued, first + q, list_start, left);
   }
 }
 
@@ -508,8 +518,8 @@ __global__ __launch_bounds__(kSpreadThreads, 8) void spread_long_kernel(TileSort
 }  // namespace
 
 int launch_tile_sort(const vgr_scene& scene, const vgr_cameras& cameras, const vgr_workspace& ws,
-                     const ScratchLayout& layout, char* scratch, int64_t global_tiles, int tile_size, bool partitioned_in_out,
-                     hipStream_t stream) {
+                     const ScratchLayout& layout, char* scratch, int64_t global_tiles, int tile_size,
+                     bool partitioned_in_out, hipStream_t stream) {
   if (global_tiles <= 0) return 0;
   TileSortArgs args;
   args.keys_in = partitioned_in_out ? ws.keys_out : ws.keys_in;
@@ -525,12 +535,14 @@ int launch_tile_sort(const vgr_scene& scene, const vgr_cameras& cameras, const v
   args.partition = layout.partition;
   // The look-back flags are read no more: their scratch holds the queues, with a place
   // per sort tile (at most 8192 entries) for a part of over 8192 entries, so those always
-  // fit.  The other parts number at most 88 per 8192 entries: 32 crowded ones of over
-  // kSplitLeast, 32 of longer lists (two neighbours hold over 512 entries under small
-  // tiles) and four runs per spread of the part or bin that holds them, of which a 32-bit
-  // depth and a 32-bit tie word allow six.  The default digits leave at least 127 places;
+  // fit.  The other parts number at most 65 per 8192 entries: 32 crowded ones of over
+  // kSplitLeast, nine of longer lists (two neighbours hold over 2048 entries) and four
+  // runs per spread of the part or bin that holds them, of which a 32-bit depth and a
+  // 32-bit tie word allow six.  The default digits leave at least 127 places;
   // explicit digits of four or five bits may leave fewer, and parts beyond them are
-  // sorted where they are found, by the workgroup that found them.
+  // sorted where they are found, by the workgroup that found them.  tile_sort_kernel has
+  // a form of its own for that, since the code alone costs the usual one scalar registers
+  // and 9 % (127M entries 497 -> 542 us); under small tiles it costs nothing.
   static_assert(sizeof(Run) == 16 && kSortThreads * kDefaultSortItems <= kRunCapacity,
                 "a part that is spread takes more entries than a sort tile");
   args.long_runs = reinterpret_cast<Run*>(scratch + layout.sort_flags);
@@ -538,8 +550,10 @@ int launch_tile_sort(const vgr_scene& scene, const vgr_cameras& cameras, const v
   args.runs = args.long_runs + args.long_capacity;
   args.run_capacity = static_cast<uint32_t>(layout.sort_flag_words / 4 - layout.sort_tiles);
   args.state = reinterpret_cast<uint32_t*>(scratch + layout.work_counter) + 4;
-  constexpr int64_t kMaxGrid = 1 << 22;
+  constexpr int64_t kPartsPerSortTile = 65;
+  const bool may_refuse = args.run_capacity < kPartsPerSortTile * layout.sort_tiles;
   const int64_t capacity = ws.intersection_capacity;
+  constexpr int64_t kMaxGrid = 1 << 22;
   if (tile_size <= 4) {
     constexpr int64_t kMost = kMaxGrid * kSmallTiles;  // tiles of a grid
     for (int64_t first = 0; first < global_tiles; first += kMost) {
@@ -548,7 +562,8 @@ int launch_tile_sort(const vgr_scene& scene, const vgr_cameras& cameras, const v
                          dim3(kTileThreads), 0, stream, args, first);
     }
   } else {
-    hipLaunchKernelGGL(tile_sort_kernel, dim3(static_cast<unsigned>(global_tiles < kMaxGrid ? global_tiles : kMaxGrid)),
+    hipLaunchKernelGGL(may_refuse ? tile_sort_kernel<true> : tile_sort_kernel<false>,
+                       dim3(static_cast<unsigned>(global_tiles < kMaxGrid ? global_tiles : kMaxGrid)),
                        dim3(kTileThreads), 0, stream, args);
   }
   // A list holds a Gaussian once for every time its camera is active (active_ids may
