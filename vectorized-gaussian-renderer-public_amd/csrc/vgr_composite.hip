@@ -32,21 +32,24 @@ using namespace dev;
 // forward+backward 9.6 -> 8.0 ms.
 constexpr int kOrderBuckets = 1024;
 constexpr int kOrderThreads = 1024;
-// A tile is long when its list holds more than half of the entries that a CU gets on
-// average: a wave that walks it alone would still run when the other CUs are done.
-// Lists count up to 4,096 entries towards the average, since a tile with more is mostly
-// opaque before its end.  Compositing of 48 room cameras of 160x120 in three submissions
-// of 1,280 tiles, and of one submission of 1,024 tiles of 128x128 views whose lists (23k
-// on average) are opaque early: no tile long 1,829 and 540 us; without the cap 1,699 and
-// 704; cap 4,096 1,186 and 763; cap 2,048 1,127 and 779, but 215 instead of 177 for the
-// 1,200 tiles of a VGA view over 1M Gaussians.
+// A tile is long when it takes more than about half of the list entries that a CU gets on
+// average: a wave that walks it alone would still run when the other CUs are done (alone
+// on its SIMD a wave takes some 390 cycles an entry, a full CU 180).  What a tile takes is
+// its reach where that is known (tile_reach_kernel), else the length of its list, of
+// which up to 4,096 entries count towards the average, since a tile with more is mostly
+// opaque before its end.  Compositing with limits of 0.4, 0.45, 0.5 and 0.6 by reach: 48
+// room cameras of 160x120 in three submissions (of one) 447, 439, 668 and 823 us; by
+// length, which exceeds what a tile takes, 0.45 and 0.5: a VGA view of 1M 195 and 175,
+// of 300k 102 and 108, four 320x240 views in a room of 500k 163 and 189.
 constexpr int32_t kLongCap = 4096;
+constexpr float kLongReachShare = 0.45f / 256.0f;
 constexpr float kLongShare = 0.5f / 256.0f;
 
 __device__ __forceinline__ int32_t list_length(const CameraParams* __restrict__ table,
                                                const int32_t* __restrict__ tile_starts,
                                                const int32_t* __restrict__ tile_ends, int active_count,
-                                               int uniform_tiles, int64_t block) {
+                                               int uniform_tiles, const int32_t* __restrict__ reach, int64_t block) {
+  if (reach != nullptr) return reach[block];
   int active;
   int64_t image_tile;
   if (uniform_tiles > 0) {
@@ -74,6 +77,7 @@ __global__ __launch_bounds__(kOrderThreads) void tile_order_kernel(const CameraP
                                                                    const int32_t* __restrict__ tile_starts,
                                                                    const int32_t* __restrict__ tile_ends,
                                                                    int active_count, int uniform_tiles, int64_t blocks,
+                                                                   const int32_t* __restrict__ reach,
                                                                    int32_t* __restrict__ order,
                                                                    uint32_t* __restrict__ long_tiles) {
   __shared__ uint32_t s_next[kOrderBuckets];
@@ -83,9 +87,9 @@ __global__ __launch_bounds__(kOrderThreads) void tile_order_kernel(const CameraP
   __syncthreads();
   float entries = 0.0f;
   for (int64_t b = threadIdx.x; b < blocks; b += kOrderThreads) {
-    const int32_t length = list_length(table, tile_starts, tile_ends, active_count, uniform_tiles, b);
+    const int32_t length = list_length(table, tile_starts, tile_ends, active_count, uniform_tiles, reach, b);
     atomicAdd(&s_next[order_bucket(length)], 1u);
-    entries += static_cast<float>(length < kLongCap ? length : kLongCap);
+    entries += static_cast<float>(reach != nullptr || length < kLongCap ? length : kLongCap);
   }
   if (long_tiles != nullptr) {  // uniform
 #pragma unroll
@@ -113,12 +117,12 @@ __global__ __launch_bounds__(kOrderThreads) void tile_order_kernel(const CameraP
   if (long_tiles != nullptr) {
     float total = 0.0f;
     for (int w = 0; w < kOrderThreads / kWave; ++w) total += s_wave_entries[w];
-    const int limit = order_bucket(static_cast<int32_t>(total * kLongShare));
+    const int limit = order_bucket(static_cast<int32_t>(total * (reach != nullptr ? kLongReachShare : kLongShare)));
     if (bucket == limit) *long_tiles = prefix + inclusive - count;  // the tiles of the buckets above
   }
   __syncthreads();
   for (int64_t b = threadIdx.x; b < blocks; b += kOrderThreads) {
-    const int k = order_bucket(list_length(table, tile_starts, tile_ends, active_count, uniform_tiles, b));
+    const int k = order_bucket(list_length(table, tile_starts, tile_ends, active_count, uniform_tiles, reach, b));
     order[atomicAdd(&s_next[k], 1u)] = static_cast<int32_t>(b);
   }
 }
@@ -374,6 +378,112 @@ __device__ __forceinline__ void composite_tile(const CompositeArgsFor<kDegree>& 
   }
 }
 
+// ---- how far tiles are composited --------------------------------------------------
+//
+// A tile's work is the part of its list up to where its last pixel turns opaque, which
+// the length of the list says little about: tiles of a room that look out of it are
+// read to the end, while 128x128 views of an open million are opaque after 5,000 entries
+// of lists of up to 107,000.  A wave per tile samples the front of the list and adds up,
+// at 8x8 points of the tile, the optical thickness that every sample spreads there (its
+// integral over the plane, as a Gaussian widened so that small splats count for their
+// neighbourhood); the point that takes longest to pass the depth at which pixels end
+// sets the tile's.  Only the schedule depends on it.  Against the entries that are read,
+// on six workloads of 1,024 to 1,280 tiles, three of them in rooms or with lists read to
+// the end: the sum over the tiles is 1.02 to 1.52 of it, 99 % of the tiles of each at 0.89
+// of theirs or more.  Fewer points miss tiles that are open in one corner, which then end
+// the grid alone; twice the samples come closer and cost as much more as they gain.
+constexpr int kReachLeast = 512;         // shorter lists are taken as they are
+constexpr int kReachSpan = 8192;         // entries that the samples are spread over
+constexpr int kReachSamples = 1;         // of a lane
+constexpr float kReachDepth = 1.1f * 9.21f;  // of a transmittance of 1e-4, with an allowance
+constexpr float kReachWiden = 12.0f;     // variance added to a splat's
+// A sample stands for up to 128 entries; where one near splat does so, it does not make
+// the tile opaque alone.
+constexpr float kReachSampleDepth = 2.0f;
+
+template <bool kSlots>
+__global__ __launch_bounds__(256) void tile_reach_kernel(CompositeArgs args, int64_t blocks,
+                                                         int32_t* __restrict__ reach) {
+  constexpr int kCount = kWave * kReachSamples;
+  __shared__ f32x4 s_form[4][kCount];   // mean, xx and xy coefficients of the exponent
+  __shared__ float s_peak[4][kCount][2];  // yy coefficient, thickness at the mean
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int64_t block = static_cast<int64_t>(blockIdx.x) * 4 + wave;
+  int32_t length = 0;
+  if (block < blocks) {
+    length = list_length(args.table, args.tile_starts, args.tile_ends, args.active_count, args.uniform_tiles, nullptr,
+                         block);
+  }
+  const int32_t span = length < kReachSpan ? length : kReachSpan;
+  const float weight = static_cast<float>(span) / kCount;  // entries a sample stands for
+  int tile_x = 0, tile_y = 0, width = 0, height = 0;
+  if (length > kReachLeast) {
+    const int active = args.uniform_tiles > 0 ? static_cast<int>(block / args.uniform_tiles)
+                                              : find_active_camera(args.table, args.active_count, block);
+    const CameraParams& cam = args.table[active];
+    const int64_t image_tile = block - (args.uniform_tiles > 0 ? static_cast<int64_t>(active) * args.uniform_tiles
+                                                               : cam.active_tile_begin);
+    tile_x = static_cast<int>(image_tile % cam.tiles_x) * 16;
+    tile_y = static_cast<int>(image_tile / cam.tiles_x) * 16;
+    width = cam.width;
+    height = cam.height;
+    const int64_t start = args.tile_starts[cam.tile_base + static_cast<uint32_t>(image_tile)];
+    int32_t records[kReachSamples];
+#pragma unroll
+    for (int k = 0; k < kReachSamples; ++k) {
+      // The middle entry of those it stands for: the first of a list are the largest.
+      records[k] = args.sorted_values[start + (2 * (k * kWave + lane) + 1) * span / (2 * kCount)];
+    }
+#pragma unroll
+    for (int k = 0; k < kReachSamples; ++k) {
+      int32_t record = records[k];
+      if (kSlots) record = record >= 0 ? args.slot_records[record] : -1;
+      f32x4 a = {}, b = {};
+      if (record >= 0 && record < args.visible_capacity) {  // else a corrupted list
+        const f32x4* src = reinterpret_cast<const f32x4*>(args.records + record);
+        a = src[0];  // mean_x, mean_y, conic_0, conic_1
+        b = src[1];  // conic_2, opacity, depth, red
+      }
+      const float inverse = __builtin_amdgcn_rcpf(fmaxf(a.z * b.x - a.w * a.w, 1.0e-12f));
+      const float xx = b.x * inverse + kReachWiden, yy = a.z * inverse + kReachWiden, xy = -a.w * inverse;
+      const float wide = __builtin_amdgcn_rcpf(xx * yy - xy * xy);
+      const float scale = -0.7213475f * wide;  // -1/2 log2(e)
+      s_form[wave][k * kWave + lane] = f32x4{a.x, a.y, scale * yy, -2.0f * scale * xy};
+      s_peak[wave][k * kWave + lane][0] = scale * xx;
+      // The integral of -ln(1 - alpha) over the plane is 2 pi / sqrt(det) times the
+      // dilogarithm of the opacity, here its first terms.
+      const float o = b.y;
+      s_peak[wave][k * kWave + lane][1] = weight * o * (1.0f + o * (0.25f + o * (0.1111f + o * 0.0625f))) *
+                                          __builtin_amdgcn_sqrtf(inverse * wide);
+    }
+  }
+  __syncthreads();
+  if (block >= blocks) return;
+  if (length <= kReachLeast) {
+    if (lane == 0) reach[block] = length;
+    return;
+  }
+  const int x = tile_x + (lane & 7) * 2, y = tile_y + (lane >> 3) * 2;
+  const float px = static_cast<float>(x + 1), py = static_cast<float>(y + 1);
+  float thickness = 0.0f;
+  int samples = 0;  // before the point's depth is passed
+#pragma unroll 4
+  for (int i = 0; i < kCount; ++i) {
+    const f32x4 form = s_form[wave][i];
+    const float dx = px - form.x, dy = py - form.y;
+    const float power = dx * (form.z * dx + form.w * dy) + s_peak[wave][i][0] * dy * dy;
+    thickness += fminf(kReachSampleDepth, s_peak[wave][i][1] * __builtin_amdgcn_exp2f(power));
+    samples += thickness < kReachDepth ? 1 : 0;
+  }
+  float entries = weight * (samples < kCount ? static_cast<float>(samples + 1)
+                                             : kCount * kReachDepth / fmaxf(thickness, 1.0e-6f));
+  if (x >= width || y >= height) entries = 0.0f;  // no pixel to finish
+#pragma unroll
+  for (int offset = 1; offset < kWave; offset <<= 1) entries = fmaxf(entries, __shfl_xor(entries, offset, kWave));
+  if (lane == 0) reach[block] = entries < static_cast<float>(length) ? static_cast<int32_t>(entries) : length;
+}
+
 // ---- few long lists: a workgroup per 8x8 block ---------------------------------------
 //
 // Where a handful of tiles outlast the rest of the grid (a small image; tiles that
@@ -514,7 +624,7 @@ __device__ __forceinline__ void composite_block(const CompositeArgsFor<kDegree>&
     int64_t batch_start = range_start;
     int parity = 0;
     while (batch_start < range_end) {  // uniform
-      // Stage batches until the kept entries fill half of the rows.
+      // Stage batches while another one fits the rows whole.
       int kept = 0;
       while (batch_start < range_end && kept <= kBlockRows - kBlockBatch) {
         const bool listed = batch_start + thread < range_end;
@@ -1037,10 +1147,19 @@ __global__ __launch_bounds__(kBlockBatch, kMixedWavesPerSimd) void composite_mix
 
 // Grids up to this many tiles: at five workgroups a CU all of them are resident, so the
 // lower occupancy of the mixed kernel (five waves a SIMD for eight) costs little.  1,200
-// tiles: VGA views of 100k, 300k and 1M Gaussians 51 -> 43, 134 -> 109 and 168 -> 177 us,
-// four 320x240 views of 500k 294 -> 313, of a room 154 -> 83.  At 2,400 and 3,600 tiles of
-// open scenes the occupancy alone costs 36 and 41 %.
+// tiles: VGA views of 100k and 300k Gaussians 55 -> 42 and 143 -> 108 us.  At 2,400 and
+// 3,600 tiles of open scenes the occupancy alone costs 36 and 41 %.
 constexpr int64_t kMixedCompositeTiles = 1280;
+// Where whole and long tiles compete for the CUs (three workgroups and more a CU) and the
+// lists may be long (the capacity holds this many entries a tile: lists of 2,000 on
+// average with the usual headroom), the reach decides instead of the length, for 10 to
+// 12 us.  No tile long / by length / by reach, with
+// those: 16 views of 128x128 over an open 1M 574 / 770 / 563 us and 300k 512 / 564 / 501,
+// two 480x320 views of 1M 223 / 258 / 224, four 320x240 views of 500k 306 / 313 / 299, 16
+// room cameras of 160x120 837 / 446 / 449.  600 tiles (two 320x240 views of 500k) 273 /
+// 237 / 266; a VGA view of 1M (lists of 1,661) 180 / 175 / 184.
+constexpr int64_t kReachTiles = 768;
+constexpr int64_t kReachLists = 3072;
 // 8x8 tiles are a block each; up to this many all take the block kernel.  2,400 tiles
 // 166 -> 81 us, 4,800 tiles 124 -> 128 (open scene) and 176 -> 115 (room); 14,400 tiles
 // would go 182 -> 253.
@@ -1166,10 +1285,10 @@ void launch_batch(int batch, bool full, const CompositeArgs& args, int64_t block
 
 int launch_tile_order(const CameraParams* table, const int32_t* tile_starts, const int32_t* tile_ends,
                       int active_count, int uniform_tiles, int64_t blocks, int32_t* order, hipStream_t stream,
-                      uint32_t* long_tiles) {
+                      uint32_t* long_tiles, const int32_t* reach) {
   if (blocks <= 0 || active_count <= 0) return 0;
   hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(kOrderThreads), 0, stream, table, tile_starts, tile_ends,
-                     active_count, uniform_tiles, blocks, order, long_tiles);
+                     active_count, uniform_tiles, blocks, reach, order, long_tiles);
   const hipError_t error = hipGetLastError();
   if (error != hipSuccess) {
     set_error("tile order launch failed: %s", hipGetErrorString(error));
@@ -1277,8 +1396,22 @@ int launch_composite(const vgr_scene& scene, const vgr_cameras& cameras, const v
   args.tile_order = nullptr;
   if (blocks <= kOrderedCompositeBlocks) {
     int32_t* order = reinterpret_cast<int32_t*>(const_cast<char*>(scratch) + layout.tile_order);
+    int32_t* reach = nullptr;
+    if (!front && options.tile_size == 16 && options.statistics == nullptr && blocks > kReachTiles &&
+        blocks <= kMixedCompositeTiles && ws.intersection_capacity >= blocks * kReachLists &&
+        layout.sort_flag_words >= blocks) {
+      // The sort's flags are read no more.
+      reach = reinterpret_cast<int32_t*>(const_cast<char*>(scratch) + layout.sort_flags);
+      const dim3 grid(static_cast<unsigned>((blocks + 3) / 4));
+      if (args.final_transmittance != nullptr) {
+        hipLaunchKernelGGL(tile_reach_kernel<true>, grid, dim3(256), 0, stream, args, blocks, reach);
+      } else {
+        hipLaunchKernelGGL(tile_reach_kernel<false>, grid, dim3(256), 0, stream, args, blocks, reach);
+      }
+    }
     const int order_status = launch_tile_order(args.table, args.tile_starts, args.tile_ends, args.active_count,
-                                               args.uniform_tiles, blocks, order, stream, args.work_counter + 1);
+                                               args.uniform_tiles, blocks, order, stream, args.work_counter + 1,
+                                               reach);
     if (order_status != 0) return order_status;
     args.tile_order = order;
     args.long_tiles = args.work_counter + 1;

@@ -151,7 +151,7 @@ int launch_covariance_backward(const float* scales, const float* rotations, cons
 // `long_tiles` how many of them hold more than a fair share of the list entries.
 int launch_tile_order(const CameraParams* table, const int32_t* tile_starts, const int32_t* tile_ends,
                       int active_count, int uniform_tiles, int64_t blocks, int32_t* order, hipStream_t stream,
-                      uint32_t* long_tiles = nullptr);
+                      uint32_t* long_tiles = nullptr, const int32_t* reach = nullptr);
 // Tile-front ordering (vgr_front.hip): bucketed emission, front sort, fallback full sort.
 int launch_front_projection(const vgr_scene& scene, const vgr_cameras& cameras, const vgr_options& options,
                             const vgr_workspace& ws, const ScratchLayout& layout, char* scratch, int64_t global_tiles,
