@@ -543,13 +543,15 @@ int launch_sort(const vgr_workspace& ws, const ScratchLayout& layout, char* scra
                      digit_bits, passes, tiles, layout.sort_tile, histogram, tickets, flags, global_tiles, ws.tile_starts,
                      ws.tile_ends, reinterpret_cast<uint32_t*>(scratch + layout.work_counter) + 4);
   const int items = layout.sort_tile / kSortThreads;
-  // Every workgroup ends with an atomic per digit value on the same counters, and 512 of
-  // them (eight waves a CU) are too few to read at the rate of the memory: 87M keys
-  // 500 / 275 / 188 us with 512 / 1,024 / 2,048 workgroups, 9M 59 / 46 / 55; 127M of 64
-  // VGA views 828 with 512 and 296 with this rule.
+  // Every workgroup ends with an atomic per digit value and pass on the same counters (a
+  // thousand workgroups: 40 us), so it takes 16k keys at least where there are many; 512
+  // workgroups, eight waves a CU, are too few to read 87M keys at the rate of the memory.
+  // 4.4M keys 30 / 46 us with 512 / 1,024, 9M 59 / 46 / 55 with 512 / 1,024 / 2,048, 87M
+  // 500 / 275 / 188; 127M of 64 VGA views 828 with 512 and 296 with 2,048.
+  constexpr int64_t kFew = 512, kMany = 2048;
   int64_t histogram_blocks = (capacity + kBlockThreads * 16 - 1) / (kBlockThreads * 16);
-  if (histogram_blocks > 1024) {
-    histogram_blocks = histogram_blocks / 2 < 1024 ? 1024 : (histogram_blocks / 2 > 2048 ? 2048 : histogram_blocks / 2);
+  if (histogram_blocks > kFew) {
+    histogram_blocks = histogram_blocks / 4 < kFew ? kFew : (histogram_blocks / 4 > kMany ? kMany : histogram_blocks / 4);
   }
   histogram_blocks = histogram_blocks < 1 ? 1 : histogram_blocks;
   hipLaunchKernelGGL(sort_histogram_kernel, dim3(static_cast<unsigned>(histogram_blocks)), dim3(kBlockThreads), 0,
