@@ -37,13 +37,24 @@ constexpr int kOrderThreads = 1024;
 // on its SIMD a wave takes some 390 cycles an entry, a full CU 180).  What a tile takes is
 // its reach where that is known (tile_reach_kernel), else the length of its list, of
 // which up to 4,096 entries count towards the average, since a tile with more is mostly
-// opaque before its end.  Compositing with limits of 0.4, 0.45, 0.5 and 0.6 by reach: 48
-// room cameras of 160x120 in three submissions (of one) 447, 439, 668 and 823 us; by
-// length, which exceeds what a tile takes, 0.45 and 0.5: a VGA view of 1M 195 and 175,
-// of 300k 102 and 108, four 320x240 views in a room of 500k 163 and 189.
+// opaque before its end.  By length, 0.45 and 0.5: a VGA view of 1M Gaussians 195 and 175
+// us, of 300k 102 and 108, four 320x240 views in a room of 500k 163 and 189; by reach,
+// which overestimates the sum more than the longest, 0.40 and 0.43: 16 views of 128x128
+// over 300k 586 and 490, 48 room cameras of 160x120 1,203 and 1,278.
 constexpr int32_t kLongCap = 4096;
-constexpr float kLongReachShare = 0.45f / 256.0f;
+constexpr float kLongReachShare = 0.43f / 256.0f;
 constexpr float kLongShare = 0.5f / 256.0f;
+// Where whole and long tiles compete for the CUs (three workgroups and more a CU) and the
+// lists are long (5,000 entries on average, known on the device only), the reach decides
+// instead of the length, for 11 to 16 us.  No tile long / by length / by reach, with
+// those: 16 views of 128x128 over an open 1M 583 / 774 / 537 us and 300k 508 / 560 / 500,
+// 13 of 700k 600 / 595 / 526, ten 160x120 views of 1M 461 / 548 / 461, 16 room cameras of
+// 128x128 over 5M 517 / 345 / 318; but twelve of 160x120 over 3M 289 / 280 / 340.  With
+// shorter lists it gains little and may lose: two 480x320 views of 1M (lists of 2,781)
+// 222 / 254 / 225, four 320x240 views of 500k 307 / 311 / 304, 48 room cameras of 160x120
+// in three submissions 1,906 / 1,182 / 1,304.
+constexpr int64_t kReachTiles = 768;
+constexpr int64_t kReachLists = 5000;
 
 __device__ __forceinline__ int32_t list_length(const CameraParams* __restrict__ table,
                                                const int32_t* __restrict__ tile_starts,
@@ -78,8 +89,10 @@ __global__ __launch_bounds__(kOrderThreads) void tile_order_kernel(const CameraP
                                                                    const int32_t* __restrict__ tile_ends,
                                                                    int active_count, int uniform_tiles, int64_t blocks,
                                                                    const int32_t* __restrict__ reach,
+                                                                   const int64_t* __restrict__ intersections,
                                                                    int32_t* __restrict__ order,
                                                                    uint32_t* __restrict__ long_tiles) {
+  if (reach != nullptr && *intersections < blocks * kReachLists) reach = nullptr;  // uniform: not written either
   __shared__ uint32_t s_next[kOrderBuckets];
   __shared__ uint32_t s_wave_totals[kOrderThreads / kWave];
   __shared__ float s_wave_entries[kOrderThreads / kWave];
@@ -383,102 +396,106 @@ __device__ __forceinline__ void composite_tile(const CompositeArgsFor<kDegree>& 
 // A tile's work is the part of its list up to where its last pixel turns opaque, which
 // the length of the list says little about: tiles of a room that look out of it are
 // read to the end, while 128x128 views of an open million are opaque after 5,000 entries
-// of lists of up to 107,000.  A wave per tile samples the front of the list and adds up,
+// of lists of up to 107,000.  A workgroup per tile samples the front of the list and adds up,
 // at 8x8 points of the tile, the optical thickness that every sample spreads there (its
 // integral over the plane, as a Gaussian widened so that small splats count for their
 // neighbourhood); the point that takes longest to pass the depth at which pixels end
-// sets the tile's.  Only the schedule depends on it.  Against the entries that are read,
-// on six workloads of 1,024 to 1,280 tiles, three of them in rooms or with lists read to
-// the end: the sum over the tiles is 1.02 to 1.52 of it, 99 % of the tiles of each at 0.89
-// of theirs or more.  Fewer points miss tiles that are open in one corner, which then end
-// the grid alone; twice the samples come closer and cost as much more as they gain.
+// sets the tile's.  Only the schedule depends on it.  A model of it with the crossing
+// sample instead of the interpolated part, against the entries that are read, on four
+// workloads of 1,024 and 1,280 tiles: the sum over the tiles is 1.06 to 1.39 of it, 99 %
+// of the tiles of each at 0.92 of theirs or more.  Fewer points miss tiles that are open
+// in one corner, which then end the grid alone.
 constexpr int kReachLeast = 512;         // shorter lists are taken as they are
 constexpr int kReachSpan = 8192;         // entries that the samples are spread over
-constexpr int kReachSamples = 1;         // of a lane
-constexpr float kReachDepth = 1.1f * 9.21f;  // of a transmittance of 1e-4, with an allowance
-constexpr float kReachWiden = 12.0f;     // variance added to a splat's
-// A sample stands for up to 128 entries; where one near splat does so, it does not make
+constexpr int kReachWaves = 4;           // of a tile
+constexpr int kReachParts = 4;           // of a wave's samples, whose sums are kept
+constexpr int kReachSamples = 8;         // of a part
+constexpr float kReachDepth = 1.25f * 9.21f;  // of a transmittance of 1e-4, with an allowance
+constexpr float kReachWiden = 8.0f;      // variance added to a splat's
+// A sample stands for up to 64 entries; where one near splat does so, it does not make
 // the tile opaque alone.
 constexpr float kReachSampleDepth = 2.0f;
 
 template <bool kSlots>
-__global__ __launch_bounds__(256) void tile_reach_kernel(CompositeArgs args, int64_t blocks,
-                                                         int32_t* __restrict__ reach) {
-  constexpr int kCount = kWave * kReachSamples;
-  __shared__ f32x4 s_form[4][kCount];   // mean, xx and xy coefficients of the exponent
-  __shared__ float s_peak[4][kCount][2];  // yy coefficient, thickness at the mean
+__global__ __launch_bounds__(kReachWaves* kWave) void tile_reach_kernel(CompositeArgs args,
+                                                                        const int64_t* __restrict__ intersections,
+                                                                        int32_t* __restrict__ reach) {
+  if (*intersections < static_cast<int64_t>(gridDim.x) * kReachLists) return;
+  constexpr int kOwn = kReachParts * kReachSamples;  // samples of a wave
+  constexpr int kCount = kReachWaves * kOwn;
+  __shared__ f32x4 s_form[kCount];      // mean, xx and xy coefficients of the exponent
+  __shared__ float2 s_peak[kCount];      // yy coefficient, thickness at the mean
+  __shared__ float s_sums[kReachWaves * kReachParts][kWave];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int64_t block = static_cast<int64_t>(blockIdx.x) * 4 + wave;
-  int32_t length = 0;
-  if (block < blocks) {
-    length = list_length(args.table, args.tile_starts, args.tile_ends, args.active_count, args.uniform_tiles, nullptr,
-                         block);
-  }
-  const int32_t span = length < kReachSpan ? length : kReachSpan;
-  const float weight = static_cast<float>(span) / kCount;  // entries a sample stands for
-  int tile_x = 0, tile_y = 0, width = 0, height = 0;
-  if (length > kReachLeast) {
-    const int active = args.uniform_tiles > 0 ? static_cast<int>(block / args.uniform_tiles)
-                                              : find_active_camera(args.table, args.active_count, block);
-    const CameraParams& cam = args.table[active];
-    const int64_t image_tile = block - (args.uniform_tiles > 0 ? static_cast<int64_t>(active) * args.uniform_tiles
-                                                               : cam.active_tile_begin);
-    tile_x = static_cast<int>(image_tile % cam.tiles_x) * 16;
-    tile_y = static_cast<int>(image_tile / cam.tiles_x) * 16;
-    width = cam.width;
-    height = cam.height;
-    const int64_t start = args.tile_starts[cam.tile_base + static_cast<uint32_t>(image_tile)];
-    int32_t records[kReachSamples];
-#pragma unroll
-    for (int k = 0; k < kReachSamples; ++k) {
-      // The middle entry of those it stands for: the first of a list are the largest.
-      records[k] = args.sorted_values[start + (2 * (k * kWave + lane) + 1) * span / (2 * kCount)];
-    }
-#pragma unroll
-    for (int k = 0; k < kReachSamples; ++k) {
-      int32_t record = records[k];
-      if (kSlots) record = record >= 0 ? args.slot_records[record] : -1;
-      f32x4 a = {}, b = {};
-      if (record >= 0 && record < args.visible_capacity) {  // else a corrupted list
-        const f32x4* src = reinterpret_cast<const f32x4*>(args.records + record);
-        a = src[0];  // mean_x, mean_y, conic_0, conic_1
-        b = src[1];  // conic_2, opacity, depth, red
-      }
-      const float inverse = __builtin_amdgcn_rcpf(fmaxf(a.z * b.x - a.w * a.w, 1.0e-12f));
-      const float xx = b.x * inverse + kReachWiden, yy = a.z * inverse + kReachWiden, xy = -a.w * inverse;
-      const float wide = __builtin_amdgcn_rcpf(xx * yy - xy * xy);
-      const float scale = -0.7213475f * wide;  // -1/2 log2(e)
-      s_form[wave][k * kWave + lane] = f32x4{a.x, a.y, scale * yy, -2.0f * scale * xy};
-      s_peak[wave][k * kWave + lane][0] = scale * xx;
-      // The integral of -ln(1 - alpha) over the plane is 2 pi / sqrt(det) times the
-      // dilogarithm of the opacity, here its first terms.
-      const float o = b.y;
-      s_peak[wave][k * kWave + lane][1] = weight * o * (1.0f + o * (0.25f + o * (0.1111f + o * 0.0625f))) *
-                                          __builtin_amdgcn_sqrtf(inverse * wide);
-    }
-  }
-  __syncthreads();
-  if (block >= blocks) return;
+  const int64_t block = blockIdx.x;
+  const int32_t length = list_length(args.table, args.tile_starts, args.tile_ends, args.active_count,
+                                     args.uniform_tiles, nullptr, block);
   if (length <= kReachLeast) {
-    if (lane == 0) reach[block] = length;
+    if (threadIdx.x == 0) reach[block] = length;
     return;
   }
-  const int x = tile_x + (lane & 7) * 2, y = tile_y + (lane >> 3) * 2;
-  const float px = static_cast<float>(x + 1), py = static_cast<float>(y + 1);
-  float thickness = 0.0f;
-  int samples = 0;  // before the point's depth is passed
-#pragma unroll 4
-  for (int i = 0; i < kCount; ++i) {
-    const f32x4 form = s_form[wave][i];
-    const float dx = px - form.x, dy = py - form.y;
-    const float power = dx * (form.z * dx + form.w * dy) + s_peak[wave][i][0] * dy * dy;
-    thickness += fminf(kReachSampleDepth, s_peak[wave][i][1] * __builtin_amdgcn_exp2f(power));
-    samples += thickness < kReachDepth ? 1 : 0;
+  const int active = args.uniform_tiles > 0 ? static_cast<int>(block / args.uniform_tiles)
+                                            : find_active_camera(args.table, args.active_count, block);
+  const CameraParams& cam = args.table[active];
+  const int image_tile = static_cast<int>(block - (args.uniform_tiles > 0
+                                                       ? static_cast<int64_t>(active) * args.uniform_tiles
+                                                       : cam.active_tile_begin));
+  const int x = image_tile % cam.tiles_x * 16 + (lane & 7) * 2, y = image_tile / cam.tiles_x * 16 + (lane >> 3) * 2;
+  const int32_t span = length < kReachSpan ? length : kReachSpan;
+  const float weight = static_cast<float>(span) / kCount;  // entries a sample stands for
+  if (lane < kOwn) {
+    const int i = wave * kOwn + lane;
+    // The middle entry of those it stands for: the first of a list are the largest.
+    int32_t record = args.sorted_values[args.tile_starts[cam.tile_base + static_cast<uint32_t>(image_tile)] +
+                                        static_cast<int64_t>(2 * i + 1) * span / (2 * kCount)];
+    if (kSlots) record = record >= 0 ? args.slot_records[record] : -1;
+    f32x4 a = {}, b = {};
+    if (record >= 0 && record < args.visible_capacity) {  // else a corrupted list
+      const f32x4* src = reinterpret_cast<const f32x4*>(args.records + record);
+      a = src[0];  // mean_x, mean_y, conic_0, conic_1
+      b = src[1];  // conic_2, opacity, depth, red
+    }
+    const float inverse = __builtin_amdgcn_rcpf(fmaxf(a.z * b.x - a.w * a.w, 1.0e-12f));
+    const float xx = b.x * inverse + kReachWiden, yy = a.z * inverse + kReachWiden, xy = -a.w * inverse;
+    const float wide = __builtin_amdgcn_rcpf(xx * yy - xy * xy);
+    const float scale = -0.7213475f * wide;  // -1/2 log2(e)
+    s_form[i] = f32x4{a.x, a.y, scale * yy, -2.0f * scale * xy};
+    // The integral of -ln(1 - alpha) over the plane is 2 pi / sqrt(det) times the
+    // dilogarithm of the opacity, here its first terms.
+    const float o = b.y;
+    s_peak[i] = float2{scale * xx, weight * o * (1.0f + o * (0.25f + o * (0.1111f + o * 0.0625f))) *
+                                      __builtin_amdgcn_sqrtf(inverse * wide)};
   }
-  float entries = weight * (samples < kCount ? static_cast<float>(samples + 1)
-                                             : kCount * kReachDepth / fmaxf(thickness, 1.0e-6f));
-  if (x >= width || y >= height) entries = 0.0f;  // no pixel to finish
+  __syncthreads();
+  const float px = static_cast<float>(x + 1), py = static_cast<float>(y + 1);
+#pragma unroll
+  for (int part = 0; part < kReachParts; ++part) {
+    float thickness = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kReachSamples; ++k) {
+      const int i = (wave * kReachParts + part) * kReachSamples + k;
+      const f32x4 form = s_form[i];
+      const float2 peak = s_peak[i];
+      const float dx = px - form.x, dy = py - form.y;
+      const float power = dx * (form.z * dx + form.w * dy) + peak.x * dy * dy;
+      thickness += fminf(kReachSampleDepth, peak.y * __builtin_amdgcn_exp2f(power));
+    }
+    s_sums[wave * kReachParts + part][lane] = thickness;
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  // Parts up to the one in which the point's depth is passed, and the share of that one.
+  float total = 0.0f, parts = 0.0f;
+#pragma unroll
+  for (int p = 0; p < kReachWaves * kReachParts; ++p) {
+    const float own = s_sums[p][lane];
+    parts += fminf(1.0f, fmaxf(0.0f, kReachDepth - total) / fmaxf(own, 1.0e-6f));
+    total += own;
+  }
+  constexpr float kAll = kReachWaves * kReachParts;
+  float entries = weight * kReachSamples * (total < kReachDepth ? kAll * kReachDepth / fmaxf(total, 1.0e-6f) : parts);
+  if (x >= cam.width || y >= cam.height) entries = 0.0f;  // no pixel to finish
 #pragma unroll
   for (int offset = 1; offset < kWave; offset <<= 1) entries = fmaxf(entries, __shfl_xor(entries, offset, kWave));
   if (lane == 0) reach[block] = entries < static_cast<float>(length) ? static_cast<int32_t>(entries) : length;
@@ -708,8 +725,7 @@ __global__ __launch_bounds__(kBlockBatch) void composite_block_persistent_kernel
     __syncthreads();
     if (item >= total) break;
     composite_block<kTileSize, kFull, kCheckpoint, kDegree>(
-        args, args.tile_order != nullptr ? args.tile_order[item / kBlocks] : item / kBlocks,
-        static_cast<int>(item % kBlocks), s);
+        args, args.tile_order[item / kBlocks], static_cast<int>(item % kBlocks), s);
     __syncthreads();
   }
 }
@@ -1100,7 +1116,7 @@ composite_persistent_kernel(CompositeArgsFor<kDegree> args) {
     __syncthreads();
     if (item >= total) break;
     composite_tile<kTileSize, kBatch, kFull, kCount, kCheckpoint, kDegree>(
-        args, args.tile_order != nullptr ? args.tile_order[item] : item, s);
+        args, args.tile_order[item], s);
   }
 }
 
@@ -1150,16 +1166,6 @@ __global__ __launch_bounds__(kBlockBatch, kMixedWavesPerSimd) void composite_mix
 // tiles: VGA views of 100k and 300k Gaussians 55 -> 42 and 143 -> 108 us.  At 2,400 and
 // 3,600 tiles of open scenes the occupancy alone costs 36 and 41 %.
 constexpr int64_t kMixedCompositeTiles = 1280;
-// Where whole and long tiles compete for the CUs (three workgroups and more a CU) and the
-// lists may be long (the capacity holds this many entries a tile: lists of 2,000 on
-// average with the usual headroom), the reach decides instead of the length, for 10 to
-// 12 us.  No tile long / by length / by reach, with
-// those: 16 views of 128x128 over an open 1M 574 / 770 / 563 us and 300k 512 / 564 / 501,
-// two 480x320 views of 1M 223 / 258 / 224, four 320x240 views of 500k 306 / 313 / 299, 16
-// room cameras of 160x120 837 / 446 / 449.  600 tiles (two 320x240 views of 500k) 273 /
-// 237 / 266; a VGA view of 1M (lists of 1,661) 180 / 175 / 184.
-constexpr int64_t kReachTiles = 768;
-constexpr int64_t kReachLists = 3072;
 // 8x8 tiles are a block each; up to this many all take the block kernel.  2,400 tiles
 // 166 -> 81 us, 4,800 tiles 124 -> 128 (open scene) and 176 -> 115 (room); 14,400 tiles
 // would go 182 -> 253.
@@ -1285,10 +1291,10 @@ void launch_batch(int batch, bool full, const CompositeArgs& args, int64_t block
 
 int launch_tile_order(const CameraParams* table, const int32_t* tile_starts, const int32_t* tile_ends,
                       int active_count, int uniform_tiles, int64_t blocks, int32_t* order, hipStream_t stream,
-                      uint32_t* long_tiles, const int32_t* reach) {
+                      uint32_t* long_tiles, const int32_t* reach, const int64_t* intersections) {
   if (blocks <= 0 || active_count <= 0) return 0;
   hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(kOrderThreads), 0, stream, table, tile_starts, tile_ends,
-                     active_count, uniform_tiles, blocks, reach, order, long_tiles);
+                     active_count, uniform_tiles, blocks, reach, intersections, order, long_tiles);
   const hipError_t error = hipGetLastError();
   if (error != hipSuccess) {
     set_error("tile order launch failed: %s", hipGetErrorString(error));
@@ -1402,16 +1408,13 @@ int launch_composite(const vgr_scene& scene, const vgr_cameras& cameras, const v
         layout.sort_flag_words >= blocks) {
       // The sort's flags are read no more.
       reach = reinterpret_cast<int32_t*>(const_cast<char*>(scratch) + layout.sort_flags);
-      const dim3 grid(static_cast<unsigned>((blocks + 3) / 4));
-      if (args.final_transmittance != nullptr) {
-        hipLaunchKernelGGL(tile_reach_kernel<true>, grid, dim3(256), 0, stream, args, blocks, reach);
-      } else {
-        hipLaunchKernelGGL(tile_reach_kernel<false>, grid, dim3(256), 0, stream, args, blocks, reach);
-      }
+      hipLaunchKernelGGL(args.final_transmittance != nullptr ? tile_reach_kernel<true> : tile_reach_kernel<false>,
+                         dim3(static_cast<unsigned>(blocks)), dim3(kReachWaves * kWave), 0, stream, args,
+                         ws.counters + VGR_COUNTER_INTERSECTIONS, reach);
     }
     const int order_status = launch_tile_order(args.table, args.tile_starts, args.tile_ends, args.active_count,
                                                args.uniform_tiles, blocks, order, stream, args.work_counter + 1,
-                                               reach);
+                                               reach, ws.counters + VGR_COUNTER_INTERSECTIONS);
     if (order_status != 0) return order_status;
     args.tile_order = order;
     args.long_tiles = args.work_counter + 1;

@@ -65,8 +65,8 @@ struct ScratchLayout {
   size_t item_masks;       // uint64[projection_blocks]
   size_t item_totals;      // int64[2]: kept item count
   size_t work_counter;     // uint32[8]: [1] long tiles, [4..7] queues of the tile sort
-  size_t tile_order;       // int32[global_tiles]: long-list queue of the tile sort, then the compositing order
-                           // (longest lists first), which the backward reuses
+  size_t tile_order;       // int32[global_tiles]: compositing order (longest tiles first), which the backward
+                           // reuses
   // Tile-front ordering only (zero-sized otherwise).
   size_t front_counts;       // int64[2 * global_tiles]: (entries, 0) per tile
   size_t front_bases;        // int64[2 * (global_tiles + scan partials)]: exclusive bases per tile
@@ -127,7 +127,7 @@ int launch_projection(const vgr_scene& scene, const vgr_cameras& cameras,
                       const vgr_options& options, const vgr_workspace& ws,
                       const ScratchLayout& layout, char* scratch,
                       hipStream_t stream);
-// Partition by tile (also clears the tile ranges and the long-list queue), ranges of
+// Partition by tile (also clears the tile ranges and the tile sort's queues), ranges of
 // the partitioned tiles, then the depth order inside every tile; the depth order
 // leaves the result in the other buffer pair than the partition.
 int launch_sort(const vgr_workspace& ws, const ScratchLayout& layout, char* scratch, int64_t global_tiles,
@@ -147,11 +147,13 @@ int launch_backward(const vgr_scene& scene, const vgr_cameras& cameras, const vg
 int launch_covariance_backward(const float* scales, const float* rotations, const float* grad_covariances,
                                int64_t count, float* grad_scales, float* grad_rotations, hipStream_t stream);
 // Writes the (camera, tile) compositing blocks [0, blocks) into `order` sorted by
-// descending tile-list length, so the longest tiles are launched first, and into
-// `long_tiles` how many of them hold more than a fair share of the list entries.
+// descending tile-list length (by `reach` where given and the lists are long), so the longest tiles are
+// launched first, and into `long_tiles` how many of them take more than a fair share of
+// the list entries.
 int launch_tile_order(const CameraParams* table, const int32_t* tile_starts, const int32_t* tile_ends,
                       int active_count, int uniform_tiles, int64_t blocks, int32_t* order, hipStream_t stream,
-                      uint32_t* long_tiles = nullptr, const int32_t* reach = nullptr);
+                      uint32_t* long_tiles = nullptr, const int32_t* reach = nullptr,
+                      const int64_t* intersections = nullptr);
 // Tile-front ordering (vgr_front.hip): bucketed emission, front sort, fallback full sort.
 int launch_front_projection(const vgr_scene& scene, const vgr_cameras& cameras, const vgr_options& options,
                             const vgr_workspace& ws, const ScratchLayout& layout, char* scratch, int64_t global_tiles,
