@@ -176,22 +176,27 @@ typedef struct vgr_options {
   int32_t deterministic;            /* accepted; ordering is always deterministic */
   int32_t full_sensor_output;       /* 1: rgb+depth+alpha+semantic, 0: rgb only */
   int32_t fixed_capacity_sort;      /* accepted; the sort never reads the count on the host */
-  int32_t sort_digit_bits;          /* 0 = default (9, or what one pass over the partition needs); 4..9 */
+  int32_t sort_digit_bits;          /* 0 = default (9, or the whole key's width where that is less); 4..9 */
   int32_t raster_batch;             /* Gaussians staged per LDS batch: 0 = default (256); 64..512 */
   int32_t cameras_per_block;        /* projection camera group: 0 = default (32); 1..64 */
   int32_t reuse_projection;         /* 1: composite only, reusing the sorted intersections and
                                        tile ranges of the previous render into this workspace
-                                       (reference projection cache, cuda_backend.py:607-619) */
+                                       (reference projection cache, cuda_backend.py:607-619); they are
+                                       read from the *_out buffers, which the caller swaps with *_in
+                                       where that render's selector was 0 */
   /* Optional instrumentation (NULL / 0 to disable). */
   void* const* stage_events;        /* 5 hipEvent_t recorded on the stream: start, after projection +
-                                       emission, after sort, after tile ranges, after compositing */
+                                       emission, after sort, after tile ranges, after compositing.
+                                       The sort event follows the partition by tile; the depth order
+                                       inside the tiles needs the ranges and lies between the sort and
+                                       the ranges event.  Tile-front: the whole ordering is sort */
   int32_t stage_event_count;        /* 0 or 5 */
   int32_t sort_tile_items;          /* keys per thread of a 512-thread sort tile: 0 = default (16); 8, 12 or 16 */
   int64_t* statistics;              /* int64[4], zeroed then filled: [0] compositor (pixel, Gaussian)
                                        evaluations; [1] sort look-back give-ups (as counters[5]);
                                        [2] projection work items kept by chunk culling; [3] tiles the
                                        tile-front ordering had to sort in full */
-  int32_t persistent_composite;     /* >= 0, accepted for any value: the compositor launches one
+  int32_t persistent_composite;     /* 0 to 2^20, selects nothing: the compositor launches one
                                        workgroup per (camera, tile), which is the faster form */
   int32_t chunk_culling;            /* 1: cull (camera group x chunk) items against camera frusta using
                                        scene.chunk_bounds (scratch sized for it) */

@@ -114,7 +114,7 @@ def test_chunk_culling_drops_work_in_a_room_and_keeps_results():
     print(f"[batched] culling kept {kept} of {chunks * groups} (group, chunk) items", flush=True)
     assert 0 < kept < chunks * groups
     out = flat_numpy(culled.outputs)
-    unculled = build([(0, scene)], specs, chunk_culling=False, spatial_order=False, persistent_composite=0)
+    unculled = build([(0, scene)], specs, chunk_culling=False, spatial_order=False)
     unculled.calibrate(rig.viewmats.to(device()), rig.intrinsics.to(device()))
     reference = flat_numpy(unculled.outputs)
     for name in out:

@@ -1,5 +1,5 @@
-// Workgroup sort of one tile's intersections in LDS, shared by the global
-// ordering (depth order inside a tile) and the tile-front ordering.
+// Sort of one tile's intersections in LDS, by a workgroup or by a wave: the depth
+// order inside a tile of the global ordering.
 //
 // The entries are spread over as many bins as there are entries (up to kBins),
 // evenly over the range of their keys, by LDS counters; each entry then counts

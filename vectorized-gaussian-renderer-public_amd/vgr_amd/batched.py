@@ -111,9 +111,7 @@ class BatchedRenderer:
         self.requested_sh_degree = sh_degree
         self.spatial_order = spatial_order
         self.chunk_culling = chunk_culling
-        if persistent_composite is None:
-            persistent_composite = torch.cuda.get_device_properties(self.device).multi_processor_count * 5
-        self.persistent_composite = persistent_composite
+        self.persistent_composite = persistent_composite or 0  # accepted; selects nothing
         self.tuning = dict(sort_digit_bits=sort_digit_bits, sort_tile_items=sort_tile_items,
                            raster_batch=raster_batch, cameras_per_block=cameras_per_block)
         # The plain per-group path keeps the constructed launch parameters: configure()
