@@ -58,15 +58,31 @@ __device__ __forceinline__ int64_t element_count(const int64_t* counters, int64_
   return n < capacity ? n : capacity;
 }
 
+// Most workgroups of the histogram that count n keys.  Every one ends with an atomic per
+// digit value and pass on the same counters (a thousand workgroups: 40 us), so it takes
+// 16k keys at least where there are many; 512 workgroups, eight waves a CU, are too few
+// to read 87M keys at the rate of the memory.  4.4M keys 30 / 46 us with 512 / 1,024, 9M
+// 59 / 46 / 55 with 512 / 1,024 / 2,048, 87M 500 / 275 / 188; 127M of 64 VGA views 828
+// with 512 and 296 with 2,048.  The host knows the capacity only, so the grid is made for
+// that and workgroups beyond what the count needs leave.
+__host__ __device__ __forceinline__ int64_t histogram_limit(int64_t n) {
+  constexpr int64_t kFew = 512, kMany = 2048;
+  const int64_t workgroups = (n + 16383) / 16384;
+  return workgroups < kFew ? kFew : (workgroups < kMany ? workgroups : kMany);
+}
+
 __global__ __launch_bounds__(kBlockThreads) void sort_histogram_kernel(const uint64_t* __restrict__ keys,
                                                                        const int64_t* __restrict__ counters,
                                                                        int64_t capacity, PartitionKey pk, int digit_bits,
                                                                        int passes, uint32_t* __restrict__ histogram) {
   __shared__ uint32_t local[16 * 256];
   const int radix = 1 << digit_bits;
+  const int64_t n = element_count(counters, capacity);
+  const int64_t limit = histogram_limit(n);
+  const int64_t workgroups = limit < gridDim.x ? limit : gridDim.x;
+  if (blockIdx.x >= workgroups) return;
   for (int i = threadIdx.x; i < passes * radix; i += kBlockThreads) local[i] = 0;
   __syncthreads();
-  const int64_t n = element_count(counters, capacity);
   const uint32_t mask = static_cast<uint32_t>(radix - 1);
   // Keys are read coalesced (lane i takes key i of a 64-key run); per pass, a lane
   // adds to LDS only if it starts a run of equal digits among its wave's keys, and
@@ -78,7 +94,7 @@ __global__ __launch_bounds__(kBlockThreads) void sort_histogram_kernel(const uin
   constexpr int kRuns = 4;
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t wave_id = (static_cast<int64_t>(blockIdx.x) * kBlockThreads + threadIdx.x) / kWave;
-  const int64_t wave_count = static_cast<int64_t>(gridDim.x) * (kBlockThreads / kWave);
+  const int64_t wave_count = workgroups * (kBlockThreads / kWave);
   const uint64_t above = lane == kWave - 1 ? 0ull : (~0ull << (lane + 1));
   for (int64_t base = wave_id * kRuns * kWave; base < n; base += wave_count * kRuns * kWave) {
     uint32_t image[kRuns];
@@ -543,19 +559,11 @@ int launch_sort(const vgr_workspace& ws, const ScratchLayout& layout, char* scra
                      digit_bits, passes, tiles, layout.sort_tile, histogram, tickets, flags, global_tiles, ws.tile_starts,
                      ws.tile_ends, reinterpret_cast<uint32_t*>(scratch + layout.work_counter) + 4);
   const int items = layout.sort_tile / kSortThreads;
-  // Every workgroup ends with an atomic per digit value and pass on the same counters (a
-  // thousand workgroups: 40 us), so it takes 16k keys at least where there are many; 512
-  // workgroups, eight waves a CU, are too few to read 87M keys at the rate of the memory.
-  // 4.4M keys 30 / 46 us with 512 / 1,024, 9M 59 / 46 / 55 with 512 / 1,024 / 2,048, 87M
-  // 500 / 275 / 188; 127M of 64 VGA views 828 with 512 and 296 with 2,048.
-  constexpr int64_t kFew = 512, kMany = 2048;
+  const int64_t limit_blocks = histogram_limit(capacity);
   int64_t histogram_blocks = (capacity + kBlockThreads * 16 - 1) / (kBlockThreads * 16);
-  if (histogram_blocks > kFew) {
-    histogram_blocks = histogram_blocks / 4 < kFew ? kFew : (histogram_blocks / 4 > kMany ? kMany : histogram_blocks / 4);
-  }
-  histogram_blocks = histogram_blocks < 1 ? 1 : histogram_blocks;
-  hipLaunchKernelGGL(sort_histogram_kernel, dim3(static_cast<unsigned>(histogram_blocks)), dim3(kBlockThreads), 0,
-                     stream, ws.keys_in, ws.counters, capacity, pk, digit_bits, passes, histogram);
+  histogram_blocks = histogram_blocks < limit_blocks ? (histogram_blocks < 1 ? 1 : histogram_blocks) : limit_blocks;
+  hipLaunchKernelGGL(sort_histogram_kernel, dim3(static_cast<unsigned>(histogram_blocks)), dim3(kBlockThreads), 0, stream,
+                     ws.keys_in, ws.counters, capacity, pk, digit_bits, passes, histogram);
   hipLaunchKernelGGL(sort_digit_scan_kernel, dim3(1), dim3(kSortThreads), 0, stream, histogram, digit_bits, passes,
                      digit_base);
   const uint64_t* source_keys = ws.keys_in;
