@@ -344,6 +344,7 @@ struct SpreadShared {
   bool queued;
 };
 
+template <bool kMayRefuse>
 __global__ __launch_bounds__(kSpreadThreads, 8) void spread_long_kernel(TileSortArgs args) {
   __shared__ SpreadShared s;
   const int t = threadIdx.x;
@@ -486,12 +487,19 @@ __global__ __launch_bounds__(kSpreadThreads, 8) void spread_long_kernel(TileSort
           bin = low;
           if (length == 0u) continue;  // uniform
           if (t == 0) {
-            s.queued = push_run(args, Run{static_cast<uint32_t>(base) + run_begin, length, tile,
-                                          static_cast<uint32_t>(to)});
+            const bool queued = push_run(args, Run{static_cast<uint32_t>(base) + run_begin, length, tile,
+                                                   static_cast<uint32_t>(to)});
+            if constexpr (kMayRefuse) {
+              s.queued = queued;
+            } else if (!queued) {
+              atomicAdd(reinterpret_cast<unsigned long long*>(args.failures), 1ull);  // never, by the bound
+            }
           }
-          __syncthreads();
-          if (!s.queued) sort_in_place<kSpreadThreads>(args, base + run_begin, length, keys_of[to], values_of[to]);
-          __syncthreads();  // s.queued read before the next run
+          if constexpr (kMayRefuse) {
+            __syncthreads();
+            if (!s.queued) sort_in_place<kSpreadThreads>(args, base + run_begin, length, keys_of[to], values_of[to]);
+            __syncthreads();  // s.queued read before the next run
+          }
           continue;
         }
         const uint32_t length = s.first[bin + 1] - run_begin;
@@ -540,9 +548,10 @@ int launch_tile_sort(const vgr_scene& scene, const vgr_cameras& cameras, const v
   // runs per spread of the part or bin that holds them, of which a 32-bit depth and a
   // 32-bit tie word allow six.  The default digits leave at least 127 places;
   // explicit digits of four or five bits may leave fewer, and parts beyond them are
-  // sorted where they are found, by the workgroup that found them.  tile_sort_kernel has
-  // a form of its own for that, since the code alone costs the usual one scalar registers
-  // and 9 % (127M entries 497 -> 542 us); under small tiles it costs nothing.
+  // sorted where they are found, by the workgroup that found them.  tile_sort_kernel and
+  // spread_long_kernel have a form of their own for that: in the usual ones the code costs
+  // scalar registers and 9 % (127M entries 497 -> 542 us), or two barriers a run (7 %);
+  // under small tiles it costs nothing.
   static_assert(sizeof(Run) == 16 && kSortThreads * kDefaultSortItems <= kRunCapacity,
                 "a part that is spread takes more entries than a sort tile");
   args.long_runs = reinterpret_cast<Run*>(scratch + layout.sort_flags);
@@ -574,8 +583,9 @@ int launch_tile_sort(const vgr_scene& scene, const vgr_cameras& cameras, const v
   constexpr int64_t kPersistent = 512;
   if (longest > kRunCapacity) {
     const int64_t most = capacity / kRunCapacity + 1;
-    hipLaunchKernelGGL(spread_long_kernel, dim3(static_cast<unsigned>(most < kPersistent ? most : kPersistent)),
-                       dim3(kSpreadThreads), 0, stream, args);
+    hipLaunchKernelGGL(may_refuse ? spread_long_kernel<true> : spread_long_kernel<false>,
+                       dim3(static_cast<unsigned>(most < kPersistent ? most : kPersistent)), dim3(kSpreadThreads), 0,
+                       stream, args);
   }
   if (longest > kSplitLeast) {
     const int64_t most = capacity / kSplitLeast + 1;
