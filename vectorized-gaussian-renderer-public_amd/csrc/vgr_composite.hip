@@ -52,7 +52,9 @@ constexpr float kLongShare = 0.5f / 256.0f;
 // 128x128 over 5M 517 / 345 / 318; but twelve of 160x120 over 3M 289 / 280 / 340.  With
 // shorter lists it gains little and may lose: two 480x320 views of 1M (lists of 2,781)
 // 222 / 254 / 225, four 320x240 views of 500k 307 / 311 / 304, 48 room cameras of 160x120
-// in three submissions 1,906 / 1,182 / 1,304.
+// in three submissions 1,906 / 1,182 / 1,304.  A capacity that was fixed beforehand does
+// not hint at long lists, and finding none on the device costs such a submission 10 us, 1
+// % of those room cameras' 2.9 ms: there the length decides.
 constexpr int64_t kReachTiles = 768;
 constexpr int64_t kReachLists = 5000;
 
@@ -1404,8 +1406,8 @@ int launch_composite(const vgr_scene& scene, const vgr_cameras& cameras, const v
     int32_t* order = reinterpret_cast<int32_t*>(const_cast<char*>(scratch) + layout.tile_order);
     int32_t* reach = nullptr;
     if (!front && options.tile_size == 16 && options.statistics == nullptr && blocks > kReachTiles &&
-        blocks <= kMixedCompositeTiles && ws.intersection_capacity >= blocks * kReachLists &&
-        layout.sort_flag_words >= blocks) {
+        blocks <= kMixedCompositeTiles && options.fixed_capacity_sort == 0 &&
+        ws.intersection_capacity >= blocks * kReachLists && layout.sort_flag_words >= blocks) {
       // The sort's flags are read no more.
       reach = reinterpret_cast<int32_t*>(const_cast<char*>(scratch) + layout.sort_flags);
       hipLaunchKernelGGL(args.final_transmittance != nullptr ? tile_reach_kernel<true> : tile_reach_kernel<false>,
