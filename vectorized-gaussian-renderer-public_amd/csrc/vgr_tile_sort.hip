@@ -24,9 +24,10 @@
 // each other's barriers, and two of 8192 entries fit.  Bound by those barriers and
 // the LDS round trips between them.  Measured on 64 cameras of 640x480 over 1M
 // Gaussians (127M intersections, lists of 1651 on average): the whole ordering
-// 5.27 -> 3.56 ms, of it 1.72 for the two partition passes, 0.50 for the lists of
-// up to 2048 entries (82M entries, 4.4 ps each at 24 bytes in and out) and 0.79 for
-// the longer ones; 1 camera of 640x480 over 100k: 118 -> 70 us.
+// 5.27 -> 3.62 ms, of it 1.72 for the two partition passes, 0.30 for their histogram,
+// 0.29 for the ranges, 0.49 for the lists of up to 2048 entries (82M entries, 4.4 ps
+// each at 24 bytes in and out) and 0.79 for the longer ones; 1 camera of 640x480 over
+// 100k: 118 -> 70 us.
 #include "vgr_tile_sort_device.h"
 
 namespace vgr {
