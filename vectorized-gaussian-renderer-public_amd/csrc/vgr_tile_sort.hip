@@ -560,7 +560,8 @@ int launch_tile_sort(const vgr_scene& scene, const vgr_cameras& cameras, const v
   args.runs = args.long_runs + args.long_capacity;
   args.run_capacity = static_cast<uint32_t>(layout.sort_flag_words / 4 - layout.sort_tiles);
   args.state = reinterpret_cast<uint32_t*>(scratch + layout.work_counter) + 4;
-  constexpr int64_t kPartsPerSortTile = 65;
+  constexpr int64_t kPartsPerSortTile = kRunCapacity / kSplitLeast + 2 * kRunCapacity / kTileCapacity + 1 + 6 * 4;
+  static_assert(kPartsPerSortTile == 65, "the bound above");
   const bool may_refuse = args.run_capacity < kPartsPerSortTile * layout.sort_tiles;
   const int64_t capacity = ws.intersection_capacity;
   constexpr int64_t kMaxGrid = 1 << 22;
