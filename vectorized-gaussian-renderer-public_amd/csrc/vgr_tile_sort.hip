@@ -14,7 +14,7 @@
 //                       workgroup takes four: a list of up to 512 entries is one
 //                       wave's, the rest the workgroup's;
 //   spread_long_kernel: parts that do not fit the LDS of run_sort_kernel either are
-//                       spread over 4096 depth bins in global memory and queued as
+//                       spread over up to 4096 depth bins in global memory and queued as
 //                       runs of whole bins that do; a bin that does not fit is spread
 //                       again over its own range (over the tie order when all its
 //                       depths are equal), or sorted in place when its tie words are
@@ -325,7 +325,14 @@ __global__ __launch_bounds__(kRunThreads, 4) void run_sort_kernel(TileSortArgs a
 }
 
 constexpr int kSpreadThreads = 1024;
+// Depth bins of a spread: one per 1024 entries.  Every bin in use keeps a cache line of
+// keys and one of values open for writing, so more of them cost: 256 cameras of four
+// resolutions (the spread of 446M intersections' long lists) 3.9 ms with 4096 bins
+// always, 2.2 with a bin per 256 or 1024 entries, 2.4 per 2048; 16 views of 128x128 over
+// 2M Gaussians (lists of 45,000) 672, 414, 322 and 313 us.
 constexpr int kSpreadBins = 4096;
+constexpr uint32_t kSpreadBinEntries = 1024;
+constexpr uint32_t kSpreadLeastBins = 32;
 constexpr int kSpreadStack = 256;
 constexpr int kSpreadLoads = 4;  // entries in flight per thread
 constexpr uint32_t kSpreadSample = 4096;
@@ -413,7 +420,9 @@ __global__ __launch_bounds__(kSpreadThreads, 8) void spread_long_kernel(TileSort
           continue;
         }
       }
-      const BinMap bin_of(lo, hi, kSpreadBins);
+      uint32_t bins = count / kSpreadBinEntries;
+      bins = bins < kSpreadLeastBins ? kSpreadLeastBins : (bins < kSpreadBins ? bins : kSpreadBins);
+      const BinMap bin_of(lo, hi, bins);
       for (int b = t; b < kSpreadBins; b += kSpreadThreads) s.cursor[b] = 0u;
       __syncthreads();
       for (uint32_t i0 = 0u; i0 < count; i0 += kSpreadThreads * kSpreadLoads) {
@@ -544,10 +553,11 @@ int launch_tile_sort(const vgr_scene& scene, const vgr_cameras& cameras, const v
   args.partition = layout.partition;
   // The look-back flags are read no more: their scratch holds the queues, with a place
   // per sort tile (at most 8192 entries) for a part of over 8192 entries, so those always
-  // fit.  The other parts number at most 65 per 8192 entries: 32 crowded ones of over
+  // fit.  The other parts number at most 101 per 8192 entries: 32 crowded ones of over
   // kSplitLeast, nine of longer lists (two neighbours hold over 2048 entries) and four
-  // runs per spread of the part or bin that holds them, of which a 32-bit depth and a
-  // 32-bit tie word allow six.  The default digits leave at least 127 places;
+  // runs per spread of the part or bin that holds them, of which there is one over a
+  // sampled range and, at kSpreadLeastBins or more a time, seven over a 32-bit depth and
+  // seven over a 32-bit tie word.  The default digits leave at least 127 places;
   // explicit digits of four or five bits may leave fewer, and parts beyond them are
   // sorted where they are found, by the workgroup that found them.  tile_sort_kernel and
   // spread_long_kernel have a form of their own for that: in the usual ones the code costs
@@ -560,8 +570,11 @@ int launch_tile_sort(const vgr_scene& scene, const vgr_cameras& cameras, const v
   args.runs = args.long_runs + args.long_capacity;
   args.run_capacity = static_cast<uint32_t>(layout.sort_flag_words / 4 - layout.sort_tiles);
   args.state = reinterpret_cast<uint32_t*>(scratch + layout.work_counter) + 4;
-  constexpr int64_t kPartsPerSortTile = kRunCapacity / kSplitLeast + 2 * kRunCapacity / kTileCapacity + 1 + 6 * 4;
-  static_assert(kPartsPerSortTile == 65, "the bound above");
+  constexpr int kSpreads = 1 + 2 * 7;
+  static_assert(kSpreadLeastBins == 32, "five bits a spread");
+  constexpr int64_t kPartsPerSortTile =
+      kRunCapacity / kSplitLeast + 2 * kRunCapacity / kTileCapacity + 1 + 4 * kSpreads;
+  static_assert(kPartsPerSortTile == 101, "the bound above");
   const bool may_refuse = args.run_capacity < kPartsPerSortTile * layout.sort_tiles;
   const int64_t capacity = ws.intersection_capacity;
   constexpr int64_t kMaxGrid = 1 << 22;
